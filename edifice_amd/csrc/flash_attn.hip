@@ -17,7 +17,7 @@
 //     (keys permuted consistently in the V^T reads), so P never goes through LDS;
 //   * causal: key tiles above the diagonal are skipped, only diagonal tiles are
 //     masked, and query blocks are issued heaviest-first.
-// f32 (or odd head_dim) path: one wave per query, lanes over head_dim, for parity.
+// float32 and the other head widths: flash_attn_f32.hip (to 128), here one wave per query (wider).
 #include "edf_abi.hpp"
 #include "edf_common.hpp"
 #include "edf_mfma.hpp"
@@ -25,6 +25,9 @@
 #include <type_traits>
 
 namespace edf {
+bool fa32_takes(int batch_heads, int T, int HD, int dtype);
+int fa32_forward(hipStream_t s, const void* q, const void* k, const void* v, const void* cs, void* out, float* lse,
+                 int BH, int T, int HD, int causal, int dtype);
 namespace {
 
 constexpr float LN2 = 0.6931471805599453f;
@@ -531,7 +534,7 @@ __global__ __launch_bounds__(256, 2) void fa_fwd128_kernel(const bf16* __restric
   if (myq < T && g == 0 && LSE != nullptr) LSE[bh * T + myq] = (m * scale_log2 + __log2f(lsum)) * LN2;
 }
 
-// Generic path: one wave per query row, lanes over head_dim (any dtype, any head_dim <= 256).
+// Heads wider than 128: one wave per query row, lanes over head_dim (any dtype, head_dim <= 256).
 template <typename TT, int DPL>
 __global__ __launch_bounds__(256) void fa_fwd_wave_kernel(const TT* __restrict__ Q, const TT* __restrict__ K,
                                                           const TT* __restrict__ V, TT* __restrict__ O,
@@ -611,7 +614,7 @@ __global__ void debug_tr16_kernel(const bf16* x, bf16* out) {
 
 template <int HD>
 void launch_mfma_fwd(hipStream_t s, const void* q, const void* k, const void* v, void* o, float* lse, int BH, int T,
-                     int causal, float scale_log2, const void* cs = nullptr, float sqd = 0.0f) {
+                     int causal, float scale_log2, const void* cs, float sqd) {
   const dim3 grid((T + 127) / 128, BH);
   const bf16 *Q = (const bf16*)q, *K = (const bf16*)k, *V = (const bf16*)v, *CS = (const bf16*)cs;
   if constexpr (HD == 128) {
@@ -635,18 +638,33 @@ void launch_mfma_fwd(hipStream_t s, const void* q, const void* k, const void* v,
 
 template <typename TT>
 void launch_wave_fwd(hipStream_t s, const void* q, const void* k, const void* v, void* o, float* lse, int BH, int T,
-                     int HD, int causal, float scale_log2, const void* cs = nullptr, float sqd = 0.0f) {
+                     int HD, int causal, float scale_log2, const void* cs, float sqd) {
   const long rows = (long)BH * T;
   const unsigned grid = (unsigned)((rows + 3) / 4);
-  if (HD <= 64)
-    fa_fwd_wave_kernel<TT, 1><<<grid, 256, 0, s>>>((const TT*)q, (const TT*)k, (const TT*)v, (TT*)o, lse, BH, T, HD,
-                                                   scale_log2, causal, (const TT*)cs, sqd);
-  else if (HD <= 128)
-    fa_fwd_wave_kernel<TT, 2><<<grid, 256, 0, s>>>((const TT*)q, (const TT*)k, (const TT*)v, (TT*)o, lse, BH, T, HD,
-                                                   scale_log2, causal, (const TT*)cs, sqd);
+  fa_fwd_wave_kernel<TT, 4><<<grid, 256, 0, s>>>((const TT*)q, (const TT*)k, (const TT*)v, (TT*)o, lse, BH, T, HD,
+                                                 scale_log2, causal, (const TT*)cs, sqd);
+}
+
+// Flash attention (cs null) and FoX attention (causal).  bf16 at head_dim 32, 64 and 128 takes the
+// bf16 MFMA kernels; float32, and bf16 at the other widths up to 128, keep scores and probabilities
+// in float32 on the f32 MFMA (flash_attn_f32.hip); wider heads one wave per query row.
+int fa_fwd_run(hipStream_t s, const void* q, const void* k, const void* v, const void* cs, void* out, float* lse,
+               int BH, int T, int HD, int causal, int dtype) {
+  const float scale_log2 = LOG2E / sqrtf((float)HD);
+  const float sqd = sqrtf((float)HD);
+  if (dtype == EDF_BF16 && HD == 128)
+    launch_mfma_fwd<128>(s, q, k, v, out, lse, BH, T, causal, scale_log2, cs, sqd);
+  else if (dtype == EDF_BF16 && HD == 64)
+    launch_mfma_fwd<64>(s, q, k, v, out, lse, BH, T, causal, scale_log2, cs, sqd);
+  else if (dtype == EDF_BF16 && HD == 32)
+    launch_mfma_fwd<32>(s, q, k, v, out, lse, BH, T, causal, scale_log2, cs, sqd);
+  else if (fa32_takes(BH, T, HD, dtype))
+    return fa32_forward(s, q, k, v, cs, out, lse, BH, T, HD, causal, dtype);
+  else if (dtype == EDF_BF16)
+    launch_wave_fwd<bf16>(s, q, k, v, out, lse, BH, T, HD, causal, scale_log2, cs, sqd);
   else
-    fa_fwd_wave_kernel<TT, 4><<<grid, 256, 0, s>>>((const TT*)q, (const TT*)k, (const TT*)v, (TT*)o, lse, BH, T, HD,
-                                                   scale_log2, causal, (const TT*)cs, sqd);
+    launch_wave_fwd<float>(s, q, k, v, out, lse, BH, T, HD, causal, scale_log2, cs, sqd);
+  return check_launch(cs != nullptr ? "fox attention" : "flash attention");
 }
 
 }  // namespace
@@ -674,22 +692,7 @@ int edf_fused_flash_attention(void* stream, const void* q, const void* k, const 
   EDF_REQUIRE(valid_dtype(dtype), EDF_ERR_INVALID_ARG, "dtype must be 0 (f32) or 1 (bf16)");
   EDF_REQUIRE(head_dim <= 256, EDF_ERR_UNSUPPORTED, "head_dim %d > 256 unsupported", head_dim);
   EDF_REQUIRE(q && k && v && out, EDF_ERR_INVALID_ARG, "null tensor pointer");
-  hipStream_t s = as_stream(stream);
-  const int BH = batch * num_heads;
-  const float scale_log2 = LOG2E / sqrtf((float)head_dim);
-  if (dtype == EDF_BF16 && (head_dim == 32 || head_dim == 64 || head_dim == 128)) {
-    if (head_dim == 128)
-      launch_mfma_fwd<128>(s, q, k, v, out, lse, BH, seq_len, causal, scale_log2);
-    else if (head_dim == 64)
-      launch_mfma_fwd<64>(s, q, k, v, out, lse, BH, seq_len, causal, scale_log2);
-    else
-      launch_mfma_fwd<32>(s, q, k, v, out, lse, BH, seq_len, causal, scale_log2);
-  } else if (dtype == EDF_BF16) {
-    launch_wave_fwd<bf16>(s, q, k, v, out, lse, BH, seq_len, head_dim, causal, scale_log2);
-  } else {
-    launch_wave_fwd<float>(s, q, k, v, out, lse, BH, seq_len, head_dim, causal, scale_log2);
-  }
-  return check_launch("flash attention");
+  return fa_fwd_run(as_stream(stream), q, k, v, nullptr, out, lse, batch * num_heads, seq_len, head_dim, causal, dtype);
 }
 
 int edf_fused_fox_attention(void* stream, const void* q, const void* k, const void* v, const void* cs, void* out,
@@ -700,23 +703,7 @@ int edf_fused_fox_attention(void* stream, const void* q, const void* k, const vo
   EDF_REQUIRE(valid_dtype(dtype), EDF_ERR_INVALID_ARG, "dtype must be 0 (f32) or 1 (bf16)");
   EDF_REQUIRE(head_dim <= 256, EDF_ERR_UNSUPPORTED, "head_dim %d > 256 unsupported", head_dim);
   EDF_REQUIRE(q && k && v && cs && out, EDF_ERR_INVALID_ARG, "null tensor pointer");
-  hipStream_t s = as_stream(stream);
-  const int BH = batch * num_heads;
-  const float scale_log2 = LOG2E / sqrtf((float)head_dim);
-  const float sqd = sqrtf((float)head_dim);
-  if (dtype == EDF_BF16 && (head_dim == 32 || head_dim == 64 || head_dim == 128)) {
-    if (head_dim == 128)
-      launch_mfma_fwd<128>(s, q, k, v, out, lse, BH, seq_len, 1, scale_log2, cs, sqd);
-    else if (head_dim == 64)
-      launch_mfma_fwd<64>(s, q, k, v, out, lse, BH, seq_len, 1, scale_log2, cs, sqd);
-    else
-      launch_mfma_fwd<32>(s, q, k, v, out, lse, BH, seq_len, 1, scale_log2, cs, sqd);
-  } else if (dtype == EDF_BF16) {
-    launch_wave_fwd<bf16>(s, q, k, v, out, lse, BH, seq_len, head_dim, 1, scale_log2, cs, sqd);
-  } else {
-    launch_wave_fwd<float>(s, q, k, v, out, lse, BH, seq_len, head_dim, 1, scale_log2, cs, sqd);
-  }
-  return check_launch("fox attention");
+  return fa_fwd_run(as_stream(stream), q, k, v, cs, out, lse, batch * num_heads, seq_len, head_dim, 1, dtype);
 }
 
 }  // extern "C"

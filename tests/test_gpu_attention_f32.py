@@ -1,0 +1,92 @@
+"""GPU parity: attention on the f32 matrix cores (float32, and bfloat16 head widths off 32 / 64 / 128)
+at the edges of its 32-row tiles, its four-wave split and its padded widths."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import scans
+from tests.conftest import assert_close
+from tests.gpu_util import TOL, announce, host, rounded, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(q, k, v, do, dtype, causal, cs=None):
+    from edifice_amd import fused_scan as fs
+    ts = [to_dev(a, dtype).requires_grad_() for a in (q, k, v)]
+    if cs is not None:
+        ts.append(to_dev(cs, dtype).requires_grad_())
+        out = fs.fox_attention(*ts)
+    else:
+        out = fs.flash_attention(*ts, causal=causal)
+    return [out] + list(torch.autograd.grad(out, ts, to_dev(do, dtype)))
+
+
+# float32 sums of up to a few hundred terms differ from float64 by a few 1e-7 of the largest value
+# (measured 5e-7); bfloat16 results by their rounding, half an ulp = 2^-9 of a value
+REL = {torch.float32: 5e-6, torch.bfloat16: 2.0 ** -8}
+# the bfloat16 gradients also take D = rowsum(dO o O) from the rounded O: an error of 2^-9 |dO| |O| in every
+# dP - D, whose own size is the spread of dO . V over the keys, which the fewest keys leave smallest (two: a
+# quarter of |dO| |V| is common), so 8 x 2^-9
+REL_GRAD = {torch.float32: 5e-6, torch.bfloat16: 2.0 ** -6}
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("shape", [(1, 1, 2, 5), (2, 1, 31, 24), (1, 3, 33, 36), (1, 2, 129, 96), (1, 1, 160, 33),
+                                   (1, 2, 97, 104), (1, 1, 300, 80), (3, 1, 64, 128)])
+def test_attention_tile_edges(shape, causal, dtype, rng):
+    if dtype == torch.bfloat16 and shape[3] in (32, 64, 128):
+        pytest.skip("bf16 at this width takes the bf16 kernels")
+    announce("attention_tile_edges", shape=shape, causal=causal, dtype=dtype)
+    q, k, v, do = (rng.normal(scale=shape[3] ** -0.25, size=shape) for _ in range(4))
+    got = _run(q, k, v, do, dtype, causal)
+    qr, kr, vr, dor = (rounded(a, dtype) for a in (q, k, v, do))
+    want = [scans.flash_attention(qr, kr, vr, causal), *scans.flash_attention_backward(qr, kr, vr, dor, causal)]
+    for name, g, w in zip(("o", "dq", "dk", "dv"), got, want):
+        err = np.linalg.norm(host(g) - w) / np.linalg.norm(w)
+        assert err <= (REL if name in ("o", "dv") else REL_GRAD)[dtype], f"{name}: {err:.2e}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("shape", [(1, 2, 70, 48), (1, 1, 33, 128), (2, 1, 40, 7)])
+def test_fox_tile_edges(shape, dtype, rng):
+    if dtype == torch.bfloat16 and shape[3] == 128:
+        pytest.skip("bf16 at this width takes the bf16 kernels")
+    announce("fox_tile_edges", shape=shape, dtype=dtype)
+    q, k, v, do = (rng.normal(scale=shape[3] ** -0.25, size=shape) for _ in range(4))
+    cs = np.cumsum(-np.abs(rng.normal(scale=0.2, size=shape[:3])), axis=-1)
+    got = _run(q, k, v, do, dtype, True, cs)
+    qr, kr, vr, cr, dor = (rounded(a, dtype) for a in (q, k, v, cs, do))
+    want = [scans.fox_attention(qr, kr, vr, cr), *scans.fox_attention_backward(qr, kr, vr, cr, dor)]
+    for name, g, w in zip(("o", "dq", "dk", "dv", "dcs"), got, want):
+        assert_close(host(g), w, TOL[dtype], name)
+
+
+@pytest.mark.parametrize("d", [64, 40, 33])
+def test_masked_values_take_no_part(d, rng):
+    """Causal rows before a position do not see it: with q, k, v (and the output gradient) infinite
+    or NaN from row 70 on, the first 70 rows of the output and of dQ are those of the finite call (to
+    float32 rounding: the tile holding row 70 sums its visible pairs one by one), and so are the later
+    rows of dK and dV where the earlier rows' output gradient is infinite."""
+    announce("masked_values", d=d)
+    shape, cut = (1, 2, 90, d), 70
+    q, k, v, do = (rng.normal(scale=d ** -0.25, size=shape) for _ in range(4))
+    do[:, :, cut:] = 0
+    near = dict(rtol=1e-4, atol=1e-6)
+    base = _run(q, k, v, do, torch.float32, True)
+    bad_k, bad_v = k.copy(), v.copy()
+    bad_k[:, :, cut:] = np.inf
+    bad_v[:, :, cut:] = np.nan
+    got = _run(q, bad_k, bad_v, do, torch.float32, True)
+    assert torch.allclose(got[0][:, :, :cut], base[0][:, :, :cut], **near)
+    assert torch.allclose(got[1][:, :, :cut], base[1][:, :, :cut], **near)
+    # keys from row 70 on see only later queries: the earlier ones, infinite, take no part
+    do2 = do.copy()
+    do2[:, :, cut:] = rng.normal(size=do2[:, :, cut:].shape)
+    base = _run(q, k, v, do2, torch.float32, True)
+    bad_do = do2.copy()
+    bad_do[:, :, :cut] = np.inf
+    got = _run(q, k, v, bad_do, torch.float32, True)
+    for i in (2, 3):
+        assert torch.allclose(got[i][:, :, cut:], base[i][:, :, cut:], **near)
