@@ -54,6 +54,7 @@ def sources():
 PER_FILE_FLAGS = {
     "flash_attn_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "delta_rule_chunk.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "delta_rule_row.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 
 

@@ -1,8 +1,8 @@
 // C-ABI entry points of the delta rule (DeltaNet / GatedDeltaNet), forward and backward.
 // Dispatch: the chunked MFMA kernels (delta_rule_chunk.hip) take bf16, per-head beta,
 // head_dim 64 .. 128 (a multiple of 8; zero-padded to 128 inside), seq >= 64 (forward and
-// backward); the exact per-step kernels
-// (delta_rule_seq.hip) serve every other case.
+// backward); every other case takes the row scans (delta_rule_row.hip) forward and the exact
+// per-step kernels (delta_rule_seq.hip) backward.
 #include "edf_abi.hpp"
 
 namespace edf {

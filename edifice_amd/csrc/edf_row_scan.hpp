@@ -1,0 +1,271 @@
+// Building blocks of the row-wise delta-rule scans (delta_rule_row.hip): one wave holds 16 rows of
+// a head's state over all its columns and takes 16 steps at a time on the matrix cores.
+//
+// Layout.  Lane l of the wave is (li = l % 16, grp = l / 16).  The state S of the wave's rows is held
+// transposed in 16 x 16 accumulator tiles: register r of tile jt is S[row li][column 16 jt + 4 grp + r].
+// Quantities per (step, row) of the 16-step chunk are accumulator tiles too, with the steps in the
+// order that makes register r of group grp step 4 r + grp: a register then is one block of four
+// consecutive steps, spread over the groups as the B operand of v_mfma_f32_16x16x4_f32 wants it, and
+// four registers are the B operand of the 16-deep bf16 product.  Row operands of the chunk's k and q
+// read row sigma(li) of the staged tile for the same reason.
+//
+// bf16 inputs use bf16 products: k and q are exact, and the float32 factor (state, update) is split
+// into three bf16 parts that add up to it exactly (8 + 8 + 8 mantissa bits, by truncation), so a
+// product carries float32 accuracy at three bf16 products.  float32 inputs use the f32 MFMA.
+#pragma once
+
+#include "edf_common.hpp"
+#include "edf_mfma.hpp"
+
+namespace edf {
+namespace rowscan {
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+constexpr int CH = 16;  // steps per chunk
+constexpr int RW = 16;  // state rows per wave
+
+EDF_DEVICE int sigma(int x) { return 4 * (x & 3) + (x >> 2); }
+
+EDF_DEVICE f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+EDF_DEVICE f32x4 mfma32k(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// x = hi + mid + lo, each a bf16, by truncation (exact for finite x)
+EDF_DEVICE unsigned hi_bits(float x) { return __builtin_bit_cast(unsigned, x) & 0xffff0000u; }
+EDF_DEVICE float bits_to_f32(unsigned v) { return __builtin_bit_cast(float, v); }
+EDF_DEVICE unsigned pack_hi(float lo, float hi) {  // the upper halves of two floats, as two bf16
+  return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x07060302u);
+}
+struct Split4 {
+  bf16x4 part[3];
+};
+EDF_DEVICE Split4 split4(f32x4 x) {
+  typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
+  Split4 s;
+#pragma unroll
+  for (int n = 0; n < 3; ++n) {
+    u32x2 w = {pack_hi(x[0], x[1]), pack_hi(x[2], x[3])};
+    s.part[n] = __builtin_bit_cast(bf16x4, w);
+    if (n < 2) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] -= bits_to_f32(hi_bits(x[e]));
+    }
+  }
+  return s;
+}
+
+// ---- a staged 16-step tile of k or q and its operands ------------------------------------------
+template <typename TT, int DP>
+constexpr int tile_ld() {
+  return DP + (sizeof(TT) == 2 ? 8 : 4);
+}
+
+// Row fragments over W columns (tile: stride LD, from the first of them): for bf16, columns
+// 32 kk + 4 grp .. + 3 and 32 kk + 16 + 4 grp .. + 3 of row sigma(li); for float, columns 16 jt + 4 grp .. + 3.
+template <typename TT, int W> struct RowFrag;
+template <int W> struct RowFrag<bf16, W> {
+  bf16x8 f[W / 32];
+  template <int LD> EDF_DEVICE void load(const bf16* tile, int li, int grp) {
+    const bf16* row = tile + sigma(li) * LD + 4 * grp;
+#pragma unroll
+    for (int kk = 0; kk < W / 32; ++kk)
+      f[kk] = cat4(*(const bf16x4*)(row + 32 * kk), *(const bf16x4*)(row + 32 * kk + 16));
+  }
+};
+template <int W> struct RowFrag<float, W> {
+  f32x4 f[W / 16];
+  template <int LD> EDF_DEVICE void load(const float* tile, int li, int grp) {
+    const float* row = tile + sigma(li) * LD + 4 * grp;
+#pragma unroll
+    for (int jt = 0; jt < W / 16; ++jt) f[jt] = *(const f32x4*)(row + 16 * jt);
+  }
+};
+
+// The chunk's Gram tile a b^T: register r of (li, grp) = a[step 4 r + grp] . b[step sigma(li)], the A
+// operand of block r in a sum over a's steps.
+template <int DP>
+EDF_DEVICE f32x4 gram(const RowFrag<bf16, DP>& a, const RowFrag<bf16, DP>& b) {
+  f32x4 c = {0, 0, 0, 0};
+#pragma unroll
+  for (int kk = 0; kk < DP / 32; ++kk) c = mfma32k(a.f[kk], b.f[kk], c);
+  return c;
+}
+template <int DP>
+EDF_DEVICE f32x4 gram(const RowFrag<float, DP>& a, const RowFrag<float, DP>& b) {
+  f32x4 c = {0, 0, 0, 0};
+#pragma unroll
+  for (int jt = 0; jt < DP / 16; ++jt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = mfma4(a.f[jt][e], b.f[jt][e], c);
+  return c;
+}
+
+// pa, pb: the [step][row] tiles of a[step] . S[row] and b[step] . S[row] over W columns (one split of
+// S serves both).  The parts of S have accumulators of their own: more chains of products, and the
+// small terms are added up before they meet the large ones.
+template <int W>
+EDF_DEVICE void state_dots(const RowFrag<bf16, W>& a, const RowFrag<bf16, W>& b, const f32x4 (&S)[W / 16], f32x4& pa,
+                           f32x4& pb) {
+  f32x4 ca[3] = {}, cb[3] = {};
+#pragma unroll
+  for (int kk = 0; kk < W / 32; ++kk) {
+    const Split4 s0 = split4(S[2 * kk]), s1 = split4(S[2 * kk + 1]);
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      const bf16x8 s = cat4(s0.part[n], s1.part[n]);
+      ca[n] = mfma32k(a.f[kk], s, ca[n]);
+      cb[n] = mfma32k(b.f[kk], s, cb[n]);
+    }
+  }
+  pa = (ca[2] + ca[1]) + ca[0];
+  pb = (cb[2] + cb[1]) + cb[0];
+}
+template <int W>
+EDF_DEVICE void state_dots(const RowFrag<float, W>& a, const RowFrag<float, W>& b, const f32x4 (&S)[W / 16], f32x4& pa,
+                           f32x4& pb) {
+  pa = pb = f32x4{0, 0, 0, 0};
+#pragma unroll
+  for (int jt = 0; jt < W / 16; ++jt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      pa = mfma4(a.f[jt][e], S[jt][e], pa);
+      pb = mfma4(b.f[jt][e], S[jt][e], pb);
+    }
+}
+
+// The A operands of S += u^T tile over W columns: for bf16 element r of f[jt] is step 4 r + grp, column
+// 16 jt + li; for float f[jt][r].
+template <typename TT, int W> struct ColFrag;
+template <int W> struct ColFrag<bf16, W> {
+  bf16x4 f[W / 16];
+  template <int LD> EDF_DEVICE void load(const bf16* tile, int li, int grp) {
+    const bf16* at = tile + (4 * (li >> 2) + grp) * LD + 4 * (li & 3);
+#pragma unroll
+    for (int jt = 0; jt < W / 16; ++jt) f[jt] = lds_read_tr16(at + 16 * jt);
+  }
+};
+template <int W> struct ColFrag<float, W> {
+  f32x4 f[W / 16];
+  template <int LD> EDF_DEVICE void load(const float* tile, int li, int grp) {
+    const float* at = tile + grp * LD + li;
+#pragma unroll
+    for (int jt = 0; jt < W / 16; ++jt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) f[jt][r] = at[4 * r * LD + 16 * jt];
+  }
+};
+
+// S[row][column] += sum over the chunk's steps of u[step][row] tile[step][column].  Both products of
+// a tile are 32 deep (the second half of the small one zero): a 16-deep product accumulated into by
+// a 32-deep one right behind it lost part of its result (half of a tile's registers, seen as 1e-6
+// differences in the state), so chained products keep to one shape.
+template <int W>
+EDF_DEVICE void state_add(f32x4 (&S)[W / 16], const ColFrag<bf16, W>& k, f32x4 u) {
+  const Split4 s = split4(u);
+  const bf16x8 hm = cat4(s.part[0], s.part[1]), lo = cat4(s.part[2], bf16x4{});
+#pragma unroll
+  for (int jt = 0; jt < W / 16; ++jt) S[jt] = mfma32k(cat4(k.f[jt], k.f[jt]), lo, S[jt]);
+#pragma unroll
+  for (int jt = 0; jt < W / 16; ++jt) S[jt] = mfma32k(cat4(k.f[jt], k.f[jt]), hm, S[jt]);
+}
+template <int W>
+EDF_DEVICE void state_add(f32x4 (&S)[W / 16], const ColFrag<float, W>& k, f32x4 u) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int jt = 0; jt < W / 16; ++jt) S[jt] = mfma4(k.f[jt][r], u[r], S[jt]);
+}
+
+// Value of each of the four groups, in every lane of the same li.  The swaps are not volatile (unlike
+// swap16 / swap32): a gather is a function of its input, free to move among the chunk's other work.
+EDF_DEVICE void gather4(float x, float (&v)[4]) {
+  float a = x, b = x;
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));  // a: groups 0 0 2 2, b: groups 1 1 3 3
+  float c = a, d = b;
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\tv_permlane32_swap_b32 %2, %3" : "+v"(a), "+v"(c), "+v"(b), "+v"(d));
+  v[0] = a, v[1] = b, v[2] = c, v[3] = d;
+}
+EDF_DEVICE float pick4(float v0, float v1, float v2, float v3, int grp) {
+  const float lo = (grp & 1) ? v1 : v0, hi = (grp & 1) ? v3 : v2;
+  return (grp & 2) ? hi : lo;
+}
+EDF_DEVICE float lane_value(float v, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+
+// ---- 16 steps of [B, T, H, d] rows: memory -> registers (a chunk ahead) -> LDS -------------------
+// A lane's byte offset runs ahead by 16 steps per load.  Steps past T and columns past d read as
+// zero (offsets past the batch row; the caller keeps the steps it runs ahead below 2^31 bytes).
+// VEC: d is a multiple of 8 (bf16) or 4 (float) and rows start on 4-byte boundaries, so a row's
+// 16-byte pieces lie whole inside or outside it.
+template <typename TT, int DP, bool VEC> struct TileRegs;
+template <typename TT, int DP> struct TileRegs<TT, DP, true> {
+  static constexpr int EPV = 16 / (int)sizeof(TT);   // elements per 16 bytes
+  static constexpr int PPR = DP / EPV;               // pieces per row
+  static constexpr int N = CH * PPR / 64;            // pieces per lane, 64 / PPR steps apart
+  static_assert(N >= 1 && 64 % PPR == 0, "a wave-wide load takes whole rows");
+  u32x4 v[N];
+  unsigned off;
+  EDF_DEVICE void at(unsigned base, unsigned stepb, int t0, int d, int l) {
+    const int col = (l % PPR) * EPV;
+    off = col < d ? base + (unsigned)(t0 + l / PPR) * stepb + col * (unsigned)sizeof(TT) : OOB_OFF;
+  }
+  EDF_DEVICE void load(rsrc_t r, unsigned stepb, int advance) {
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+      v[n] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(off + n * (64 / PPR) * stepb), 0, 0));
+    off += (unsigned)advance * stepb;
+  }
+  EDF_DEVICE void store(TT* tile, int l) const {
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+      *(u32x4*)(tile + (l / PPR + n * (64 / PPR)) * tile_ld<TT, DP>() + (l % PPR) * EPV) = v[n];
+  }
+};
+template <typename TT, int DP> struct TileRegs<TT, DP, false> {
+  static constexpr int N = CH * DP / 64;
+  typename Bits<TT>::type v[N];
+  unsigned base, t;
+  int d, l;
+  EDF_DEVICE void at(unsigned base_, unsigned, int t0, int d_, int l_) { base = base_, t = t0, d = d_, l = l_; }
+  EDF_DEVICE void load(rsrc_t r, unsigned stepb, int advance) {
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const int e = l + 64 * n, col = e % DP;
+      v[n] = bload<TT>(r, col < d ? base + (t + e / DP) * stepb + col * (unsigned)sizeof(TT) : OOB_OFF);
+    }
+    t += advance;
+  }
+  EDF_DEVICE void store(TT* tile, int l_) const {
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const int e = l_ + 64 * n;
+      tile[e / DP * tile_ld<TT, DP>() + e % DP] = __builtin_bit_cast(TT, v[n]);
+    }
+  }
+};
+
+// This lane's four values (steps t0 + 4 r + grp, a byte offset running ahead) of a per-row or
+// per-head tensor.
+template <typename TT> struct GateRegs {
+  typename Bits<TT>::type v[4];
+  unsigned off;
+  EDF_DEVICE void at(unsigned base, unsigned stepb, int t0, int grp) { off = base + (unsigned)(t0 + grp) * stepb; }
+  EDF_DEVICE void load(rsrc_t r, unsigned stepb, int advance) {
+#pragma unroll
+    for (int n = 0; n < 4; ++n) v[n] = bload<TT>(r, off + 4 * n * stepb);
+    off += (unsigned)advance * stepb;
+  }
+};
+
+// LDS traffic of the workgroup's waves ordered around a barrier; global loads and stores stay in flight.
+EDF_DEVICE void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+}  // namespace rowscan
+}  // namespace edf

@@ -1,0 +1,89 @@
+"""GPU parity: the 16-step row scans of the delta rule (per-row beta, float32, KDA) at the edges of their
+chunks, blocks of four steps, row blocks and padded widths."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import scans
+from tests.gpu_util import announce, host, rounded, to_dev
+
+pytestmark = pytest.mark.gpu
+
+# float32: sums of up to d + T terms against float64 (measured 1.5e-7 at T = 777); bfloat16: the rounding of
+# the result, half an ulp = 2^-9 of a value
+REL = {torch.float32: 3e-6, torch.bfloat16: 2.0 ** -8}
+
+
+def _inputs(rng, B, T, H, d, kind):
+    def unit(x):
+        return x / np.linalg.norm(x, axis=-1, keepdims=True)
+
+    a = {"q": rng.normal(size=(B, T, H, d)), "k": unit(rng.normal(size=(B, T, H, d))), "v": rng.normal(size=(B, T, H, d))}
+    sig = lambda *s: 1 / (1 + np.exp(-rng.normal(size=s)))  # noqa: E731
+    if kind == "kda":
+        a["alpha"], a["beta"] = -0.3 * rng.uniform(size=(B, T, H, d)), sig(B, T, H)
+    else:
+        a["beta"] = sig(B, T, H) if kind == "head" else sig(B, T, H, d)
+        if kind == "gated":
+            a["alpha"] = sig(B, T, H)
+            a["alpha"][:, ::5] = 0.0  # a full reset of the state
+    return a
+
+
+def _call(kind, t):
+    from edifice_amd import fused_scan as fs
+    if kind == "kda":
+        return fs.kda_scan(t["q"], t["k"], t["v"], t["alpha"], t["beta"])
+    if kind == "gated":
+        return fs.gated_delta_net_scan(t["q"], t["k"], t["v"], t["beta"], t["alpha"])
+    return fs.delta_net_scan(t["q"], t["k"], t["v"], t["beta"])
+
+
+def _oracle(kind, a, do=None):
+    if kind == "kda":
+        args = (a["q"], a["k"], a["v"], a["alpha"], a["beta"])
+        return scans.kda_scan(*args) if do is None else scans.kda_scan_backward(*args, do)
+    args = (a["q"], a["k"], a["v"], a["beta"])
+    alpha = a.get("alpha")
+    return scans.delta_rule(*args, alpha) if do is None else scans.delta_rule_backward(*args, do, alpha)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("kind", ["element", "head", "gated", "kda"])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 3), (2, 15, 1, 16), (1, 16, 2, 17), (1, 17, 3, 32), (2, 35, 1, 48),
+                                   (1, 50, 2, 64), (1, 33, 1, 90), (1, 63, 1, 128)])
+def test_row_scan_edges(shape, kind, dtype, rng):
+    announce("row_scan_edges", shape=shape, kind=kind, dtype=dtype)
+    a = _inputs(rng, *shape, kind)
+    do = rng.normal(size=shape)
+    t = {n: to_dev(x, dtype).requires_grad_() for n, x in a.items()}
+    out = _call(kind, t)
+    grads = dict(zip(t, torch.autograd.grad(out, list(t.values()), to_dev(do, dtype))))
+    r = {n: rounded(x, dtype) for n, x in a.items()}
+    want = _oracle(kind, r, rounded(do, dtype))
+    pairs = [("o", out, _oracle(kind, r))] + [("d" + n, g, want["d" + n]) for n, g in grads.items()]
+    for name, g, w in pairs:
+        norm = np.linalg.norm(w)
+        assert np.linalg.norm(host(g) - w) <= REL[dtype] * norm + 1e-30, f"{name}: {np.linalg.norm(host(g) - w) / norm:.2e}"
+    again = _call(kind, t)
+    assert torch.equal(out, again)
+
+
+@pytest.mark.parametrize("kind", ["element", "kda"])
+def test_later_steps_take_no_part(kind, rng):
+    """Infinite or NaN values from step 21 on (inside a chunk and a block of four) leave the outputs before it
+    as they are, and a NaN value row stays in its row."""
+    announce("later_steps", kind=kind)
+    a = _inputs(rng, 1, 40, 2, 64, kind)
+    base = _call(kind, {n: to_dev(x, torch.bfloat16) for n, x in a.items()})
+    for name, bad in (("v", np.nan), ("k", np.inf), ("q", np.nan)):
+        b = {n: x.copy() for n, x in a.items()}
+        b[name][:, 21:] = bad
+        out = _call(kind, {n: to_dev(x, torch.bfloat16) for n, x in b.items()})
+        assert torch.allclose(out[:, :21].float(), base[:, :21].float(), rtol=2.0 ** -7, atol=1e-6), name
+    b = {n: x.copy() for n, x in a.items()}
+    b["v"][:, 5, :, 9] = np.nan
+    out = _call(kind, {n: to_dev(x, torch.bfloat16) for n, x in b.items()})
+    rest = [i for i in range(64) if i != 9]
+    assert torch.allclose(out[..., rest].float(), base[..., rest].float(), rtol=2.0 ** -7, atol=1e-6)
+    assert bool(out[:, 5:, :, 9].isnan().all()) and not bool(out[:, :5, :, 9].isnan().any())
