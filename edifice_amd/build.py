@@ -55,6 +55,7 @@ PER_FILE_FLAGS = {
     "flash_attn_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "delta_rule_chunk.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "delta_rule_row.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "delta_rule_row_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 
 

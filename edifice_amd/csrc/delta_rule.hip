@@ -1,8 +1,9 @@
 // C-ABI entry points of the delta rule (DeltaNet / GatedDeltaNet), forward and backward.
 // Dispatch: the chunked MFMA kernels (delta_rule_chunk.hip) take bf16, per-head beta,
 // head_dim 64 .. 128 (a multiple of 8; zero-padded to 128 inside), seq >= 64 (forward and
-// backward); every other case takes the row scans (delta_rule_row.hip) forward and the exact
-// per-step kernels (delta_rule_seq.hip) backward.
+// backward); every other case takes the row scans (delta_rule_row.hip) forward, and backward
+// the row scans without a decay (delta_rule_row_bwd.hip), the exact per-step kernels
+// (delta_rule_seq.hip) with one.
 #include "edf_abi.hpp"
 
 namespace edf {
@@ -15,6 +16,14 @@ int dr_seq_backward_run(void* stream, const void* q, const void* k, const void* 
                         const void* alpha, const void* grad_out, void* dq, void* dk, void* dv, void* dbeta,
                         void* dalpha, void* workspace, int batch, int seq, int heads, int d, int dtype,
                         int beta_per_head, int alpha_per_row, const float* context);
+bool dr_row_takes(int batch, int heads, int seq, int d);
+size_t dr_row_context_bytes(int batch, int heads, int seq, int d);
+int dr_row_record_run(void* stream, const void* q, const void* k, const void* v, const void* beta, void* out,
+                      int batch, int seq, int heads, int d, int dtype, int beta_per_head, void* context);
+size_t dr_row_backward_workspace_bytes(int batch, int heads, int seq, int d);
+int dr_row_backward_run(void* stream, const void* q, const void* k, const void* v, const void* beta,
+                        const void* grad_out, void* dq, void* dk, void* dv, void* dbeta, void* workspace, int batch,
+                        int seq, int heads, int d, int dtype, int beta_per_head, const void* context);
 bool dr_chunk_eligible(int seq, int d, int dtype, int beta_per_head);
 size_t dr_chunk_workspace_bytes(int batch, int seq, int heads, int d);
 int dr_chunk_run(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
@@ -39,6 +48,22 @@ int check_dr(int batch, int seq, int heads, int d, int dtype, int beta_mode) {
   return EDF_OK;
 }
 
+// Whether the row scans take a call's backward too (and its forward's record is theirs).
+bool row_backward(const void* alpha, int batch, int heads, int seq, int d) {
+  return alpha == nullptr && dr_row_takes(batch, heads, seq, d);
+}
+
+// The size queries do not know whether a decay is given: the larger of the two paths' needs.
+size_t unchunked_context_bytes(int batch, int heads, int seq, int d) {
+  const size_t a = dr_seq_context_bytes(batch, heads, seq, d), b = dr_row_context_bytes(batch, heads, seq, d);
+  return a > b ? a : b;
+}
+size_t unchunked_backward_bytes(int batch, int heads, int seq, int d) {
+  const size_t a = dr_seq_backward_workspace_bytes(batch, heads, seq, d);
+  const size_t b = dr_row_backward_workspace_bytes(batch, heads, seq, d);
+  return a > b ? a : b;
+}
+
 int fwd(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha, void* out,
         void* workspace, size_t ws_bytes, int batch, int seq, int heads, int d, int dtype, int beta_mode) {
   int rc = check_dr(batch, seq, heads, d, dtype, beta_mode);
@@ -52,9 +77,13 @@ int fwd(void* stream, const void* q, const void* k, const void* v, const void* b
     EDF_REQUIRE(workspace && ws_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
     return dr_chunk_run(stream, q, k, v, beta, alpha, out, workspace, batch, seq, heads, d);
   }
-  // per-step path: a workspace of edf_delta_rule_forward_context_bytes() (optional) also
-  // receives the states every 16 steps, which the saved backward then reads
-  const bool keep = workspace && ws_bytes >= dr_seq_context_bytes(batch, heads, seq, d);
+  // a workspace of edf_delta_rule_forward_context_bytes() (optional) also receives what the saved
+  // backward reads: the states every 16 steps, or without a decay every 64 and err
+  if (row_backward(alpha, batch, heads, seq, d) && workspace &&
+      ws_bytes >= unchunked_context_bytes(batch, heads, seq, d))
+    return dr_row_record_run(stream, q, k, v, beta, out, batch, seq, heads, d, dtype, per_head, workspace);
+  const bool keep = !row_backward(alpha, batch, heads, seq, d) && workspace &&
+                    ws_bytes >= unchunked_context_bytes(batch, heads, seq, d);
   return dr_seq_run(stream, q, k, v, beta, alpha, out, batch, seq, heads, d, dtype, per_head, 0,
                     keep ? (float*)workspace : nullptr);
 }
@@ -73,10 +102,13 @@ int bwd(void* stream, const void* q, const void* k, const void* v, const void* b
     return dr_chunk_backward_run(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch,
                                  seq, heads, d);
   }
-  const size_t need = dr_seq_backward_workspace_bytes(batch, heads, seq, d);
+  const size_t need = unchunked_backward_bytes(batch, heads, seq, d);
   EDF_REQUIRE(workspace && ws_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
+  if (row_backward(alpha, batch, heads, seq, d))
+    return dr_row_backward_run(stream, q, k, v, beta, grad_out, dq, dk, dv, dbeta, workspace, batch, seq, heads, d,
+                               dtype, per_head, nullptr);
   return dr_seq_backward_run(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch,
-                             seq, heads, d, dtype, beta_mode == EDF_BETA_PER_HEAD, 0, nullptr);
+                             seq, heads, d, dtype, per_head, 0, nullptr);
 }
 int bwd_saved(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
               const void* grad_out, void* dq, void* dk, void* dv, void* dbeta, void* dalpha, const void* fwd_ws,
@@ -98,11 +130,13 @@ int bwd_saved(void* stream, const void* q, const void* k, const void* v, const v
     return dr_chunk_saved_backward_run(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, fwd_ws,
                                        workspace, batch, seq, heads, d);
   }
-  // per-step path: the forward's stored states when its workspace held them, else the
-  // backward recomputes them
-  const size_t need = dr_seq_backward_workspace_bytes(batch, heads, seq, d);
+  // the forward's record when its workspace held one, else the backward recomputes it
+  const size_t need = unchunked_backward_bytes(batch, heads, seq, d);
   EDF_REQUIRE(workspace && ws_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
-  const bool saved = fwd_ws && fwd_ws_bytes >= dr_seq_context_bytes(batch, heads, seq, d);
+  const bool saved = fwd_ws && fwd_ws_bytes >= unchunked_context_bytes(batch, heads, seq, d);
+  if (row_backward(alpha, batch, heads, seq, d))
+    return dr_row_backward_run(stream, q, k, v, beta, grad_out, dq, dk, dv, dbeta, workspace, batch, seq, heads, d,
+                               dtype, per_head, saved ? fwd_ws : nullptr);
   return dr_seq_backward_run(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch,
                              seq, heads, d, dtype, per_head, 0, saved ? (const float*)fwd_ws : nullptr);
 }
@@ -116,7 +150,7 @@ size_t edf_delta_rule_saved_backward_workspace_bytes(int batch, int seq_len, int
   if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
   if (edf::dr_chunk_eligible(seq_len, head_dim, dtype, beta_mode == EDF_BETA_PER_HEAD))
     return edf::dr_chunk_saved_backward_workspace_bytes(batch, seq_len, num_heads, head_dim);
-  return edf::dr_seq_backward_workspace_bytes(batch, num_heads, seq_len, head_dim);
+  return edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim);
 }
 
 int edf_fused_delta_rule_scan_backward_saved(void* stream, const void* q, const void* k, const void* v,
@@ -136,7 +170,7 @@ size_t edf_delta_rule_forward_context_bytes(int batch, int seq_len, int num_head
   if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0 || head_dim > 128) return 0;
   if (edf::dr_chunk_eligible(seq_len, head_dim, dtype, beta_mode == EDF_BETA_PER_HEAD))
     return edf::dr_chunk_workspace_bytes(batch, seq_len, num_heads, head_dim);
-  return edf::dr_seq_context_bytes(batch, num_heads, seq_len, head_dim);
+  return edf::unchunked_context_bytes(batch, num_heads, seq_len, head_dim);
 }
 
 size_t edf_delta_rule_workspace_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype,
@@ -152,7 +186,7 @@ size_t edf_delta_rule_backward_workspace_bytes(int batch, int seq_len, int num_h
   if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
   if (edf::dr_chunk_eligible(seq_len, head_dim, dtype, beta_mode == EDF_BETA_PER_HEAD))
     return edf::dr_chunk_backward_workspace_bytes(batch, seq_len, num_heads, head_dim);
-  return edf::dr_seq_backward_workspace_bytes(batch, num_heads, seq_len, head_dim);
+  return edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim);
 }
 
 int edf_fused_delta_net_scan(void* stream, const void* q, const void* k, const void* v, const void* beta, void* out,

@@ -38,46 +38,6 @@ namespace edf {
 namespace {
 using namespace rowscan;
 
-struct RowArgs {
-  const void *q, *k, *v, *beta, *alpha;
-  void* out;
-  float* ckpt;  // [BH][nck][cw][cw]: the state after each chunk, or null
-  int H, T, d, nrb, cw;
-  int beta_per_head, alpha_per_row;
-};
-
-// What both waves of a block address: buffer resources over the batch row and the lane's byte
-// offsets at step 0 and per step (lanes past d at an offset that reads zero and drops stores).
-template <typename TT> struct RowIO {
-  rsrc_t rQ, rK, rV, rO, rB, rA;
-  unsigned step, base, row0, bbase, bstep, abase, astep;
-  long bh;
-  int i;
-  bool in;
-  EDF_DEVICE RowIO(const RowArgs& p, int li) {
-    const int id = remap_xcd((int)blockIdx.x, (int)gridDim.x);  // a head's row blocks on one XCD
-    bh = id / p.nrb;
-    i = (id % p.nrb) * RW + li;
-    in = i < p.d;
-    const int b = (int)(bh / p.H), h = (int)(bh % p.H);
-    const long rowel = (long)p.T * p.H * p.d, headel = (long)p.T * p.H;
-    const unsigned rowb = (unsigned)(rowel * sizeof(TT)), headb = (unsigned)(headel * sizeof(TT));
-    rQ = make_rsrc((const TT*)p.q + b * rowel, rowb), rK = make_rsrc((const TT*)p.k + b * rowel, rowb);
-    rV = make_rsrc((const TT*)p.v + b * rowel, rowb);
-    rO = make_rsrc(p.out != nullptr ? (const TT*)p.out + b * rowel : (const TT*)p.k, p.out != nullptr ? rowb : 0u);
-    rB = p.beta_per_head ? make_rsrc((const TT*)p.beta + b * headel, headb)
-                         : make_rsrc((const TT*)p.beta + b * rowel, rowb);
-    rA = p.alpha == nullptr ? rB
-         : p.alpha_per_row  ? make_rsrc((const TT*)p.alpha + b * rowel, rowb)
-                            : make_rsrc((const TT*)p.alpha + b * headel, headb);
-    step = (unsigned)((long)p.H * p.d * sizeof(TT));
-    base = (unsigned)((long)h * p.d * sizeof(TT));
-    row0 = in ? base + i * (unsigned)sizeof(TT) : OOB_OFF;
-    const unsigned hstep = (unsigned)(p.H * sizeof(TT)), head0 = in ? h * (unsigned)sizeof(TT) : OOB_OFF;
-    bbase = p.beta_per_head ? head0 : row0, bstep = p.beta_per_head ? hstep : step;
-    abase = p.alpha_per_row ? row0 : head0, astep = p.alpha_per_row ? step : hstep;
-  }
-};
 
 // The decay of the lane's steps; a step past T and a row past d are identities (a = 1; beta = v = 0).
 template <typename TT>
@@ -98,9 +58,6 @@ struct BlockDecay {
     end = pick4(r30, r31, r32, 1.0f, grp);
   }
 };
-
-// Scalars of the block solves: k_m . k_n of the four steps of block r, m < n, at r * 8 + pair(m, n).
-EDF_DEVICE constexpr int pair(int m, int n) { return n * (n - 1) / 2 + m; }
 
 template <typename TT, int DP>
 struct RowShared {
@@ -134,6 +91,11 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_fwd_kern
       if (DECAY) na.load(io.rA, io.astep, CH);
     };
     load();
+    const long rowel = (long)p.T * p.H * p.d;
+    const bool keep = !DECAY && p.err != nullptr;
+    const rsrc_t rE = make_rsrc(keep ? p.err + io.bh / p.H * rowel : p.ckpt, keep ? (unsigned)(rowel * 4) : 0u);
+    const unsigned estep = (unsigned)p.H * p.d * 4;
+    unsigned eoff = io.in ? ((unsigned)(io.bh % p.H) * p.d + io.i) * 4 + (unsigned)grp * estep : OOB_OFF;
     f32x4 U = {0, 0, 0, 0};  // u of the chunk before, decayed to its end
     float dtot = 1.0f;       // decay of the chunk before
     lds_barrier();
@@ -171,12 +133,16 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_fwd_kern
         float y[4], u[4];
         gather4(DECAY ? fmaf(-D.pre, pk[r], v[r]) : v[r] - pk[r], y);
         u[0] = bb[r][0] * y[0];
-        u[1] = bb[r][1] * fmaf(-(DECAY ? g(0, 1) * D.r10 : g(0, 1)), u[0], y[1]);
-        u[2] = bb[r][2] * fmaf(-(DECAY ? g(1, 2) * D.r21 : g(1, 2)), u[1],
-                               fmaf(-(DECAY ? g(0, 2) * D.r20 : g(0, 2)), u[0], y[2]));
-        u[3] = bb[r][3] * fmaf(-(DECAY ? g(2, 3) * D.r32 : g(2, 3)), u[2],
-                               fmaf(-(DECAY ? g(1, 3) * D.r31 : g(1, 3)), u[1],
-                                    fmaf(-(DECAY ? g(0, 3) * D.r30 : g(0, 3)), u[0], y[3])));
+        y[1] = fmaf(-(DECAY ? g(0, 1) * D.r10 : g(0, 1)), u[0], y[1]);
+        u[1] = bb[r][1] * y[1];
+        y[2] = fmaf(-(DECAY ? g(1, 2) * D.r21 : g(1, 2)), u[1],
+                    fmaf(-(DECAY ? g(0, 2) * D.r20 : g(0, 2)), u[0], y[2]));
+        u[2] = bb[r][2] * y[2];
+        y[3] = fmaf(-(DECAY ? g(2, 3) * D.r32 : g(2, 3)), u[2],
+                    fmaf(-(DECAY ? g(1, 3) * D.r31 : g(1, 3)), u[1],
+                         fmaf(-(DECAY ? g(0, 3) * D.r30 : g(0, 3)), u[0], y[3])));
+        u[3] = bb[r][3] * y[3];
+        if (!DECAY && p.err != nullptr) bstore<float>(rE, eoff + 4 * r * estep, pick4(y[0], y[1], y[2], y[3], grp));
         const float uo = pick4(u[0], u[1], u[2], u[3], grp);
         const float ue = DECAY ? uo * D.end : uo;
         if (r < 3) pk = mfma4(G[r], ue, DECAY ? pk * D.all : pk);
@@ -188,6 +154,7 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_fwd_kern
         U[r] = ue;
         raw[r] = uo;
       }
+      eoff += CH * estep;
       sh.u[b][l] = raw;
       lds_barrier();
     }
@@ -227,8 +194,9 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_fwd_kern
           for (int jt = 0; jt < W / 16; ++jt) S[jt] *= dtot;
         }
         state_add<W>(S, kc, U);
-        if (p.ckpt != nullptr && io.i < p.cw) {
-          float* cp = p.ckpt + ((io.bh * nch + c - 1) * p.cw + io.i) * p.cw + W * half + 4 * grp;
+        if (p.ckpt != nullptr && io.i < p.cw && (DECAY || (c % (CPS / CH) == 0 && c < nch))) {
+          const long slot = DECAY ? io.bh * nch + c - 1 : io.bh * ((p.T + CPS - 1) / CPS - 1) + c / (CPS / CH) - 1;
+          float* cp = p.ckpt + (slot * p.cw + io.i) * p.cw + W * half + 4 * grp;
 #pragma unroll
           for (int jt = 0; jt < W / 16; ++jt)
             if (W * half + 16 * jt < p.cw) *(f32x4*)(cp + 16 * jt) = S[jt];
@@ -355,18 +323,19 @@ void by_width(hipStream_t s, const RowArgs& a, unsigned grid) {
 
 }  // namespace
 
-// Whether the row-wise kernels take a call: a batch row addressed by 31-bit byte offsets.
-bool dr_row_takes(int batch, int heads, int seq, int d, int dtype) {
-  const long bytes = (long)(seq + 6 * CH) * heads * d * (dtype == EDF_BF16 ? 2 : 4);
+// Whether the row-wise kernels take a call: a batch row, of float32 too (err), addressed by 31-bit
+// byte offsets.
+bool dr_row_takes(int batch, int heads, int seq, int d) {
+  const long bytes = (long)(seq + 6 * CH) * heads * d * 4;
   return d <= 128 && bytes < (1L << 31) && (long)batch * heads * ((d + RW - 1) / RW) < (1L << 31);
 }
 
-// ckpt (may be null): the states after every 16 steps, [BH][chunks][cw][cw] with cw columns >= d
+// ckpt, err, cw: see RowArgs (null: no backward follows)
 int dr_row_run(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
                void* out, int batch, int seq, int heads, int d, int dtype, int beta_per_head, int alpha_per_row,
-               float* ckpt, int cw) {
+               float* ckpt, float* err, int cw) {
   RowArgs a{};
-  a.q = q, a.k = k, a.v = v, a.beta = beta, a.alpha = alpha, a.out = out, a.ckpt = ckpt;
+  a.q = q, a.k = k, a.v = v, a.beta = beta, a.alpha = alpha, a.out = out, a.ckpt = ckpt, a.err = err;
   a.H = heads, a.T = seq, a.d = d, a.cw = cw;
   a.nrb = ((ckpt != nullptr ? cw : d) + RW - 1) / RW;  // with states kept, the padding rows (zero) too
   a.beta_per_head = beta_per_head, a.alpha_per_row = alpha_per_row;

@@ -30,10 +30,10 @@
 #include "edf_common.hpp"
 
 namespace edf {
-bool dr_row_takes(int batch, int heads, int seq, int d, int dtype);
+bool dr_row_takes(int batch, int heads, int seq, int d);
 int dr_row_run(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
                void* out, int batch, int seq, int heads, int d, int dtype, int beta_per_head, int alpha_per_row,
-               float* ckpt, int cw);
+               float* ckpt, float* err, int cw);
 namespace {
 
 constexpr int CK = 16;  // steps per staged chunk / checkpoint interval
@@ -468,9 +468,10 @@ size_t dr_seq_context_bytes(int batch, int heads, int seq, int d) {
 int dr_seq_run(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
                void* out, int batch, int seq, int heads, int d, int dtype, int beta_per_head, int alpha_per_row,
                float* context) {
-  if (dr_row_takes(batch, heads, seq, d, dtype))
+  // (a call without decay that keeps states, and that the row scans take, does not come here)
+  if (dr_row_takes(batch, heads, seq, d))
     return dr_row_run(stream, q, k, v, beta, alpha, out, batch, seq, heads, d, dtype, beta_per_head, alpha_per_row,
-                      context, pad_dim(d));
+                      context, nullptr, pad_dim(d));
   DRArgs a{};
   a.q = q; a.k = k; a.v = v; a.beta = beta; a.alpha = alpha; a.out = out;
   a.ckpt = context;  // also store the checkpoints (one pass writes both)

@@ -23,6 +23,7 @@ namespace rowscan {
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 constexpr int CH = 16;  // steps per chunk
 constexpr int RW = 16;  // state rows per wave
+constexpr int CPS = 64; // steps between the states kept for a backward without decay
 
 EDF_DEVICE int sigma(int x) { return 4 * (x & 3) + (x >> 2); }
 
@@ -134,6 +135,27 @@ EDF_DEVICE void state_dots(const RowFrag<float, W>& a, const RowFrag<float, W>& 
     }
 }
 
+template <int W>
+EDF_DEVICE f32x4 state_dot(const RowFrag<bf16, W>& a, const f32x4 (&S)[W / 16]) {
+  f32x4 c[3] = {};
+#pragma unroll
+  for (int kk = 0; kk < W / 32; ++kk) {
+    const Split4 s0 = split4(S[2 * kk]), s1 = split4(S[2 * kk + 1]);
+#pragma unroll
+    for (int n = 0; n < 3; ++n) c[n] = mfma32k(a.f[kk], cat4(s0.part[n], s1.part[n]), c[n]);
+  }
+  return (c[2] + c[1]) + c[0];
+}
+template <int W>
+EDF_DEVICE f32x4 state_dot(const RowFrag<float, W>& a, const f32x4 (&S)[W / 16]) {
+  f32x4 c[2] = {};
+#pragma unroll
+  for (int jt = 0; jt < W / 16; ++jt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c[e & 1] = mfma4(a.f[jt][e], S[jt][e], c[e & 1]);
+  return c[0] + c[1];
+}
+
 // The A operands of S += u^T tile over W columns: for bf16 element r of f[jt] is step 4 r + grp, column
 // 16 jt + li; for float f[jt][r].
 template <typename TT, int W> struct ColFrag;
@@ -177,6 +199,33 @@ EDF_DEVICE void state_add(f32x4 (&S)[W / 16], const ColFrag<float, W>& k, f32x4 
     for (int jt = 0; jt < W / 16; ++jt) S[jt] = mfma4(k.f[jt][r], u[r], S[jt]);
 }
 
+// S[row][column] += sum over the chunk's steps of x[step][row] q[step][column] - w[step][row] k[step][column],
+// x given as stored (bf16: exact, so it shares a product with the first part of w).
+template <int W>
+EDF_DEVICE void state_add2(f32x4 (&S)[W / 16], const ColFrag<bf16, W>& q, const unsigned short (&x)[4],
+                           const ColFrag<bf16, W>& k, f32x4 w) {
+  typedef __attribute__((ext_vector_type(4))) unsigned short u16x4;
+  const Split4 s = split4(-w);
+  const u16x4 xv = {x[0], x[1], x[2], x[3]};
+  const bf16x8 xh = cat4(__builtin_bit_cast(bf16x4, xv), s.part[0]), ml = cat4(s.part[1], s.part[2]);
+#pragma unroll
+  for (int jt = 0; jt < W / 16; ++jt) S[jt] = mfma32k(cat4(k.f[jt], k.f[jt]), ml, S[jt]);
+#pragma unroll
+  for (int jt = 0; jt < W / 16; ++jt) S[jt] = mfma32k(cat4(q.f[jt], k.f[jt]), xh, S[jt]);
+}
+template <int W>
+EDF_DEVICE void state_add2(f32x4 (&S)[W / 16], const ColFrag<float, W>& q, const unsigned (&x)[4],
+                           const ColFrag<float, W>& k, f32x4 w) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int jt = 0; jt < W / 16; ++jt) S[jt] = mfma4(q.f[jt][r], bits_f32(x[r]), S[jt]);
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int jt = 0; jt < W / 16; ++jt) S[jt] = mfma4(k.f[jt][r], -w[r], S[jt]);
+}
+
 // Value of each of the four groups, in every lane of the same li.  The swaps are not volatile (unlike
 // swap16 / swap32): a gather is a function of its input, free to move among the chunk's other work.
 EDF_DEVICE void gather4(float x, float (&v)[4]) {
@@ -195,8 +244,9 @@ EDF_DEVICE float lane_value(float v, int lane) {
 }
 
 // ---- 16 steps of [B, T, H, d] rows: memory -> registers (a chunk ahead) -> LDS -------------------
-// A lane's byte offset runs ahead by 16 steps per load.  Steps past T and columns past d read as
-// zero (offsets past the batch row; the caller keeps the steps it runs ahead below 2^31 bytes).
+// A lane's byte offset moves by 16 steps per load, forward or back.  Steps outside 0 .. T - 1 and
+// columns past d read as zero (their offsets lie past the batch row, modulo 2^32; the caller keeps
+// the steps it runs ahead below 2^31 bytes; a padding column of a step before 0 may read something).
 // VEC: d is a multiple of 8 (bf16) or 4 (float) and rows start on 4-byte boundaries, so a row's
 // 16-byte pieces lie whole inside or outside it.
 template <typename TT, int DP, bool VEC> struct TileRegs;
@@ -209,7 +259,7 @@ template <typename TT, int DP> struct TileRegs<TT, DP, true> {
   unsigned off;
   EDF_DEVICE void at(unsigned base, unsigned stepb, int t0, int d, int l) {
     const int col = (l % PPR) * EPV;
-    off = col < d ? base + (unsigned)(t0 + l / PPR) * stepb + col * (unsigned)sizeof(TT) : OOB_OFF;
+    off = (col < d ? base + col * (unsigned)sizeof(TT) : OOB_OFF) + (unsigned)(t0 + l / PPR) * stepb;
   }
   EDF_DEVICE void load(rsrc_t r, unsigned stepb, int advance) {
 #pragma unroll
@@ -266,6 +316,53 @@ EDF_DEVICE void lds_barrier() {
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
+
+struct RowArgs {
+  const void *q, *k, *v, *beta, *alpha;
+  void* out;
+  // what a backward reads, or null.  With a decay, for the per-step backward: the state after each
+  // chunk, [BH][chunks][cw][cw].  Without, for delta_rule_row_bwd.hip: the state before every
+  // CPS steps but the first, [BH][ceil(T / CPS) - 1][cw][cw], and err, [B, T, H, d].
+  float *ckpt, *err;
+  int H, T, d, nrb, cw;
+  int beta_per_head, alpha_per_row;
+};
+
+// What a block's waves address: buffer resources over the batch row and the lane's byte offsets at
+// step 0 and per step (lanes past d at an offset that reads zero and drops stores).
+template <typename TT> struct RowIO {
+  rsrc_t rQ, rK, rV, rO, rB, rA;
+  unsigned step, base, row0, bbase, bstep, abase, astep;
+  long bh;
+  int i;
+  bool in;
+  EDF_DEVICE RowIO(const RowArgs& p, int li) {
+    const int id = remap_xcd((int)blockIdx.x, (int)gridDim.x);  // a head's row blocks on one XCD
+    bh = id / p.nrb;
+    i = (id % p.nrb) * RW + li;
+    in = i < p.d;
+    const int b = (int)(bh / p.H), h = (int)(bh % p.H);
+    const long rowel = (long)p.T * p.H * p.d, headel = (long)p.T * p.H;
+    const unsigned rowb = (unsigned)(rowel * sizeof(TT)), headb = (unsigned)(headel * sizeof(TT));
+    rQ = make_rsrc((const TT*)p.q + b * rowel, rowb), rK = make_rsrc((const TT*)p.k + b * rowel, rowb);
+    rV = make_rsrc((const TT*)p.v + b * rowel, rowb);
+    rO = make_rsrc(p.out != nullptr ? (const TT*)p.out + b * rowel : (const TT*)p.k, p.out != nullptr ? rowb : 0u);
+    rB = p.beta_per_head ? make_rsrc((const TT*)p.beta + b * headel, headb)
+                         : make_rsrc((const TT*)p.beta + b * rowel, rowb);
+    rA = p.alpha == nullptr ? rB
+         : p.alpha_per_row  ? make_rsrc((const TT*)p.alpha + b * rowel, rowb)
+                            : make_rsrc((const TT*)p.alpha + b * headel, headb);
+    step = (unsigned)((long)p.H * p.d * sizeof(TT));
+    base = (unsigned)((long)h * p.d * sizeof(TT));
+    row0 = in ? base + i * (unsigned)sizeof(TT) : OOB_OFF;
+    const unsigned hstep = (unsigned)(p.H * sizeof(TT)), head0 = in ? h * (unsigned)sizeof(TT) : OOB_OFF;
+    bbase = p.beta_per_head ? head0 : row0, bstep = p.beta_per_head ? hstep : step;
+    abase = p.alpha_per_row ? row0 : head0, astep = p.alpha_per_row ? step : hstep;
+  }
+};
+
+// Scalars of the block solves: k_m . k_n of the four steps of block r, m < n, at r * 8 + pair(m, n).
+EDF_DEVICE constexpr int pair(int m, int n) { return n * (n - 1) / 2 + m; }
 
 }  // namespace rowscan
 }  // namespace edf
