@@ -1,9 +1,8 @@
 // C-ABI entry points of the delta rule (DeltaNet / GatedDeltaNet), forward and backward.
 // Dispatch: the chunked MFMA kernels (delta_rule_chunk.hip) take bf16, per-head beta,
 // head_dim 64 .. 128 (a multiple of 8; zero-padded to 128 inside), seq >= 64 (forward and
-// backward); every other case takes the row scans (delta_rule_row.hip) forward, and backward
-// the row scans without a decay (delta_rule_row_bwd.hip), the exact per-step kernels
-// (delta_rule_seq.hip) with one.
+// backward); every other case takes the row scans (delta_rule_row.hip, delta_rule_row_bwd.hip), the
+// exact per-step kernels (delta_rule_seq.hip) only batch rows of 2 GiB and more.
 #include "edf_abi.hpp"
 
 namespace edf {
@@ -17,13 +16,15 @@ int dr_seq_backward_run(void* stream, const void* q, const void* k, const void* 
                         void* dalpha, void* workspace, int batch, int seq, int heads, int d, int dtype,
                         int beta_per_head, int alpha_per_row, const float* context);
 bool dr_row_takes(int batch, int heads, int seq, int d);
-size_t dr_row_context_bytes(int batch, int heads, int seq, int d);
-int dr_row_record_run(void* stream, const void* q, const void* k, const void* v, const void* beta, void* out,
-                      int batch, int seq, int heads, int d, int dtype, int beta_per_head, void* context);
-size_t dr_row_backward_workspace_bytes(int batch, int heads, int seq, int d);
+size_t dr_row_context_bytes(int batch, int heads, int seq, int d, bool decay);
+int dr_row_record_run(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
+                      void* out, int batch, int seq, int heads, int d, int dtype, int beta_per_head,
+                      int alpha_per_row, void* context);
+size_t dr_row_backward_workspace_bytes(int batch, int heads, int seq, int d, bool decay);
 int dr_row_backward_run(void* stream, const void* q, const void* k, const void* v, const void* beta,
-                        const void* grad_out, void* dq, void* dk, void* dv, void* dbeta, void* workspace, int batch,
-                        int seq, int heads, int d, int dtype, int beta_per_head, const void* context);
+                        const void* alpha, const void* grad_out, void* dq, void* dk, void* dv, void* dbeta,
+                        void* dalpha, void* workspace, int batch, int seq, int heads, int d, int dtype,
+                        int beta_per_head, int alpha_per_row, const void* context);
 bool dr_chunk_eligible(int seq, int d, int dtype, int beta_per_head);
 size_t dr_chunk_workspace_bytes(int batch, int seq, int heads, int d);
 int dr_chunk_run(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
@@ -48,20 +49,38 @@ int check_dr(int batch, int seq, int heads, int d, int dtype, int beta_mode) {
   return EDF_OK;
 }
 
-// Whether the row scans take a call's backward too (and its forward's record is theirs).
-bool row_backward(const void* alpha, int batch, int heads, int seq, int d) {
-  return alpha == nullptr && dr_row_takes(batch, heads, seq, d);
-}
-
-// The size queries do not know whether a decay is given: the larger of the two paths' needs.
+// The record of a forward and the workspace of a backward off the chunked path: the row scans' (the
+// queries of the delta rule do not know whether a decay is given: the larger need), the per-step
+// kernels' for batch rows of 2 GiB and more.
 size_t unchunked_context_bytes(int batch, int heads, int seq, int d) {
-  const size_t a = dr_seq_context_bytes(batch, heads, seq, d), b = dr_row_context_bytes(batch, heads, seq, d);
-  return a > b ? a : b;
+  if (!dr_row_takes(batch, heads, seq, d)) return dr_seq_context_bytes(batch, heads, seq, d);
+  return dr_row_context_bytes(batch, heads, seq, d, true);
 }
 size_t unchunked_backward_bytes(int batch, int heads, int seq, int d) {
-  const size_t a = dr_seq_backward_workspace_bytes(batch, heads, seq, d);
-  const size_t b = dr_row_backward_workspace_bytes(batch, heads, seq, d);
-  return a > b ? a : b;
+  if (!dr_row_takes(batch, heads, seq, d)) return dr_seq_backward_workspace_bytes(batch, heads, seq, d);
+  return dr_row_backward_workspace_bytes(batch, heads, seq, d, true);
+}
+
+int unchunked_fwd(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
+                  void* out, int batch, int seq, int heads, int d, int dtype, int beta_per_head, int alpha_per_row,
+                  void* context) {
+  if (context != nullptr && dr_row_takes(batch, heads, seq, d))
+    return dr_row_record_run(stream, q, k, v, beta, alpha, out, batch, seq, heads, d, dtype, beta_per_head,
+                             alpha_per_row, context);
+  return dr_seq_run(stream, q, k, v, beta, alpha, out, batch, seq, heads, d, dtype, beta_per_head, alpha_per_row,
+                    (float*)context);
+}
+
+// context null: the record is recomputed
+int unchunked_bwd(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
+                  const void* grad_out, void* dq, void* dk, void* dv, void* dbeta, void* dalpha, void* workspace,
+                  int batch, int seq, int heads, int d, int dtype, int beta_per_head, int alpha_per_row,
+                  const void* context) {
+  if (dr_row_takes(batch, heads, seq, d))
+    return dr_row_backward_run(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch,
+                               seq, heads, d, dtype, beta_per_head, alpha_per_row, context);
+  return dr_seq_backward_run(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch, seq,
+                             heads, d, dtype, beta_per_head, alpha_per_row, (const float*)context);
 }
 
 int fwd(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha, void* out,
@@ -78,14 +97,10 @@ int fwd(void* stream, const void* q, const void* k, const void* v, const void* b
     return dr_chunk_run(stream, q, k, v, beta, alpha, out, workspace, batch, seq, heads, d);
   }
   // a workspace of edf_delta_rule_forward_context_bytes() (optional) also receives what the saved
-  // backward reads: the states every 16 steps, or without a decay every 64 and err
-  if (row_backward(alpha, batch, heads, seq, d) && workspace &&
-      ws_bytes >= unchunked_context_bytes(batch, heads, seq, d))
-    return dr_row_record_run(stream, q, k, v, beta, out, batch, seq, heads, d, dtype, per_head, workspace);
-  const bool keep = !row_backward(alpha, batch, heads, seq, d) && workspace &&
-                    ws_bytes >= unchunked_context_bytes(batch, heads, seq, d);
-  return dr_seq_run(stream, q, k, v, beta, alpha, out, batch, seq, heads, d, dtype, per_head, 0,
-                    keep ? (float*)workspace : nullptr);
+  // backward reads
+  const bool keep = workspace && ws_bytes >= unchunked_context_bytes(batch, heads, seq, d);
+  return unchunked_fwd(stream, q, k, v, beta, alpha, out, batch, seq, heads, d, dtype, per_head, 0,
+                       keep ? workspace : nullptr);
 }
 
 int bwd(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
@@ -104,11 +119,8 @@ int bwd(void* stream, const void* q, const void* k, const void* v, const void* b
   }
   const size_t need = unchunked_backward_bytes(batch, heads, seq, d);
   EDF_REQUIRE(workspace && ws_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
-  if (row_backward(alpha, batch, heads, seq, d))
-    return dr_row_backward_run(stream, q, k, v, beta, grad_out, dq, dk, dv, dbeta, workspace, batch, seq, heads, d,
-                               dtype, per_head, nullptr);
-  return dr_seq_backward_run(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch,
-                             seq, heads, d, dtype, per_head, 0, nullptr);
+  return unchunked_bwd(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch, seq, heads,
+                       d, dtype, per_head, 0, nullptr);
 }
 int bwd_saved(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
               const void* grad_out, void* dq, void* dk, void* dv, void* dbeta, void* dalpha, const void* fwd_ws,
@@ -134,11 +146,8 @@ int bwd_saved(void* stream, const void* q, const void* k, const void* v, const v
   const size_t need = unchunked_backward_bytes(batch, heads, seq, d);
   EDF_REQUIRE(workspace && ws_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
   const bool saved = fwd_ws && fwd_ws_bytes >= unchunked_context_bytes(batch, heads, seq, d);
-  if (row_backward(alpha, batch, heads, seq, d))
-    return dr_row_backward_run(stream, q, k, v, beta, grad_out, dq, dk, dv, dbeta, workspace, batch, seq, heads, d,
-                               dtype, per_head, saved ? fwd_ws : nullptr);
-  return dr_seq_backward_run(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch,
-                             seq, heads, d, dtype, per_head, 0, saved ? (const float*)fwd_ws : nullptr);
+  return unchunked_bwd(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch, seq, heads,
+                       d, dtype, per_head, 0, saved ? fwd_ws : nullptr);
 }
 }  // namespace
 }  // namespace edf
@@ -226,12 +235,11 @@ int edf_fused_gated_delta_net_scan_backward(void* stream, const void* q, const v
                   workspace_bytes, batch, seq_len, num_heads, head_dim, dtype, beta_mode);
 }
 
-// KDA: per-row log-space decay, per-head beta; always the exact per-step kernels (the
-// chunked form takes one decay per head).
+// KDA: per-row log-space decay, per-head beta; never the chunked kernels (which take one decay per head).
 size_t edf_kda_scan_backward_workspace_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype) {
   (void)dtype;
   if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
-  return edf::dr_seq_backward_workspace_bytes(batch, num_heads, seq_len, head_dim);
+  return edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim);
 }
 
 int edf_fused_kda_scan(void* stream, const void* q, const void* k, const void* v, const void* alpha,
@@ -239,7 +247,7 @@ int edf_fused_kda_scan(void* stream, const void* q, const void* k, const void* v
   int rc = edf::check_dr(batch, seq_len, num_heads, head_dim, dtype, EDF_BETA_PER_HEAD);
   if (rc) return rc;
   EDF_REQUIRE(q && k && v && alpha && beta && out, EDF_ERR_INVALID_ARG, "null tensor pointer");
-  return edf::dr_seq_run(stream, q, k, v, beta, alpha, out, batch, seq_len, num_heads, head_dim, dtype, 1, 1,
+  return edf::unchunked_fwd(stream, q, k, v, beta, alpha, out, batch, seq_len, num_heads, head_dim, dtype, 1, 1,
                          nullptr);
 }
 
@@ -253,16 +261,16 @@ int edf_fused_kda_scan_backward(void* stream, const void* q, const void* k, cons
   if (rc) return rc;
   EDF_REQUIRE(q && k && v && alpha && beta && grad_out && grad_q && grad_k && grad_v && grad_alpha && grad_beta,
               EDF_ERR_INVALID_ARG, "null tensor pointer");
-  const size_t need = edf::dr_seq_backward_workspace_bytes(batch, num_heads, seq_len, head_dim);
+  const size_t need = edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim);
   EDF_REQUIRE(workspace && workspace_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
-  return edf::dr_seq_backward_run(stream, q, k, v, beta, alpha, grad_out, grad_q, grad_k, grad_v, grad_beta,
+  return edf::unchunked_bwd(stream, q, k, v, beta, alpha, grad_out, grad_q, grad_k, grad_v, grad_beta,
                                   grad_alpha, workspace, batch, seq_len, num_heads, head_dim, dtype, 1, 1, nullptr);
 }
 
 size_t edf_kda_scan_context_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype) {
   (void)dtype;
   if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0 || head_dim > 128) return 0;
-  return edf::dr_seq_context_bytes(batch, num_heads, seq_len, head_dim);
+  return edf::unchunked_context_bytes(batch, num_heads, seq_len, head_dim);
 }
 
 int edf_fused_kda_scan_with_context(void* stream, const void* q, const void* k, const void* v, const void* alpha,
@@ -271,10 +279,10 @@ int edf_fused_kda_scan_with_context(void* stream, const void* q, const void* k, 
   int rc = edf::check_dr(batch, seq_len, num_heads, head_dim, dtype, EDF_BETA_PER_HEAD);
   if (rc) return rc;
   EDF_REQUIRE(q && k && v && alpha && beta && out, EDF_ERR_INVALID_ARG, "null tensor pointer");
-  const size_t need = edf::dr_seq_context_bytes(batch, num_heads, seq_len, head_dim);
+  const size_t need = edf::unchunked_context_bytes(batch, num_heads, seq_len, head_dim);
   EDF_REQUIRE(context && context_bytes >= need, EDF_ERR_WORKSPACE, "context too small: need %zu bytes", need);
-  return edf::dr_seq_run(stream, q, k, v, beta, alpha, out, batch, seq_len, num_heads, head_dim, dtype, 1, 1,
-                         (float*)context);
+  return edf::unchunked_fwd(stream, q, k, v, beta, alpha, out, batch, seq_len, num_heads, head_dim, dtype, 1, 1,
+                         context);
 }
 
 int edf_fused_kda_scan_backward_saved(void* stream, const void* q, const void* k, const void* v, const void* alpha,
@@ -286,14 +294,14 @@ int edf_fused_kda_scan_backward_saved(void* stream, const void* q, const void* k
   if (rc) return rc;
   EDF_REQUIRE(q && k && v && alpha && beta && grad_out && grad_q && grad_k && grad_v && grad_alpha && grad_beta,
               EDF_ERR_INVALID_ARG, "null tensor pointer");
-  const size_t needc = edf::dr_seq_context_bytes(batch, num_heads, seq_len, head_dim);
+  const size_t needc = edf::unchunked_context_bytes(batch, num_heads, seq_len, head_dim);
   EDF_REQUIRE(context && context_bytes >= needc, EDF_ERR_WORKSPACE,
               "context too small: need the %zu bytes the forward filled", needc);
-  const size_t need = edf::dr_seq_backward_workspace_bytes(batch, num_heads, seq_len, head_dim);
+  const size_t need = edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim);
   EDF_REQUIRE(workspace && workspace_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
-  return edf::dr_seq_backward_run(stream, q, k, v, beta, alpha, grad_out, grad_q, grad_k, grad_v, grad_beta,
+  return edf::unchunked_bwd(stream, q, k, v, beta, alpha, grad_out, grad_q, grad_k, grad_v, grad_beta,
                                   grad_alpha, workspace, batch, seq_len, num_heads, head_dim, dtype, 1, 1,
-                                  (const float*)context);
+                                  context);
 }
 
 }  // extern "C"

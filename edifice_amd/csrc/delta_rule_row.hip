@@ -39,26 +39,6 @@ namespace {
 using namespace rowscan;
 
 
-// The decay of the lane's steps; a step past T and a row past d are identities (a = 1; beta = v = 0).
-template <typename TT>
-EDF_DEVICE float decay_of(typename Bits<TT>::type raw, bool live, int alpha_per_row) {
-  const float v = bits_f32(raw);
-  return live ? (alpha_per_row ? __expf(v) : v) : 1.0f;
-}
-
-// Decays within a block of four steps: rMN from after step n to step m, a0 of the first step, all of
-// the block, pre from the block's start to the lane's step, end from after the lane's step.
-struct BlockDecay {
-  float a0, r10, r20, r30, r21, r31, r32, all, pre, end;
-  EDF_DEVICE BlockDecay(const float (&a)[4], int grp) {
-    a0 = a[0], r10 = a[1], r21 = a[2], r32 = a[3];
-    r31 = r32 * r21, r20 = r21 * r10, r30 = r32 * r20;
-    all = r30 * a0;
-    pre = pick4(a0, r10 * a0, r20 * a0, all, grp);
-    end = pick4(r30, r31, r32, 1.0f, grp);
-  }
-};
-
 template <typename TT, int DP>
 struct RowShared {
   static constexpr int LD = tile_ld<TT, DP>();
@@ -92,8 +72,8 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_fwd_kern
     };
     load();
     const long rowel = (long)p.T * p.H * p.d;
-    const bool keep = !DECAY && p.err != nullptr;
-    const rsrc_t rE = make_rsrc(keep ? p.err + io.bh / p.H * rowel : p.ckpt, keep ? (unsigned)(rowel * 4) : 0u);
+    const bool keep = p.err != nullptr;
+    const rsrc_t rE = make_rsrc(keep ? (const void*)(p.err + io.bh / p.H * rowel) : p.k, keep ? (unsigned)(rowel * 4) : 0u);
     const unsigned estep = (unsigned)p.H * p.d * 4;
     unsigned eoff = io.in ? ((unsigned)(io.bh % p.H) * p.d + io.i) * 4 + (unsigned)grp * estep : OOB_OFF;
     f32x4 U = {0, 0, 0, 0};  // u of the chunk before, decayed to its end
@@ -142,7 +122,7 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_fwd_kern
                     fmaf(-(DECAY ? g(1, 3) * D.r31 : g(1, 3)), u[1],
                          fmaf(-(DECAY ? g(0, 3) * D.r30 : g(0, 3)), u[0], y[3])));
         u[3] = bb[r][3] * y[3];
-        if (!DECAY && p.err != nullptr) bstore<float>(rE, eoff + 4 * r * estep, pick4(y[0], y[1], y[2], y[3], grp));
+        if (keep) bstore<float>(rE, eoff + 4 * r * estep, pick4(y[0], y[1], y[2], y[3], grp));
         const float uo = pick4(u[0], u[1], u[2], u[3], grp);
         const float ue = DECAY ? uo * D.end : uo;
         if (r < 3) pk = mfma4(G[r], ue, DECAY ? pk * D.all : pk);

@@ -1,6 +1,6 @@
-// Delta rule without decay (DeltaNet), backward for per-row beta (and float32, or a head_dim that the
-// chunked kernels do not take), from what the row-scan forward keeps (err and the state every 64 steps;
-// delta_rule_row.hip).  Two kernels:
+// Delta rule, backward for per-row beta or decay (and float32, or a head_dim that the chunked kernels
+// do not take), from what the row-scan forward keeps (err and states; delta_rule_row.hip).
+// Without a decay (DeltaNet), two kernels:
 //
 // 1. The reverse scan, 16 steps at a time in the form of the forward: with dS the gradient of the state
 //    after a step, x_t = do_t,
@@ -17,6 +17,12 @@
 //    lib/edifice/cuda/fused_scan.ex:1257-1431), dv = w, dbeta = err du: contractions over the rows
 //    and over the steps, in float32 on v_mfma_f32_32x32x2_f32.  The sums over all rows of a head are inside
 //    one workgroup, so there are no per-row-block partials to write and add.
+// With a decay (GatedDeltaNet, KDA) the same two passes, the gradients per 16 steps: decays per row do not
+// factor out of M and N over more steps than a short product per pair, so those sums over the rows, and
+// the decay's gradient <dS_t - w_t k_t^T, S_{t-1}>, are formed one row per lane (dr_row_decay_grad_kernel).
+// Forward and backward, against one workgroup per 16 rows stepping through the sequence with partial dq and
+// dk per row block (its time is the chain of T steps): KDA 4x1000x8x128 bf16 875 -> 487 us (scan 92,
+// gradients 293), GatedDeltaNet 2x777x8x64 float32 436 -> 235.
 #include "edf_abi.hpp"
 #include "edf_common.hpp"
 #include "edf_row_scan.hpp"
@@ -28,7 +34,7 @@ int dr_row_run(void* stream, const void* q, const void* k, const void* v, const 
 namespace {
 using namespace rowscan;
 
-template <typename TT, int DP>
+template <typename TT, int DP, bool DECAY>
 struct RevShared {
   static constexpr int LD = tile_ld<TT, DP>();
   static constexpr int SW = DP >= 64 ? 2 : 1;  // state waves
@@ -37,14 +43,18 @@ struct RevShared {
   f32x4 pk[2][SW][64];                          // state products of k
   f32x4 x[2][64];                               // do terms of a chunk and of the one after it
   f32x4 g[2][64], gx[2][64];                    // Gram tiles of a chunk, and of the one after with it
+  f32x4 h[DECAY ? 2 : 1][DECAY ? 64 : 1], hx[DECAY ? 2 : 1][DECAY ? 64 : 1];  // the q . k tiles of the same
   float gs[2][32];                              // solve scalars
 };
 
 // p.v is do; du [B, T, H, d], p.ckpt the gradients of the states [BH][ceil(T / CPS) - 1][cw][cw] after
 // each CPS steps but the last.
-template <typename TT, int DP, bool VEC>
+// With a decay (DECAY), the state gradient runs back as dS <- a_t (dS + do_t q_t^T - w_t k_t^T), and p.ckpt
+// takes it after every chunk but the last, [BH][chunks][cw][cw]; the do terms of the chunk and of the
+// one after it then decay with the others in the chain, and x holds only those inside a block of four.
+template <typename TT, int DP, bool DECAY, bool VEC>
 __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_rev_kernel(const RowArgs p, float* du) {
-  typedef RevShared<TT, DP> Sh;
+  typedef RevShared<TT, DP, DECAY> Sh;
   constexpr int LD = Sh::LD, SW = Sh::SW, W = DP / SW;
   __shared__ __attribute__((aligned(16))) Sh sh;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -53,51 +63,87 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_rev_kern
   const int nch = (p.T + CH - 1) / CH, tl = (nch - 1) * CH;
 
   if (wave == 0) {  // chain
-    GateRegs<TT> nb;
+    GateRegs<TT> nb, na, nd;
     nb.at(io.bbase, io.bstep, tl, grp);
-    nb.load(io.rB, io.bstep, -CH);
+    if (DECAY) na.at(io.abase, io.astep, tl, grp), nd.at(io.row0, io.step, tl, grp);
+    auto load = [&]() {
+      nb.load(io.rB, io.bstep, -CH);
+      if (DECAY) na.load(io.rA, io.astep, -CH), nd.load(io.rV, io.step, -CH);
+    };
+    load();
     const long rowel = (long)p.T * p.H * p.d;
     const rsrc_t rU = make_rsrc(du + io.bh / p.H * rowel, (unsigned)(rowel * 4));
     const unsigned ustep = (unsigned)p.H * p.d * 4;
     unsigned uoff = (io.in ? ((unsigned)(io.bh % p.H) * p.d + io.i) * 4 : OOB_OFF) + (unsigned)(tl + grp) * ustep;
-    f32x4 Wn = {0, 0, 0, 0};  // w of the chunk after, negated
+    f32x4 Wn = {0, 0, 0, 0}, Dn = {0, 0, 0, 0};  // -w and do of the chunk after, decayed to its start
+    float dtot = 1.0f;                           // its decay
     lds_barrier();
     for (int j = 0; j < nch; ++j) {
-      const int b = j & 1;
-      f32x4 e = sh.x[b][l];
+      const int b = j & 1, t0 = (nch - 1 - j) * CH;
+      const f32x4 x = sh.x[b][l];
+      f32x4 e = {0, 0, 0, 0};
       if (j > 0) {
-        e += sh.pk[b][0][l];
+        e = sh.pk[b][0][l];
         if (SW == 2) e += sh.pk[b][SW - 1][l];
       }
+      e = DECAY ? e * dtot : e + x;
       const f32x4 G = sh.g[b][l], Gx = sh.gx[b][l];
+      f32x4 H, Hx;
+      if (DECAY) H = sh.h[b][l], Hx = sh.hx[b][l];
       f32x4 gs[4][2];
 #pragma unroll
       for (int r = 0; r < 4; ++r) gs[r][0] = *(const f32x4*)&sh.gs[b][8 * r], gs[r][1] = *(const f32x4*)&sh.gs[b][8 * r + 4];
-      float bb[4][4];
+      float bb[4][4], aa[4][4], dc[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) gather4(bits_f32(nb.v[r]), bb[r]);
-      nb.load(io.rB, io.bstep, -CH);
+      for (int r = 0; r < 4; ++r) {
+        gather4(bits_f32(nb.v[r]), bb[r]);
+        if (DECAY) {
+          gather4(decay_of<TT>(na.v[r], t0 + 4 * r + grp < p.T && io.in, p.alpha_per_row), aa[r]);
+          dc[r] = bits_f32(nd.v[r]);
+        } else {
+          aa[r][0] = aa[r][1] = aa[r][2] = aa[r][3] = 1.0f;
+        }
+      }
+      load();
 #pragma unroll
       for (int r = 0; r < 4; ++r) e = mfma4(Gx[r], Wn[r], e);
+      if (DECAY) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) e = mfma4(Hx[r], Dn[r], e);
+      }
+      dtot = 1.0f;
+      f32x4 raw;
 #pragma unroll
       for (int r = 3; r >= 0; --r) {
         auto g = [&](int m, int n) { return gs[r][pair(m, n) >> 2][pair(m, n) & 3]; };
+        const BlockDecay D(aa[r], grp);
         float y[4], w[4];
-        gather4(e[r], y);
+        gather4(DECAY ? fmaf(D.end, e[r], x[r]) : e[r], y);
         w[3] = bb[r][3] * y[3];
-        y[2] = fmaf(-g(2, 3), w[3], y[2]);
+        y[2] = fmaf(-(DECAY ? g(2, 3) * D.r32 : g(2, 3)), w[3], y[2]);
         w[2] = bb[r][2] * y[2];
-        y[1] = fmaf(-g(1, 2), w[2], fmaf(-g(1, 3), w[3], y[1]));
+        y[1] = fmaf(-(DECAY ? g(1, 2) * D.r21 : g(1, 2)), w[2], fmaf(-(DECAY ? g(1, 3) * D.r31 : g(1, 3)), w[3], y[1]));
         w[1] = bb[r][1] * y[1];
-        y[0] = fmaf(-g(0, 1), w[1], fmaf(-g(0, 2), w[2], fmaf(-g(0, 3), w[3], y[0])));
+        y[0] = fmaf(-(DECAY ? g(0, 1) * D.r10 : g(0, 1)), w[1],
+                    fmaf(-(DECAY ? g(0, 2) * D.r20 : g(0, 2)), w[2],
+                         fmaf(-(DECAY ? g(0, 3) * D.r30 : g(0, 3)), w[3], y[0])));
         w[0] = bb[r][0] * y[0];
-        const float wn = -pick4(w[0], w[1], w[2], w[3], grp);
-        if (r > 0) e = mfma4(G[r], wn, e);
+        const float wo = -pick4(w[0], w[1], w[2], w[3], grp), wn = DECAY ? wo * D.pre : wo;
+        raw[r] = wo;
+        if (r > 0) e = mfma4(G[r], wn, DECAY ? e * D.all : e);
+        if (DECAY) {
+          const float dn = dc[r] * D.pre;
+          if (r > 0) e = mfma4(H[r], dn, e);
+#pragma unroll
+          for (int n = r + 1; n < 4; ++n) Wn[n] *= D.all, Dn[n] *= D.all;
+          Dn[r] = dn;
+          dtot *= D.all;
+        }
         Wn[r] = wn;
         bstore<float>(rU, uoff + 4 * r * ustep, pick4(y[0], y[1], y[2], y[3], grp));
       }
       uoff -= CH * ustep;
-      sh.w[b][l] = -Wn;
+      sh.w[b][l] = -raw;
       lds_barrier();
     }
   } else if (wave <= SW) {  // state gradient, W columns
@@ -105,9 +151,10 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_rev_kern
     f32x4 S[W / 16];
 #pragma unroll
     for (int jt = 0; jt < W / 16; ++jt) S[jt] = f32x4{0, 0, 0, 0};
-    GateRegs<TT> nd;
+    GateRegs<TT> nd, na;
     nd.at(io.row0, io.step, tl, grp);
     nd.load(io.rV, io.step, -CH);
+    if (DECAY) na.at(io.abase, io.astep, tl, grp), na.load(io.rA, io.astep, -CH);
     lds_barrier();
     for (int j = 0; j < nch; ++j) {
       const int c = nch - 1 - j;
@@ -117,10 +164,29 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_rev_kern
         ColFrag<TT, W> kc, qc;
         kc.template load<LD>(sh.k[(j - 1) & 3] + W * half, li, grp);
         qc.template load<LD>(sh.q[(j - 1) & 3] + W * half, li, grp);
-        state_add2<W>(S, qc, nd.v, kc, sh.w[(j - 1) & 1][l]);
+        if (DECAY) {
+          f32x4 x, wn = -sh.w[(j - 1) & 1][l];  // decayed to the start of chunk c + 1
+          float dt = 1.0f;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float aa[4];
+            gather4(decay_of<TT>(na.v[r], (c + 1) * CH + 4 * r + grp < p.T && io.in, p.alpha_per_row), aa);
+            const BlockDecay D(aa, grp);
+            x[r] = bits_f32(nd.v[r]) * (D.pre * dt);
+            wn[r] *= D.pre * dt;
+            dt *= D.all;
+          }
+          na.load(io.rA, io.astep, -CH);
+#pragma unroll
+          for (int jt = 0; jt < W / 16; ++jt) S[jt] *= dt;
+          state_add<W>(S, qc, x);
+          state_add<W>(S, kc, wn);
+        } else {
+          state_add2<W>(S, qc, nd.v, kc, sh.w[(j - 1) & 1][l]);
+        }
         nd.load(io.rV, io.step, -CH);
-        if ((c + 1) % (CPS / CH) == 0 && io.i < p.cw) {
-          const long slot = io.bh * ((p.T + CPS - 1) / CPS - 1) + c / (CPS / CH);
+        if ((DECAY || (c + 1) % (CPS / CH) == 0) && io.i < p.cw) {
+          const long slot = DECAY ? io.bh * nch + c : io.bh * ((p.T + CPS - 1) / CPS - 1) + c / (CPS / CH);
           float* cp = p.ckpt + (slot * p.cw + io.i) * p.cw + W * half + 4 * grp;
 #pragma unroll
           for (int jt = 0; jt < W / 16; ++jt)
@@ -132,7 +198,8 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_rev_kern
     }
   } else {  // gram, do terms, staging
     TileRegs<TT, DP, VEC> nk, nq;
-    GateRegs<TT> nd;
+    GateRegs<TT> nd, na;
+    if (DECAY) na.at(io.abase, io.astep, tl, grp);
     nk.at(io.base, io.step, tl, p.d, l);
     nq.at(io.base, io.step, tl, p.d, l);
     nd.at(io.row0, io.step, tl, grp);
@@ -152,6 +219,32 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_rev_kern
       const float gv = gr == 0 ? G[0] : gr == 1 ? G[1] : gr == 2 ? G[2] : G[3];
       if (gm < gn) sh.gs[j & 1][8 * gr + pair(gm, gn)] = gv;
       f32x4 x = {0, 0, 0, 0};
+      if constexpr (DECAY) {
+        sh.h[j & 1][l] = H;
+        sh.hx[j & 1][l] = Hx;
+        const int t0 = (nch - 1 - j) * CH;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float aa[4], dd[4];
+          gather4(decay_of<TT>(na.v[r], t0 + 4 * r + grp < p.T && io.in, p.alpha_per_row), aa);
+          gather4(dc[r], dd);
+          const BlockDecay D(aa, grp);
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            // decay from after the lane's step to step s; q_s . k of the lane's step
+            const float rs = s == 3   ? pick4(D.r30, D.r31, D.r32, 1.0f, grp)
+                             : s == 2 ? pick4(D.r20, D.r21, 1.0f, 1.0f, grp)
+                             : s == 1 ? (grp == 0 ? D.r10 : 1.0f)
+                                      : 1.0f;
+            const float hs = __shfl(H[r], 16 * s + 4 * grp + r);
+            x[r] = s >= grp ? fmaf(dd[s] * rs, hs, x[r]) : x[r];
+          }
+        }
+        na.load(io.rA, io.astep, -CH);
+        sh.x[j & 1][l] = x;
+        kp = kf, qp = qf;
+        return;
+      }
 #pragma unroll
       for (int r = 0; r < 4; ++r) x = mfma4(Hx[r], dp[r], x);
       const bool finite = fabsf(dc[0]) < INFINITY && fabsf(dc[1]) < INFINITY && fabsf(dc[2]) < INFINITY &&
@@ -183,6 +276,7 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_rev_kern
     nk.load(io.rK, io.step, -CH);
     nq.load(io.rQ, io.step, -CH);
     nd.load(io.rV, io.step, -CH);
+    if (DECAY) na.load(io.rA, io.astep, -CH);
     stage(0);
     stage(1);
     grams(0);
@@ -381,32 +475,326 @@ __global__ __launch_bounds__(4 * DP) void dr_row_grad_kernel(const GradArgs p) {
   }
 }
 
+// ---- with a decay: the gradients of 16 steps ------------------------------------------------------
+struct DecayArgs {
+  const void *q, *k, *dout, *beta, *alpha;
+  const float *err, *du, *ckpt, *dckpt;  // states after each chunk, and their gradients (all but the last chunk's)
+  void *dq, *dk, *dv, *dbeta, *dalpha;
+  int H, T, d, beta_per_head, alpha_per_row;
+};
+
+// Sums over the wave's lanes: lane n receives the sum of buf[n].
+EDF_DEVICE float scatter64(float (&buf)[64], int lane) {
+  static_for<6>([&](auto step) {
+    constexpr int n = 32 >> decltype(step)::value;
+    const bool up = (lane & n) != 0;
+#pragma unroll
+    for (int k = 0; k < n; ++k) {
+      const float send = up ? buf[k] : buf[k + n], keep = up ? buf[k + n] : buf[k];
+      buf[k] = keep + __shfl_xor(send, n);
+    }
+  });
+  return buf[0];
+}
+
+// One workgroup per chunk of 16 steps of a head.  With A_t the decay from the chunk's start through step t,
+// B_t that after it to the end, R(t, s) from after s through t, S0 the state before the chunk, dS1 its
+// gradient after it (all per row i, sums over i):
+//   dq_t = (do_t A_t) S0 + sum_{s <= t} M(t, s) k_s,          M(t, s) = sum do_t R(t, s) u_s
+//   dk_t = (u_t B_t) dS1 - (w_t A_t) S0 + sum_{s >= t} M(s, t) q_s - sum_{s != t} N(t, s) k_s,
+//                                                              N(t, s) = sum u_t R(s, t) w_s, t < s, mirrored
+//   dalpha_t = sum <D_t, S_{t-1}>,  D_t = dS_t - w_t k_t^T: with z = <D_t, S0> and e_s = D_t k_s carried back over
+//   the steps, <D_t, S_{t-1}> is Horner's rule z, then v <- a_s v + u_s e_s for s < t (no division by a decay)
+// Phases: products of k, q with S0 and dS1 (f32 MFMA); one row per lane: M, N, z, e, dalpha and the decayed
+// factors; products of those with S0, dS1, k and q.  Bound by the row phase's float32 FMAs, 16 x 16 pairs a row
+// for each of M, N and Horner's rule, on the vector units.
 template <typename TT, int DP>
-void launch_bwd(hipStream_t s, const RowArgs& r, float* du, const GradArgs& a, int bh) {
-  const unsigned grid = (unsigned)((long)bh * r.nrb), threads = 64 * (2 + RevShared<TT, DP>::SW);
+__global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayArgs p) {
+  constexpr int LD = DP + 4, NT = DP / 16, LM = CH + 4, NP = 136 + 120;
+  __shared__ __attribute__((aligned(16))) float sK[CH * LD], sQ[CH * LD], sP[CH * LD], sO[CH * LD], sE[CH * LD];
+  __shared__ __attribute__((aligned(16))) float sD[CH * LD], sU[CH * LD], sW[CH * LD];
+  __shared__ __attribute__((aligned(16))) float sG[CH * CH], sH[CH * CH], sM[CH * LM], sN[CH * LM];
+  __shared__ float sZ[DP], red[DP == 128 ? 2 : 1][NP + 64];
+  __shared__ int sBad;
+  const int nch = (p.T + CH - 1) / CH;
+  const long bh = blockIdx.x / nch;
+  const int c = blockIdx.x % nch, t0 = c * CH, d = p.d;
+  const int b = (int)(bh / p.H), h = (int)(bh % p.H);
+  const long rowel = (long)p.T * p.H * d, headel = (long)p.T * p.H;
+  const unsigned rowb = (unsigned)(rowel * sizeof(TT)), rowf = (unsigned)(rowel * 4);
+  const unsigned headb = (unsigned)(headel * sizeof(TT));
+  auto row_rsrc = [&](const void* t) { return make_rsrc((const TT*)t + b * rowel, rowb); };
+  auto head_rsrc = [&](const void* t) { return make_rsrc((const TT*)t + b * headel, headb); };
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, li = l & 15, grp = l >> 4;
+  const unsigned hd = (unsigned)(p.H * d);
+  const float* S0 = p.ckpt + (bh * nch + c - 1) * DP * DP;
+  const float* S1 = p.dckpt + (bh * nch + c) * DP * DP;
+  const bool has0 = c > 0, has1 = c < nch - 1;
+  auto el_off = [&](int t, int i) {  // byte offset of (step t of the chunk, column i), out of bounds past d
+    return i < d ? ((unsigned)(t0 + t) * hd + h * d + i) * (unsigned)sizeof(TT) : OOB_OFF;
+  };
+  auto head_off = [&](int t) { return ((unsigned)(t0 + t) * p.H + h) * (unsigned)sizeof(TT); };
+
+  if (tid == 0) sBad = 0;
+  for (int i = tid; i < CH * LM; i += 256) sM[i] = sN[i] = 0.0f;
+  // one row per lane: this chunk's gates and factors (loaded first, used in the second phase)
+  const int i = tid, ic = min(tid, DP - 1);  // (head_dim 32: half the lanes of the wave idle)
+  const bool rows = w < (DP + 63) / 64, mine = tid < DP;
+  float u[CH], wv[CH], go[CH], a[CH], db[CH];
+  if (rows) {
+    const rsrc_t rG = row_rsrc(p.dout), rB = p.beta_per_head ? head_rsrc(p.beta) : row_rsrc(p.beta);
+    const rsrc_t rA = p.alpha_per_row ? row_rsrc(p.alpha) : head_rsrc(p.alpha);
+    const rsrc_t rE = make_rsrc(p.err + b * rowel, rowf), rU = make_rsrc(p.du + b * rowel, rowf);
+    const rsrc_t rDV = row_rsrc(p.dv);
+#pragma unroll
+    for (int t = 0; t < CH; ++t) {
+      const unsigned fo = i < d ? ((unsigned)(t0 + t) * hd + h * d + i) * 4u : OOB_OFF;
+      const float er = bits_f32(bload<float>(rE, fo)), du = bits_f32(bload<float>(rU, fo));
+      const float be = bits_f32(bload<TT>(rB, p.beta_per_head ? head_off(t) : el_off(t, i)));
+      go[t] = bits_f32(bload<TT>(rG, el_off(t, i)));
+      a[t] = decay_of<TT>(bload<TT>(rA, p.alpha_per_row ? el_off(t, i) : head_off(t)), t0 + t < p.T && i < d,
+                          p.alpha_per_row);
+      u[t] = be * er;
+      wv[t] = be * du;
+      db[t] = er * du;
+      bstore<TT>(rDV, el_off(t, i), wv[t]);
+    }
+  }
+  const rsrc_t rQ = row_rsrc(p.q), rK = row_rsrc(p.k);
+  __syncthreads();
+#pragma unroll
+  for (int n = 0; n < CH * DP / 256; ++n) {
+    const int e = tid + 256 * n, t = e / DP, col = e % DP;
+    const float kv = bits_f32(bload<TT>(rK, el_off(t, col))), qv = bits_f32(bload<TT>(rQ, el_off(t, col)));
+    sK[t * LD + col] = kv;
+    sQ[t * LD + col] = qv;
+    if (!(fabsf(kv) < INFINITY) || !(fabsf(qv) < INFINITY)) sBad = 1;
+  }
+  __syncthreads();
+
+  // S0 k, S0 q, dS1 k and <dS1, S0> per row; the Gram tiles
+  const f32x4 zero = {0, 0, 0, 0};
+  for (int it = w; it < NT; it += 4) {
+    f32x4 pk = zero, pq = zero, ek = zero;
+    float z = 0.0f;
+#pragma unroll
+    for (int jt = 0; jt < NT; ++jt) {
+      const int at = (16 * it + li) * DP + 16 * jt + 4 * grp, ka = li * LD + 16 * jt + 4 * grp;
+      const f32x4 s0 = has0 ? *(const f32x4*)(S0 + at) : zero, s1 = has1 ? *(const f32x4*)(S1 + at) : zero;
+      const f32x4 kv = *(const f32x4*)(sK + ka), qv = *(const f32x4*)(sQ + ka);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        pk = mfma4(kv[e], s0[e], pk);
+        pq = mfma4(qv[e], s0[e], pq);
+        ek = mfma4(kv[e], s1[e], ek);
+        z = fmaf(s0[e], s1[e], z);
+      }
+    }
+    z += __shfl_xor(z, 16);
+    z += __shfl_xor(z, 32);
+    if (grp == 0) sZ[16 * it + li] = z;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int at = (4 * grp + r) * LD + 16 * it + li;
+      sP[at] = pk[r];
+      sO[at] = pq[r];
+      sE[at] = ek[r];
+    }
+  }
+  if (w >= 2) {  // G(t, s) = k_t . k_s, H(t, s) = q_t . k_s
+    f32x4 acc = zero;
+    const float* A = w == 2 ? sK : sQ;
+#pragma unroll
+    for (int jt = 0; jt < NT; ++jt) {
+      const int at = li * LD + 16 * jt + 4 * grp;
+      const f32x4 av = *(const f32x4*)(A + at), bv = *(const f32x4*)(sK + at);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = mfma4(av[e], bv[e], acc);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) (w == 2 ? sG : sH)[(4 * grp + r) * CH + li] = acc[r];
+  }
+  __syncthreads();
+
+  if (rows) {
+    float dec = 1.0f;
+#pragma unroll
+    for (int t = 0; t < CH; ++t) {
+      dec *= a[t];
+      if (mine) sD[t * LD + i] = go[t] * dec;
+      if (mine) sW[t * LD + i] = -wv[t] * dec;
+    }
+    dec = 1.0f;
+#pragma unroll
+    for (int t = CH - 1; t >= 0; --t) {
+      if (mine) sU[t * LD + i] = u[t] * dec;
+      dec *= a[t];
+    }
+    // the decay's gradient
+    const rsrc_t rDA = p.alpha_per_row ? row_rsrc(p.dalpha) : head_rsrc(p.dalpha);
+    float da[CH];
+    {
+      float e[CH], z = sZ[ic];
+#pragma unroll
+      for (int s = 0; s < CH; ++s) e[s] = sE[s * LD + ic];
+#pragma unroll
+      for (int t = CH - 1; t >= 0; --t) {
+        z = fmaf(go[t], sO[t * LD + ic], fmaf(-wv[t], sP[t * LD + ic], z));
+        float v = z;
+#pragma unroll
+        for (int s = 0; s < t; ++s) {
+          e[s] = fmaf(go[t], sH[t * CH + s], fmaf(-wv[t], sG[t * CH + s], e[s]));
+          v = fmaf(a[s], v, u[s] * e[s]);
+          e[s] *= a[t];
+        }
+        z *= a[t];
+        da[t] = v;
+        if (p.alpha_per_row) bstore<TT>(rDA, el_off(t, i), v * a[t]);  // log space
+      }
+    }
+    if (!p.beta_per_head) {
+      const rsrc_t rDB = row_rsrc(p.dbeta);
+#pragma unroll
+      for (int t = 0; t < CH; ++t) bstore<TT>(rDB, el_off(t, i), db[t]);
+    }
+    // sums over the rows: M(t, s) at t (t + 1) / 2 + t - s, N(t, s) at 136 + s (s - 1) / 2 + s - 1 - t, then the
+    // per-head dbeta and dalpha; 64 at a time
+    float buf[64];
+#pragma unroll
+    for (int n = 0; n < 64; ++n) {
+      const bool ok = i < d;
+      buf[n] = n < CH ? (ok ? db[n < CH ? n : 0] : 0.0f) : n < 2 * CH ? (ok ? da[n < 2 * CH ? n - CH : 0] : 0.0f) : 0.0f;
+    }
+    red[w][NP + l] = scatter64(buf, l);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+      for (int t = 0; t < CH; ++t) {
+        float x = go[t];
+#pragma unroll
+        for (int s = t; s >= 0; --s) {
+          const int n = t * (t + 1) / 2 + t - s;
+          if (n / 64 == q) buf[n % 64] = x * u[s];
+          x *= a[s];
+        }
+      }
+#pragma unroll
+      for (int s = 1; s < CH; ++s) {
+        float y = -wv[s] * a[s];
+#pragma unroll
+        for (int t = s - 1; t >= 0; --t) {
+          const int n = 136 + s * (s - 1) / 2 + s - 1 - t;
+          if (n / 64 == q) buf[n % 64] = y * u[t];
+          y *= a[t];
+        }
+      }
+      red[w][64 * q + l] = scatter64(buf, l);
+    }
+  }
+  __syncthreads();
+  {
+    float v = red[0][tid];
+    if (DP == 128) v += red[DP == 128 ? 1 : 0][tid];
+    int n = tid < 136 ? tid : tid - 136, t = 0;
+    if (tid < 136) {
+      while ((t + 1) * (t + 2) / 2 <= n) ++t;
+      sM[t * LM + t - (n - t * (t + 1) / 2)] = v;
+    } else {
+      t = 1;
+      while (t * (t + 1) / 2 <= n) ++t;
+      const int s = t - 1 - (n - t * (t - 1) / 2);
+      sN[t * LM + s] = v;
+      sN[s * LM + t] = v;
+    }
+    if (tid < 2 * CH) {
+      float sum = red[0][NP + tid];
+      if (DP == 128) sum += red[DP == 128 ? 1 : 0][NP + tid];
+      if (tid < CH) {
+        if (p.beta_per_head) bstore<TT>(head_rsrc(p.dbeta), head_off(tid), sum);
+      } else if (!p.alpha_per_row) {
+        bstore<TT>(head_rsrc(p.dalpha), head_off(tid - CH), sum);
+      }
+    }
+  }
+  __syncthreads();
+
+  const rsrc_t rDQ = row_rsrc(p.dq), rDK = row_rsrc(p.dk);
+  const bool bad = sBad != 0;
+  for (int jt = w; jt < NT; jt += 4) {
+    f32x4 dq = zero, dk = zero;
+    const int j = 16 * jt + li;
+#pragma unroll
+    for (int x = 0; x < NT; ++x) {
+      const int at = li * LD + 16 * x + 4 * grp;
+      const f32x4 dv = *(const f32x4*)(sD + at), wn = *(const f32x4*)(sW + at), uv = *(const f32x4*)(sU + at);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int si = (16 * x + 4 * grp + e) * DP + j;
+        const float s0 = has0 ? S0[si] : 0.0f, s1 = has1 ? S1[si] : 0.0f;
+        dq = mfma4(dv[e], s0, dq);
+        dk = mfma4(wn[e], s0, dk);
+        dk = mfma4(uv[e], s1, dk);
+      }
+    }
+    if (!bad) {
+      const f32x4 mv = *(const f32x4*)(sM + li * LM + 4 * grp), nv = *(const f32x4*)(sN + li * LM + 4 * grp);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int s = 4 * grp + e;
+        dq = mfma4(mv[e], sK[s * LD + j], dq);
+        dk = mfma4(nv[e], sK[s * LD + j], dk);
+        dk = mfma4(sM[s * LM + li], sQ[s * LD + j], dk);
+      }
+    } else {  // a step outside a sum must not enter it even with 0
+      for (int s = 0; s < CH; ++s)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int t = 4 * grp + r;
+          if (s <= t) dq[r] = fmaf(sM[t * LM + s], sK[s * LD + j], dq[r]);
+          if (s >= t) dk[r] = fmaf(sM[s * LM + t], sQ[s * LD + j], dk[r]);
+          if (s != t) dk[r] = fmaf(sN[t * LM + s], sK[s * LD + j], dk[r]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      bstore<TT>(rDQ, el_off(4 * grp + r, j), dq[r]);
+      bstore<TT>(rDK, el_off(4 * grp + r, j), dk[r]);
+    }
+  }
+}
+
+template <typename TT, int DP>
+void launch_bwd(hipStream_t s, const RowArgs& r, float* du, const GradArgs& a, const DecayArgs& da, int bh) {
+  const unsigned grid = (unsigned)((long)bh * r.nrb), threads = 64 * (2 + (DP >= 64 ? 2 : 1));
   const uintptr_t at = (uintptr_t)r.q | (uintptr_t)r.k;
-  if (r.d % (16 / (int)sizeof(TT)) == 0 && at % 4 == 0)
-    dr_row_rev_kernel<TT, DP, true><<<grid, threads, 0, s>>>(r, du);
-  else
-    dr_row_rev_kernel<TT, DP, false><<<grid, threads, 0, s>>>(r, du);
+  const bool vec = r.d % (16 / (int)sizeof(TT)) == 0 && at % 4 == 0;
+  if (r.alpha != nullptr) {
+    vec ? dr_row_rev_kernel<TT, DP, true, true><<<grid, threads, 0, s>>>(r, du)
+        : dr_row_rev_kernel<TT, DP, true, false><<<grid, threads, 0, s>>>(r, du);
+    dr_row_decay_grad_kernel<TT, DP><<<(unsigned)((long)bh * ((r.T + CH - 1) / CH)), 256, 0, s>>>(da);
+    return;
+  }
+  vec ? dr_row_rev_kernel<TT, DP, false, true><<<grid, threads, 0, s>>>(r, du)
+      : dr_row_rev_kernel<TT, DP, false, false><<<grid, threads, 0, s>>>(r, du);
   dr_row_grad_kernel<TT, DP><<<(unsigned)((long)bh * ((r.T + CPS - 1) / CPS)), 4 * DP, 0, s>>>(a);
 }
 
 template <typename TT>
-void by_width(hipStream_t s, const RowArgs& r, float* du, const GradArgs& a, int bh) {
+void by_width(hipStream_t s, const RowArgs& r, float* du, const GradArgs& a, const DecayArgs& da, int bh) {
   if (r.cw == 32)
-    launch_bwd<TT, 32>(s, r, du, a, bh);
+    launch_bwd<TT, 32>(s, r, du, a, da, bh);
   else if (r.cw == 64)
-    launch_bwd<TT, 64>(s, r, du, a, bh);
+    launch_bwd<TT, 64>(s, r, du, a, da, bh);
   else
-    launch_bwd<TT, 128>(s, r, du, a, bh);
+    launch_bwd<TT, 128>(s, r, du, a, da, bh);
 }
 
 inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 inline int state_width(int d) { return d <= 32 ? 32 : d <= 64 ? 64 : 128; }
-inline size_t states_bytes(int batch, int heads, int seq, int d) {
-  const size_t w = state_width(d);
-  return align256((size_t)batch * heads * ((seq + CPS - 1) / CPS - 1) * w * w * 4);
+// States kept: with a decay after every chunk, without before every CPS steps but the first.
+inline size_t states_bytes(int batch, int heads, int seq, int d, bool decay) {
+  const size_t w = state_width(d), n = decay ? (seq + CH - 1) / CH : (seq + CPS - 1) / CPS - 1;
+  return align256((size_t)batch * heads * n * w * w * 4);
 }
 inline size_t rows_bytes(int batch, int heads, int seq, int d) {
   return align256((size_t)batch * seq * heads * d * 4);
@@ -415,45 +803,55 @@ inline size_t rows_bytes(int batch, int heads, int seq, int d) {
 }  // namespace
 
 // The forward's record for this backward: states, then err.
-size_t dr_row_context_bytes(int batch, int heads, int seq, int d) {
-  return states_bytes(batch, heads, seq, d) + rows_bytes(batch, heads, seq, d);
+size_t dr_row_context_bytes(int batch, int heads, int seq, int d, bool decay) {
+  return states_bytes(batch, heads, seq, d, decay) + rows_bytes(batch, heads, seq, d);
 }
 
-int dr_row_record_run(void* stream, const void* q, const void* k, const void* v, const void* beta, void* out,
-                      int batch, int seq, int heads, int d, int dtype, int beta_per_head, void* context) {
-  return dr_row_run(stream, q, k, v, beta, nullptr, out, batch, seq, heads, d, dtype, beta_per_head, 0,
-                    (float*)context, (float*)((char*)context + states_bytes(batch, heads, seq, d)), state_width(d));
+int dr_row_record_run(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
+                      void* out, int batch, int seq, int heads, int d, int dtype, int beta_per_head,
+                      int alpha_per_row, void* context) {
+  return dr_row_run(stream, q, k, v, beta, alpha, out, batch, seq, heads, d, dtype, beta_per_head, alpha_per_row,
+                    (float*)context, (float*)((char*)context + states_bytes(batch, heads, seq, d, alpha != nullptr)),
+                    state_width(d));
 }
 
 // Workspace: state gradients, du, and a record of its own for a caller without the forward's.
-size_t dr_row_backward_workspace_bytes(int batch, int heads, int seq, int d) {
-  return 2 * dr_row_context_bytes(batch, heads, seq, d);
+size_t dr_row_backward_workspace_bytes(int batch, int heads, int seq, int d, bool decay) {
+  return 2 * dr_row_context_bytes(batch, heads, seq, d, decay);
 }
 
 int dr_row_backward_run(void* stream, const void* q, const void* k, const void* v, const void* beta,
-                        const void* grad_out, void* dq, void* dk, void* dv, void* dbeta, void* workspace, int batch,
-                        int seq, int heads, int d, int dtype, int beta_per_head, const void* context) {
-  const size_t sb = states_bytes(batch, heads, seq, d), ctx = dr_row_context_bytes(batch, heads, seq, d);
+                        const void* alpha, const void* grad_out, void* dq, void* dk, void* dv, void* dbeta,
+                        void* dalpha, void* workspace, int batch, int seq, int heads, int d, int dtype,
+                        int beta_per_head, int alpha_per_row, const void* context) {
+  const bool decay = alpha != nullptr;
+  const size_t sb = states_bytes(batch, heads, seq, d, decay), ctx = dr_row_context_bytes(batch, heads, seq, d, decay);
   char* ws = (char*)workspace;
   if (context == nullptr) {
     context = ws + ctx;
-    const int rc = dr_row_record_run(stream, q, k, v, beta, nullptr, batch, seq, heads, d, dtype, beta_per_head,
-                                     ws + ctx);
+    const int rc = dr_row_record_run(stream, q, k, v, beta, alpha, nullptr, batch, seq, heads, d, dtype,
+                                     beta_per_head, alpha_per_row, ws + ctx);
     if (rc) return rc;
   }
   RowArgs r{};
-  r.q = q, r.k = k, r.v = grad_out, r.beta = beta, r.ckpt = (float*)ws;
-  r.H = heads, r.T = seq, r.d = d, r.cw = state_width(d), r.nrb = r.cw / RW, r.beta_per_head = beta_per_head;
+  r.q = q, r.k = k, r.v = grad_out, r.beta = beta, r.alpha = alpha, r.ckpt = (float*)ws;
+  r.H = heads, r.T = seq, r.d = d, r.cw = state_width(d), r.nrb = r.cw / RW;
+  r.beta_per_head = beta_per_head, r.alpha_per_row = alpha_per_row;
   float* du = (float*)(ws + sb);
   GradArgs a{};
   a.q = q, a.k = k, a.dout = grad_out, a.beta = beta, a.dq = dq, a.dk = dk, a.dv = dv, a.dbeta = dbeta;
   a.ckpt = (const float*)context, a.err = (const float*)((const char*)context + sb), a.dckpt = r.ckpt, a.du = du;
   a.H = heads, a.T = seq, a.d = d, a.beta_per_head = beta_per_head;
+  DecayArgs da{};
+  da.q = q, da.k = k, da.dout = grad_out, da.beta = beta, da.alpha = alpha;
+  da.dq = dq, da.dk = dk, da.dv = dv, da.dbeta = dbeta, da.dalpha = dalpha;
+  da.ckpt = a.ckpt, da.err = a.err, da.dckpt = a.dckpt, da.du = du;
+  da.H = heads, da.T = seq, da.d = d, da.beta_per_head = beta_per_head, da.alpha_per_row = alpha_per_row;
   hipStream_t s = as_stream(stream);
   if (dtype == EDF_BF16)
-    by_width<bf16>(s, r, du, a, batch * heads);
+    by_width<bf16>(s, r, du, a, da, batch * heads);
   else
-    by_width<float>(s, r, du, a, batch * heads);
+    by_width<float>(s, r, du, a, da, batch * heads);
   return check_launch("delta rule backward (row scan)");
 }
 

@@ -12,10 +12,8 @@
 //   dv = beta ds_k, dbeta = err ds_k, dk = dS_tot^T (beta err) - S_g^T (beta ds_k),
 //   dalpha = sum(dS_to_decayed * S_prev), dS_prev = alpha dS_to_decayed).
 //
-// This is the exact per-step path: per-element beta (where each row of S has its own gate, so the
-// chunked UT form of the per-head path does not apply), float32 I/O and any head_dim <= 128.  The forward
-// and the states a backward starts from run 16 steps at a time on the matrix cores
-// (delta_rule_row.hip); the per-step forward here serves batch rows of 2 GiB and more.
+// The exact per-step path: it serves batch rows of 2 GiB and more; smaller ones run 16 steps at a time on
+// the matrix cores (delta_rule_row.hip, delta_rule_row_bwd.hip).
 //
 // Rows of S evolve independently given k, q, alpha and the row's beta, so a workgroup
 // owns one block of RB = 16 rows of one (batch, head) state (DP / 16 workgroups per
@@ -468,10 +466,9 @@ size_t dr_seq_context_bytes(int batch, int heads, int seq, int d) {
 int dr_seq_run(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
                void* out, int batch, int seq, int heads, int d, int dtype, int beta_per_head, int alpha_per_row,
                float* context) {
-  // (a call without decay that keeps states, and that the row scans take, does not come here)
-  if (dr_row_takes(batch, heads, seq, d))
+  if (dr_row_takes(batch, heads, seq, d))  // (a call that keeps states, and that these take, does not come here)
     return dr_row_run(stream, q, k, v, beta, alpha, out, batch, seq, heads, d, dtype, beta_per_head, alpha_per_row,
-                      context, nullptr, pad_dim(d));
+                      nullptr, nullptr, 0);
   DRArgs a{};
   a.q = q; a.k = k; a.v = v; a.beta = beta; a.alpha = alpha; a.out = out;
   a.ckpt = context;  // also store the checkpoints (one pass writes both)

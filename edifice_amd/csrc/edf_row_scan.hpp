@@ -320,9 +320,9 @@ EDF_DEVICE void lds_barrier() {
 struct RowArgs {
   const void *q, *k, *v, *beta, *alpha;
   void* out;
-  // what a backward reads, or null.  With a decay, for the per-step backward: the state after each
-  // chunk, [BH][chunks][cw][cw].  Without, for delta_rule_row_bwd.hip: the state before every
-  // CPS steps but the first, [BH][ceil(T / CPS) - 1][cw][cw], and err, [B, T, H, d].
+  // what a backward (delta_rule_row_bwd.hip) reads, or null: err, [B, T, H, d], and states.  With a
+  // decay the state after each chunk, [BH][chunks][cw][cw]; without, the state before every CPS steps
+  // but the first, [BH][ceil(T / CPS) - 1][cw][cw].
   float *ckpt, *err;
   int H, T, d, nrb, cw;
   int beta_per_head, alpha_per_row;
@@ -358,6 +358,26 @@ template <typename TT> struct RowIO {
     const unsigned hstep = (unsigned)(p.H * sizeof(TT)), head0 = in ? h * (unsigned)sizeof(TT) : OOB_OFF;
     bbase = p.beta_per_head ? head0 : row0, bstep = p.beta_per_head ? hstep : step;
     abase = p.alpha_per_row ? row0 : head0, astep = p.alpha_per_row ? step : hstep;
+  }
+};
+
+// The decay of the lane's steps; a step past T and a row past d are identities (a = 1; beta = v = 0).
+template <typename TT>
+EDF_DEVICE float decay_of(typename Bits<TT>::type raw, bool live, int alpha_per_row) {
+  const float v = bits_f32(raw);
+  return live ? (alpha_per_row ? __expf(v) : v) : 1.0f;
+}
+
+// Decays within a block of four steps: rMN from after step n to step m, a0 of the first step, all of
+// the block, pre from the block's start to the lane's step, end from after the lane's step.
+struct BlockDecay {
+  float a0, r10, r20, r30, r21, r31, r32, all, pre, end;
+  EDF_DEVICE BlockDecay(const float (&a)[4], int grp) {
+    a0 = a[0], r10 = a[1], r21 = a[2], r32 = a[3];
+    r31 = r32 * r21, r20 = r21 * r10, r30 = r32 * r20;
+    all = r30 * a0;
+    pre = pick4(a0, r10 * a0, r20 * a0, all, grp);
+    end = pick4(r30, r31, r32, 1.0f, grp);
   }
 };
 
