@@ -148,11 +148,11 @@ def lib():
 
 
 def call(name: str, *args) -> None:
-    rc = getattr(lib(), name)(*args)
+    rc = getattr(_LIB or lib(), name)(*args)
     if rc != 0:
         msg = lib().edf_last_error().decode(errors="replace")
         raise EdificeHipError(f"{name} failed (code {rc}): {msg}")
 
 
 def query(name: str, *args) -> int:
-    return int(getattr(lib(), name)(*args))
+    return getattr(_LIB or lib(), name)(*args)
