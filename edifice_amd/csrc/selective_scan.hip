@@ -861,9 +861,7 @@ inline long num_chunks(int seq) { return (seq + SS_CK - 1) / SS_CK; }
 inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Channel groups per workgroup.  The kernels are compiled for G = 1 and for a wide G per
-// state size; the host takes the one whose grid loads the busiest CU with the fewest
-// waves (workgroups spread evenly over 256 CUs, at most as many per CU as LDS and the
-// 32 waves per CU allow), the wide one on a tie (fewer dC/dB partials, longer rows).
+// state size (choose_plan below takes one).
 struct SSPlan {
   int G, CT, ntile;
 };
@@ -894,31 +892,39 @@ inline int forced_plan() {
   return 0;
 }
 
+// Workgroups spread evenly over 256 CUs, so the time follows the channels of the busiest CU.
+//
+// - With at most one wide workgroup per CU and fewer than 12 narrow waves (three per SIMD) on the busiest CU,
+//   the time is a chain of T steps that more waves on a CU slow: the narrow plan from two thirds of the
+//   channels down.  16 states, D = 2048, T = 1000, forward / backward us, wide -> narrow: B = 2 bf16
+//   70 / 217 -> 45 / 147, f32 68 / 212 -> 46 / 152; B = 4 bf16 72 / 220 -> 55 / 176, f32 70 / 240 -> 58 / 218;
+//   8 states, B = 4: bf16 65 / 209 -> 58 / 188, f32 62 / 221 -> 60 / 201.  At three quarters float32 is slower
+//   (8 states, B = 5: 63 / 229 wide, 61 / 247 narrow).
+// - Otherwise the forward keeps the wide plan (fewer dB / dC partials, longer rows) unless the narrow one has
+//   fewer channels per CU: 8 states, B = 16 bf16 135 us wide, 177 narrow.
+// - The backward, whose LDS keeps few workgroups resident, counts a CU's channels as slowed where its resident
+//   waves do not fill 12 slots: 4 states, B = 24 710 us wide, 565 narrow.
 inline SSPlan choose_plan(int batch, int dim, int NP, bool bwd) {
   const int SW = NP < 4 ? NP : 4, CW = 64 / SW, NSG = NP / SW;
   const int gw = wide_groups(NP);
-  SSPlan best{gw, gw * CW, (dim + gw * CW - 1) / (gw * CW)};
+  const SSPlan wide{gw, gw * CW, (dim + gw * CW - 1) / (gw * CW)}, narrow{1, CW, (dim + CW - 1) / CW};
   const int force = forced_plan();
-  if (force == 1) return SSPlan{1, CW, (dim + CW - 1) / CW};
-  if (force == 2) return best;
-  double best_score = 1e30;
-  const int cands[2] = {gw, 1};
-  for (int G : cands) {
-    const int CT = G * CW, nt = (dim + CT - 1) / CT, nw = G * NSG;
-    const long nwg = (long)batch * nt;
-    const size_t lds = bwd ? bwd_lds(NP, G) : fwd_lds(NP, G);
+  if (force) return force == 1 ? narrow : wide;
+  struct Load {
+    long per_cu, channels, waves;
+    double slowed;
+  };
+  auto load = [&](const SSPlan& pl) {
+    const int nw = pl.G * NSG;
+    const long per_cu = ((long)batch * pl.ntile + 255) / 256;
+    const size_t lds = bwd ? bwd_lds(NP, pl.G) : fwd_lds(NP, pl.G);
     const long occ = std::max(1L, std::min((long)(163840 / lds), (long)(32 / nw)));
-    const long per_cu = (nwg + 255) / 256;
-    // the channel work the busiest CU holds, slowed where its resident waves cannot fill 12
-    // slots (three per SIMD); a tie goes to the wide plan (fewer dB / dC partials)
-    const double waves = (double)std::min(per_cu, occ) * nw;
-    const double score = (double)per_cu * CT / std::min(1.0, waves / 12.0);
-    if (score < best_score) {
-      best_score = score;
-      best = SSPlan{G, CT, nt};
-    }
-  }
-  return best;
+    const double resident = (double)std::min(per_cu, occ) * nw;
+    return Load{per_cu, per_cu * pl.CT, per_cu * nw, (double)(per_cu * pl.CT) / std::min(1.0, resident / 12.0)};
+  };
+  const Load w = load(wide), n = load(narrow);
+  if (w.per_cu == 1 && n.waves < 12) return 3 * n.channels <= 2 * w.channels ? narrow : wide;
+  return (bwd ? n.slowed < w.slowed : n.channels < w.channels) ? narrow : wide;
 }
 
 // caller-owned "states" buffer: checkpoints [batch][nck][NP][dim] float32, then y before the

@@ -250,3 +250,18 @@ def test_context_and_glue_entry_points_validate_before_launch(lib):
     assert rc == 1 and b"null" in lib.edf_last_error()
     rc = lib.edf_cross_entropy_backward(None, p, p, p, p, 0.25, p, 4, 10, 3)
     assert rc == 1 and b"dtype" in lib.edf_last_error()
+
+
+@pytest.mark.parametrize("batch,dim,n,plan", [(1, 16, 16, "narrow"), (4, 2048, 16, "narrow"), (5, 2048, 16, "wide"),
+                                              (4, 2048, 8, "narrow"), (5, 2048, 8, "wide"), (4, 2048, 4, "narrow"),
+                                              (5, 2048, 4, "wide"), (8, 2048, 16, "narrow")])
+def test_selective_scan_plan_by_grid(monkeypatch, batch, dim, n, plan):
+    """Few workgroups, or fewer channels on the busiest CU, take the narrow plan: the backward workspace holds
+    dB / dC partials per tile and shows which."""
+    from edifice_amd import _native as nat
+    size = {}
+    for p in ("", "narrow", "wide"):
+        monkeypatch.setenv("EDF_SS_PLAN", p)
+        size[p] = nat.query("edf_selective_scan_backward_workspace_bytes", batch, 64, dim, n, 0, 1)
+    assert size[""] == size[plan]
+    assert dim == 16 or size["narrow"] != size["wide"]
