@@ -21,8 +21,8 @@
 // factor out of M and N over more steps than a short product per pair, so those sums over the rows, and
 // the decay's gradient <dS_t - w_t k_t^T, S_{t-1}>, are formed one row per lane (dr_row_decay_grad_kernel).
 // Forward and backward, against one workgroup per 16 rows stepping through the sequence with partial dq and
-// dk per row block (its time is the chain of T steps): KDA 4x1000x8x128 bf16 875 -> 487 us (scan 92,
-// gradients 293), GatedDeltaNet 2x777x8x64 float32 436 -> 235.
+// dk per row block (its time is the chain of T steps): KDA 4x1000x8x128 bf16 875 -> 344 us,
+// GatedDeltaNet 2x777x8x64 float32 436 -> 213.
 #include "edf_abi.hpp"
 #include "edf_common.hpp"
 #include "edf_row_scan.hpp"
@@ -483,18 +483,33 @@ struct DecayArgs {
   int H, T, d, beta_per_head, alpha_per_row;
 };
 
-// Sums over the wave's lanes: lane n receives the sum of buf[n].
-EDF_DEVICE float scatter64(float (&buf)[64], int lane) {
-  static_for<6>([&](auto step) {
-    constexpr int n = 32 >> decltype(step)::value;
+// Sums over the wave's lanes: lane n receives the sum of buf[n].  A reduce-scatter without LDS: halves of the wave
+// and of each half exchange by swaps (of buf[k] and buf[k + n], whose sum then has either index where it belongs),
+// the last 16 lanes by DPP mirrors and quad permutes (pairings of lanes that agree in the bits already settled).
+EDF_DEVICE float scatter16(float* buf, int lane) {  // within each 16 lanes: lane n receives the sum of buf[n & 15]
+  static_for<4>([&](auto step) {
+    constexpr int n = 8 >> decltype(step)::value, ctrl[4] = {0x140, 0x141, 0x4E, 0xB1};  // ^ 15, ^ 7, ^ 2, ^ 1
     const bool up = (lane & n) != 0;
 #pragma unroll
     for (int k = 0; k < n; ++k) {
       const float send = up ? buf[k] : buf[k + n], keep = up ? buf[k + n] : buf[k];
-      buf[k] = keep + __shfl_xor(send, n);
+      buf[k] = keep + dpp_f32<ctrl[decltype(step)::value]>(send);
     }
   });
   return buf[0];
+}
+EDF_DEVICE float scatter64(float (&buf)[64], int lane) {
+#pragma unroll
+  for (int k = 0; k < 32; ++k) {
+    swap32(buf[k], buf[k + 32]);
+    buf[k] += buf[k + 32];
+  }
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    swap16(buf[k], buf[k + 16]);
+    buf[k] += buf[k + 16];
+  }
+  return scatter16(buf, lane);
 }
 
 // One workgroup per chunk of 16 steps of a head.  With A_t the decay from the chunk's start through step t,
@@ -505,17 +520,31 @@ EDF_DEVICE float scatter64(float (&buf)[64], int lane) {
 //                                                              N(t, s) = sum u_t R(s, t) w_s, t < s, mirrored
 //   dalpha_t = sum <D_t, S_{t-1}>,  D_t = dS_t - w_t k_t^T: with z = <D_t, S0> and e_s = D_t k_s carried back over
 //   the steps, <D_t, S_{t-1}> is Horner's rule z, then v <- a_s v + u_s e_s for s < t (no division by a decay)
-// Phases: products of k, q with S0 and dS1 (f32 MFMA); one row per lane: M, N, z, e, dalpha and the decayed
-// factors; products of those with S0, dS1, k and q.  Bound by the row phase's float32 FMAs, 16 x 16 pairs a row
-// for each of M, N and Horner's rule, on the vector units.
+// Phases: products of k, q with S0 and dS1 (f32 MFMA); one row per lane: z, e, dalpha and the decayed factors
+// (waves 0 and 1), M and N (waves 2 and 3); products of those with S0, dS1, k and q, each wave 16 columns of four
+// in a lane (whole 256-byte rows of S per load) and a part of the rows, the parts added in LDS.
+// The states before the first chunk and the gradients after the last are zero: an empty buffer reads so, and the
+// loads stay unconditional, in flight together (each behind a branch was waited for by itself: with the row phase on
+// two of the four waves, 159k cycles a workgroup at KDA 4x1000x8x128 bf16, 74k now).
 template <typename TT, int DP>
 __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayArgs p) {
   constexpr int LD = DP + 4, NT = DP / 16, LM = CH + 4, NP = 136 + 120;
-  __shared__ __attribute__((aligned(16))) float sK[CH * LD], sQ[CH * LD], sP[CH * LD], sO[CH * LD], sE[CH * LD];
-  __shared__ __attribute__((aligned(16))) float sD[CH * LD], sU[CH * LD], sW[CH * LD];
+  constexpr int VC = DP >= 64 ? 4 : 2, NC = DP >= 64 ? DP / 64 : 1;  // last phase: columns of a lane, groups of 16 VC
+  constexpr int KS = 4 / NC < NT ? 4 / NC : NT, KX = NT / KS;        // parts of the rows, 16-row blocks of a part
+  typedef f32x4 Part[NC][VC][64];
+  struct Products {
+    float P[CH * LD], O[CH * LD], E[CH * LD];
+  };
+  union Shared {
+    Products f;
+    Part part[2][KS > 1 ? KS - 1 : 1];  // dq, dk
+  };
+  __shared__ __attribute__((aligned(16))) float sK[CH * LD], sQ[CH * LD], sD[CH * LD], sU[CH * LD], sW[CH * LD];
+  __shared__ __attribute__((aligned(16))) Shared sh;
   __shared__ __attribute__((aligned(16))) float sG[CH * CH], sH[CH * CH], sM[CH * LM], sN[CH * LM];
-  __shared__ float sZ[DP], red[DP == 128 ? 2 : 1][NP + 64];
-  __shared__ int sBad;
+  __shared__ float sZ[DP], red[DP == 128 ? 2 : 1][NP + 2 * CH];
+  __shared__ int sBad[4];
+  float *const sP = sh.f.P, *const sO = sh.f.O, *const sE = sh.f.E;
   const int nch = (p.T + CH - 1) / CH;
   const long bh = blockIdx.x / nch;
   const int c = blockIdx.x % nch, t0 = c * CH, d = p.d;
@@ -527,25 +556,42 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
   auto head_rsrc = [&](const void* t) { return make_rsrc((const TT*)t + b * headel, headb); };
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, li = l & 15, grp = l >> 4;
   const unsigned hd = (unsigned)(p.H * d);
-  const float* S0 = p.ckpt + (bh * nch + c - 1) * DP * DP;
-  const float* S1 = p.dckpt + (bh * nch + c) * DP * DP;
   const bool has0 = c > 0, has1 = c < nch - 1;
+  const rsrc_t rS0 = make_rsrc(p.ckpt + (has0 ? (bh * nch + c - 1) * DP * DP : 0), has0 ? DP * DP * 4u : 0u);
+  const rsrc_t rS1 = make_rsrc(p.dckpt + (has1 ? (bh * nch + c) * DP * DP : 0), has1 ? DP * DP * 4u : 0u);
   auto el_off = [&](int t, int i) {  // byte offset of (step t of the chunk, column i), out of bounds past d
     return i < d ? ((unsigned)(t0 + t) * hd + h * d + i) * (unsigned)sizeof(TT) : OOB_OFF;
   };
   auto head_off = [&](int t) { return ((unsigned)(t0 + t) * p.H + h) * (unsigned)sizeof(TT); };
 
-  if (tid == 0) sBad = 0;
-  for (int i = tid; i < CH * LM; i += 256) sM[i] = sN[i] = 0.0f;
-  // one row per lane: this chunk's gates and factors (loaded first, used in the second phase)
-  const int i = tid, ic = min(tid, DP - 1);  // (head_dim 32: half the lanes of the wave idle)
-  const bool rows = w < (DP + 63) / 64, mine = tid < DP;
-  float u[CH], wv[CH], go[CH], a[CH], db[CH];
+  const rsrc_t rQ = row_rsrc(p.q), rK = row_rsrc(p.k);
+  constexpr int NE = CH * DP / 256;
+  float kv[NE], qv[NE];
+#pragma unroll
+  for (int n = 0; n < NE; ++n) {
+    const int e = tid + 256 * n, t = e / DP, col = e % DP;
+    kv[n] = bits_f32(bload<TT>(rK, el_off(t, col)));
+    qv[n] = bits_f32(bload<TT>(rQ, el_off(t, col)));
+  }
+  // one row per lane, in either pair of waves: this chunk's gates and factors
+  const bool first = w < 2;
+  const int i = tid & 127, ic = min(i, DP - 1);  // (head_dim 32: half the lanes of the wave idle)
+  const bool rows = (w & 1) < (DP + 63) / 64, mine = i < DP;
+  float u[CH], wv[CH], go[CH], a[CH];
+  // sums over all rows, one step a lane, of a value per row that is 0 past d (per-head dbeta and dalpha)
+  auto put_sums = [&](float (&x)[CH], int at) {
+#pragma unroll
+    for (int t = 0; t < CH; ++t) x[t] = i < d ? x[t] : 0.0f;
+    float v = scatter16(x, l);
+    v += __shfl_xor(v, 16);
+    v += __shfl_xor(v, 32);
+    if (l < CH) red[w & 1][at + l] = v;
+  };
   if (rows) {
     const rsrc_t rG = row_rsrc(p.dout), rB = p.beta_per_head ? head_rsrc(p.beta) : row_rsrc(p.beta);
     const rsrc_t rA = p.alpha_per_row ? row_rsrc(p.alpha) : head_rsrc(p.alpha);
     const rsrc_t rE = make_rsrc(p.err + b * rowel, rowf), rU = make_rsrc(p.du + b * rowel, rowf);
-    const rsrc_t rDV = row_rsrc(p.dv);
+    float db[CH];
 #pragma unroll
     for (int t = 0; t < CH; ++t) {
       const unsigned fo = i < d ? ((unsigned)(t0 + t) * hd + h * d + i) * 4u : OOB_OFF;
@@ -557,37 +603,54 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
       u[t] = be * er;
       wv[t] = be * du;
       db[t] = er * du;
-      bstore<TT>(rDV, el_off(t, i), wv[t]);
+    }
+    if (first) {
+      const rsrc_t rDV = row_rsrc(p.dv), rDB = p.beta_per_head ? head_rsrc(p.dbeta) : row_rsrc(p.dbeta);
+#pragma unroll
+      for (int t = 0; t < CH; ++t) {
+        bstore<TT>(rDV, el_off(t, i), wv[t]);
+        if (!p.beta_per_head) bstore<TT>(rDB, el_off(t, i), db[t]);
+      }
+      if (p.beta_per_head) put_sums(db, NP);
     }
   }
-  const rsrc_t rQ = row_rsrc(p.q), rK = row_rsrc(p.k);
-  __syncthreads();
+  for (int n = tid; n < CH * LM; n += 256) sM[n] = sN[n] = 0.0f;
+  bool bad = false;
 #pragma unroll
-  for (int n = 0; n < CH * DP / 256; ++n) {
+  for (int n = 0; n < NE; ++n) {
     const int e = tid + 256 * n, t = e / DP, col = e % DP;
-    const float kv = bits_f32(bload<TT>(rK, el_off(t, col))), qv = bits_f32(bload<TT>(rQ, el_off(t, col)));
-    sK[t * LD + col] = kv;
-    sQ[t * LD + col] = qv;
-    if (!(fabsf(kv) < INFINITY) || !(fabsf(qv) < INFINITY)) sBad = 1;
+    sK[t * LD + col] = kv[n];
+    sQ[t * LD + col] = qv[n];
+    bad = bad || !(fabsf(kv[n]) < INFINITY) || !(fabsf(qv[n]) < INFINITY);
   }
+  bad = __any(bad);
+  if (l == 0) sBad[w] = bad;
   __syncthreads();
 
   // S0 k, S0 q, dS1 k and <dS1, S0> per row; the Gram tiles
   const f32x4 zero = {0, 0, 0, 0};
+#pragma unroll 1
   for (int it = w; it < NT; it += 4) {
+    u32x4 s0[NT], s1[NT];
+#pragma unroll
+    for (int jt = 0; jt < NT; ++jt) {
+      const int at = (li * DP + 16 * jt + 4 * grp) * 4, blk = 16 * it * DP * 4;
+      s0[jt] = __builtin_amdgcn_raw_buffer_load_b128(rS0, at, blk, 0);
+      s1[jt] = __builtin_amdgcn_raw_buffer_load_b128(rS1, at, blk, 0);
+    }
     f32x4 pk = zero, pq = zero, ek = zero;
     float z = 0.0f;
 #pragma unroll
     for (int jt = 0; jt < NT; ++jt) {
-      const int at = (16 * it + li) * DP + 16 * jt + 4 * grp, ka = li * LD + 16 * jt + 4 * grp;
-      const f32x4 s0 = has0 ? *(const f32x4*)(S0 + at) : zero, s1 = has1 ? *(const f32x4*)(S1 + at) : zero;
-      const f32x4 kv = *(const f32x4*)(sK + ka), qv = *(const f32x4*)(sQ + ka);
+      const f32x4 kf = *(const f32x4*)(sK + li * LD + 16 * jt + 4 * grp);
+      const f32x4 qf = *(const f32x4*)(sQ + li * LD + 16 * jt + 4 * grp);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        pk = mfma4(kv[e], s0[e], pk);
-        pq = mfma4(qv[e], s0[e], pq);
-        ek = mfma4(kv[e], s1[e], ek);
-        z = fmaf(s0[e], s1[e], z);
+        const float x0 = bits_f32(s0[jt][e]), x1 = bits_f32(s1[jt][e]);
+        pk = mfma4(kf[e], x0, pk);
+        pq = mfma4(qf[e], x0, pq);
+        ek = mfma4(kf[e], x1, ek);
+        z = fmaf(x0, x1, z);
       }
     }
     z += __shfl_xor(z, 16);
@@ -616,7 +679,7 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
   }
   __syncthreads();
 
-  if (rows) {
+  if (rows && first) {
     float dec = 1.0f;
 #pragma unroll
     for (int t = 0; t < CH; ++t) {
@@ -631,6 +694,8 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
       dec *= a[t];
     }
     // the decay's gradient
+    int io = i;
+    asm volatile("" : "+v"(io));  // (the offsets of its stores formed here, not kept since the loads)
     const rsrc_t rDA = p.alpha_per_row ? row_rsrc(p.dalpha) : head_rsrc(p.dalpha);
     float da[CH];
     {
@@ -649,23 +714,13 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
         }
         z *= a[t];
         da[t] = v;
-        if (p.alpha_per_row) bstore<TT>(rDA, el_off(t, i), v * a[t]);  // log space
+        if (p.alpha_per_row) bstore<TT>(rDA, el_off(t, io), v * a[t]);  // log space
       }
     }
-    if (!p.beta_per_head) {
-      const rsrc_t rDB = row_rsrc(p.dbeta);
-#pragma unroll
-      for (int t = 0; t < CH; ++t) bstore<TT>(rDB, el_off(t, i), db[t]);
-    }
-    // sums over the rows: M(t, s) at t (t + 1) / 2 + t - s, N(t, s) at 136 + s (s - 1) / 2 + s - 1 - t, then the
-    // per-head dbeta and dalpha; 64 at a time
+    if (!p.alpha_per_row) put_sums(da, NP + CH);
+  } else if (rows) {
+    // sums over the rows: M(t, s) at t (t + 1) / 2 + t - s, N(t, s) at 136 + s (s - 1) / 2 + s - 1 - t, 64 at a time
     float buf[64];
-#pragma unroll
-    for (int n = 0; n < 64; ++n) {
-      const bool ok = i < d;
-      buf[n] = n < CH ? (ok ? db[n < CH ? n : 0] : 0.0f) : n < 2 * CH ? (ok ? da[n < 2 * CH ? n - CH : 0] : 0.0f) : 0.0f;
-    }
-    red[w][NP + l] = scatter64(buf, l);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
 #pragma unroll
@@ -688,10 +743,31 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
           y *= a[t];
         }
       }
-      red[w][64 * q + l] = scatter64(buf, l);
+      red[w & 1][64 * q + l] = scatter64(buf, l);
     }
   }
   __syncthreads();
+
+  const int cg = w % NC, ks = w / NC, j0 = 16 * VC * cg + VC * li;  // this lane's columns j0 .. j0 + VC - 1
+  u32x4 s0[KX][4], s1[KX][4];
+  if (ks < KS) {
+#pragma unroll
+    for (int x = 0; x < KX; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int at = ((4 * grp + e) * DP + j0) * 4, blk = 16 * (KX * ks + x) * DP * 4;
+        if constexpr (VC == 4) {
+          s0[x][e] = __builtin_amdgcn_raw_buffer_load_b128(rS0, at, blk, 0);
+          s1[x][e] = __builtin_amdgcn_raw_buffer_load_b128(rS1, at, blk, 0);
+        } else {
+#pragma unroll
+          for (int n = 0; n < VC; ++n) {
+            s0[x][e][n] = __builtin_amdgcn_raw_buffer_load_b32(rS0, at + 4 * n, blk, 0);
+            s1[x][e][n] = __builtin_amdgcn_raw_buffer_load_b32(rS1, at + 4 * n, blk, 0);
+          }
+        }
+      }
+  }
   {
     float v = red[0][tid];
     if (DP == 128) v += red[DP == 128 ? 1 : 0][tid];
@@ -706,61 +782,80 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
       sN[t * LM + s] = v;
       sN[s * LM + t] = v;
     }
-    if (tid < 2 * CH) {
+    if (tid < 2 * CH && (tid < CH ? p.beta_per_head : !p.alpha_per_row)) {
       float sum = red[0][NP + tid];
       if (DP == 128) sum += red[DP == 128 ? 1 : 0][NP + tid];
-      if (tid < CH) {
-        if (p.beta_per_head) bstore<TT>(head_rsrc(p.dbeta), head_off(tid), sum);
-      } else if (!p.alpha_per_row) {
-        bstore<TT>(head_rsrc(p.dalpha), head_off(tid - CH), sum);
-      }
+      if (tid < CH) bstore<TT>(head_rsrc(p.dbeta), head_off(tid), sum);
+      else bstore<TT>(head_rsrc(p.dalpha), head_off(tid - CH), sum);
     }
   }
-  __syncthreads();
 
-  const rsrc_t rDQ = row_rsrc(p.dq), rDK = row_rsrc(p.dk);
-  const bool bad = sBad != 0;
-  for (int jt = w; jt < NT; jt += 4) {
-    f32x4 dq = zero, dk = zero;
-    const int j = 16 * jt + li;
+  // dq, dk: wave (cg, ks) forms the products of its rows; part 0 then finishes dq, part 1 dk
+  f32x4 dq[VC], dk[VC];
 #pragma unroll
-    for (int x = 0; x < NT; ++x) {
-      const int at = li * LD + 16 * x + 4 * grp;
+  for (int n = 0; n < VC; ++n) dq[n] = dk[n] = zero;
+  if (ks < KS) {
+#pragma unroll
+    for (int x = 0; x < KX; ++x) {
+      const int at = li * LD + 16 * (KX * ks + x) + 4 * grp;
       const f32x4 dv = *(const f32x4*)(sD + at), wn = *(const f32x4*)(sW + at), uv = *(const f32x4*)(sU + at);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int si = (16 * x + 4 * grp + e) * DP + j;
-        const float s0 = has0 ? S0[si] : 0.0f, s1 = has1 ? S1[si] : 0.0f;
-        dq = mfma4(dv[e], s0, dq);
-        dk = mfma4(wn[e], s0, dk);
-        dk = mfma4(uv[e], s1, dk);
-      }
-    }
-    if (!bad) {
-      const f32x4 mv = *(const f32x4*)(sM + li * LM + 4 * grp), nv = *(const f32x4*)(sN + li * LM + 4 * grp);
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int s = 4 * grp + e;
-        dq = mfma4(mv[e], sK[s * LD + j], dq);
-        dk = mfma4(nv[e], sK[s * LD + j], dk);
-        dk = mfma4(sM[s * LM + li], sQ[s * LD + j], dk);
-      }
-    } else {  // a step outside a sum must not enter it even with 0
-      for (int s = 0; s < CH; ++s)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int t = 4 * grp + r;
-          if (s <= t) dq[r] = fmaf(sM[t * LM + s], sK[s * LD + j], dq[r]);
-          if (s >= t) dk[r] = fmaf(sM[s * LM + t], sQ[s * LD + j], dk[r]);
-          if (s != t) dk[r] = fmaf(sN[t * LM + s], sK[s * LD + j], dk[r]);
+        for (int n = 0; n < VC; ++n) {
+          dq[n] = mfma4(dv[e], bits_f32(s0[x][e][n]), dq[n]);
+          dk[n] = mfma4(wn[e], bits_f32(s0[x][e][n]), dk[n]);
+          dk[n] = mfma4(uv[e], bits_f32(s1[x][e][n]), dk[n]);
         }
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      bstore<TT>(rDQ, el_off(4 * grp + r, j), dq[r]);
-      bstore<TT>(rDK, el_off(4 * grp + r, j), dk[r]);
+    for (int n = 0; n < VC; ++n) {
+      if (ks != 0) sh.part[0][ks - 1][cg][n][l] = dq[n];
+      if (ks != 1) sh.part[1][ks == 0 ? 0 : ks - 1][cg][n][l] = dk[n];
     }
   }
+  __syncthreads();
+  if (ks > 1) return;
+  const bool isq = ks == 0;
+  f32x4 acc[VC];
+#pragma unroll
+  for (int n = 0; n < VC; ++n) {
+    acc[n] = isq ? dq[n] : dk[n];
+#pragma unroll
+    for (int m = 0; m < KS - 1; ++m) acc[n] += sh.part[isq ? 0 : 1][m][cg][n][l];
+  }
+  if (!(sBad[0] | sBad[1] | sBad[2] | sBad[3])) {
+    const f32x4 av = *(const f32x4*)((isq ? sM : sN) + li * LM + 4 * grp);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int s = 4 * grp + e;
+#pragma unroll
+      for (int n = 0; n < VC; ++n) {
+        acc[n] = mfma4(av[e], sK[s * LD + j0 + n], acc[n]);
+        if (!isq) acc[n] = mfma4(sM[s * LM + li], sQ[s * LD + j0 + n], acc[n]);
+      }
+    }
+  } else {  // a step outside a sum must not enter it even with 0
+    for (int s = 0; s < CH; ++s)
+#pragma unroll
+      for (int n = 0; n < VC; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int t = 4 * grp + r;
+          const float ks_ = sK[s * LD + j0 + n];
+          if (isq) {
+            if (s <= t) acc[n][r] = fmaf(sM[t * LM + s], ks_, acc[n][r]);
+          } else {
+            if (s >= t) acc[n][r] = fmaf(sM[s * LM + t], sQ[s * LD + j0 + n], acc[n][r]);
+            if (s != t) acc[n][r] = fmaf(sN[t * LM + s], ks_, acc[n][r]);
+          }
+        }
+  }
+  const rsrc_t rDst = row_rsrc(isq ? p.dq : p.dk);
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int n = 0; n < VC; ++n) bstore<TT>(rDst, el_off(4 * grp + r, j0 + n), acc[n][r]);
 }
 
 template <typename TT, int DP>
