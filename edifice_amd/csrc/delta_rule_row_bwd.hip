@@ -294,6 +294,7 @@ struct GradArgs {
   const float *err, *du, *ckpt, *dckpt;
   void *dq, *dk, *dv, *dbeta;
   int H, T, d, beta_per_head;
+  bool vec;  // d a multiple of 8, tensors 4-byte aligned
 };
 
 EDF_DEVICE f32x16 mfma_f32(float a, float b, f32x16 c) {
@@ -303,6 +304,9 @@ EDF_DEVICE f32x16 mfma_f32(float a, float b, f32x16 c) {
 // One workgroup per 64 steps of a head.  Wave (ct, rt) forms the 32 x 32 tile of dq and of dk at steps
 // 32 rt .., columns 32 ct ..; the row factors do, u and -w are in LDS as float32, and so are the
 // 64 x 64 tiles M = do u^T (s <= t) and N = -(u w^T, its strict upper part, mirrored).
+// One workgroup per CU (136 KB of LDS at head_dim 128), so nothing else covers its waits: the row factors move in
+// 16-byte pieces (element by element 23k cycles of a workgroup's 93k at 8x2048x8x128 bf16, 10k so), and the states
+// arrive two stages of 32 rows ahead of their products (51k -> 42k, of which the f32 MFMAs take 32k).
 template <typename TT, int DP>
 __global__ __launch_bounds__(4 * DP) void dr_row_grad_kernel(const GradArgs p) {
   constexpr int LD = DP + 4, LM = CPS + 4, CT = DP / 32, NTH = 4 * DP, PER = DP / 4;
@@ -327,9 +331,144 @@ __global__ __launch_bounds__(4 * DP) void dr_row_grad_kernel(const GradArgs p) {
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, g = l >> 5, li = l & 31;
   const int ct = w % CT, rt = w / CT, j = 32 * ct + li;
 
+  const unsigned hd = (unsigned)(p.H * d);
+  // S0 and dS1 in stages of 32 rows (an empty buffer reads zero), two stages ahead
+  const bool has0 = C > 0, has1 = C < n64 - 1;
+  const rsrc_t rS0 = make_rsrc(p.ckpt + (has0 ? (bh * (n64 - 1) + C - 1) * DP * DP : 0), has0 ? DP * DP * 4u : 0u);
+  const rsrc_t rS1 = make_rsrc(p.dckpt + (has1 ? (bh * (n64 - 1) + C) * DP * DP : 0), has1 ? DP * DP * 4u : 0u);
+  constexpr int ST = DP / 32;
+  float sv[2][16];
+  auto load_stage = [&](int st, float (&v)[16]) {
+#pragma unroll
+    for (int x = 0; x < 16; ++x)
+      v[x] = bits_f32(__builtin_amdgcn_raw_buffer_load_b32(st < ST ? rS0 : rS1, (int)(((4 * g + (x & 3)) * DP + j) * 4),
+                                                           (32 * (st % ST) + 8 * (x >> 2)) * DP * 4, 0));
+  };
+
+  // row factors, dv and dbeta
+  if (p.vec) {  // eight columns at a time (a piece is inside the head or past it)
+    constexpr int P8 = DP / 8, NV = 4 * sizeof(TT) / 8;  // 16-byte pieces of 8 elements of TT
+    auto load8 = [](rsrc_t r, unsigned off, float (&v)[8]) {
+      if constexpr (sizeof(TT) == 4) {
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+          const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(off + 16 * y), 0, 0);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[4 * y + e] = bits_f32(x[e]);
+        }
+      } else {
+        const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[2 * e] = bits_f32(x[e] << 16);
+          v[2 * e + 1] = bits_f32(x[e] & 0xffff0000u);
+        }
+      }
+    };
+    auto load8f = [](rsrc_t r, unsigned off, float (&v)[8]) {
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(r, (int)(off + 16 * y), 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[4 * y + e] = bits_f32(x[e]);
+      }
+    };
+    auto store8 = [](rsrc_t r, unsigned off, const float (&v)[8]) {
+#pragma unroll
+      for (int y = 0; y < NV; ++y) {
+        u32x4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (sizeof(TT) == 4) {
+            x[e] = __builtin_bit_cast(unsigned, v[4 * y + e]);
+          } else {
+            typedef __attribute__((ext_vector_type(2))) bf16 bf16x2;
+            x[e] = __builtin_bit_cast(unsigned, bf16x2{(bf16)v[2 * e], (bf16)v[2 * e + 1]});
+          }
+        }
+        __builtin_amdgcn_raw_buffer_store_b128(x, r, (int)(off + 16 * y), 0, 0);
+      }
+    };
+    constexpr int NI = CPS * P8 / NTH;
+    float er[NI][8], du[NI][8], go[NI][8], be[NI][8];
+#pragma unroll
+    for (int n = 0; n < NI; ++n) {
+      const int e = tid + NTH * n, i0 = 8 * (e % P8);
+      const unsigned t = t0 + e / P8, el = t * hd + h * d + i0, o = i0 < d ? el * (unsigned)sizeof(TT) : OOB_OFF;
+      load8f(rE, i0 < d ? el * 4u : OOB_OFF, er[n]);
+      load8f(rU, i0 < d ? el * 4u : OOB_OFF, du[n]);
+      load8(rG, o, go[n]);
+      if (p.beta_per_head) {
+        be[n][0] = bits_f32(bload<TT>(rB, (t * p.H + h) * (unsigned)sizeof(TT)));
+#pragma unroll
+        for (int x = 1; x < 8; ++x) be[n][x] = be[n][0];
+      } else {
+        load8(rB, o, be[n]);
+      }
+    }
+    load_stage(0, sv[0]);
+#pragma unroll
+    for (int n = 0; n < NI; ++n) {
+      const int e = tid + NTH * n, row = e / P8, i0 = 8 * (e % P8);
+      const unsigned t = t0 + row, o = i0 < d ? (t * hd + h * d + i0) * (unsigned)sizeof(TT) : OOB_OFF;
+      float wv[8], db[8];
+#pragma unroll
+      for (int x = 0; x < 8; ++x) {
+        wv[x] = be[n][x] * du[n][x];
+        db[x] = er[n][x] * du[n][x];
+        sD[row * LD + i0 + x] = go[n][x];
+        sU[row * LD + i0 + x] = be[n][x] * er[n][x];
+        sW[row * LD + i0 + x] = -wv[x];
+      }
+      store8(rDV, o, wv);
+      if (!p.beta_per_head) {
+        store8(rDB, o, db);
+      } else {  // summed over the rows: the P8 lanes of this step
+        float v = ((db[0] + db[1]) + (db[2] + db[3])) + ((db[4] + db[5]) + (db[6] + db[7]));
+#pragma unroll
+        for (int m = 1; m < P8; m *= 2) v += __shfl_xor(v, m);
+        bstore<TT>(rDB, i0 == 0 ? (t * p.H + h) * (unsigned)sizeof(TT) : OOB_OFF, v);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int n = 0; n < CPS * PER / NTH; ++n) {
+      const int e = tid + NTH * n, row = e / PER, i0 = 4 * (e % PER);
+      const unsigned t = t0 + row, el = t * hd + h * d + i0;
+      f32x4 er, du, be, go;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const bool in = i0 + x < d;
+        const unsigned o = in ? (el + x) * (unsigned)sizeof(TT) : OOB_OFF;
+        er[x] = bits_f32(bload<float>(rE, in ? (el + x) * 4u : OOB_OFF));
+        du[x] = bits_f32(bload<float>(rU, in ? (el + x) * 4u : OOB_OFF));
+        go[x] = bits_f32(bload<TT>(rG, o));
+        be[x] = bits_f32(bload<TT>(rB, p.beta_per_head ? (t * p.H + h) * (unsigned)sizeof(TT) : o));
+      }
+      const f32x4 wv = be * du, db = er * du;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const unsigned o = i0 + x < d ? (el + x) * (unsigned)sizeof(TT) : OOB_OFF;
+        bstore<TT>(rDV, o, wv[x]);
+        if (!p.beta_per_head) bstore<TT>(rDB, o, db[x]);
+      }
+      if (p.beta_per_head) {  // summed over the rows: the PER lanes of this step
+        float s = (db[0] + db[1]) + (db[2] + db[3]);
+#pragma unroll
+        for (int m = 1; m < PER; m *= 2) s += __shfl_xor(s, m);
+        bstore<TT>(rDB, i0 == 0 ? (t * p.H + h) * (unsigned)sizeof(TT) : OOB_OFF, s);
+      }
+      *(f32x4*)(sD + row * LD + i0) = go;
+      *(f32x4*)(sU + row * LD + i0) = be * er;
+      *(f32x4*)(sW + row * LD + i0) = -wv;
+    }
+    load_stage(0, sv[0]);
+  }
+  __syncthreads();
+  load_stage(1, sv[1]);
+
   // this lane's k and q values of the 64 steps (column j, steps 8 kk + 4 g + e), used last
   typename Bits<TT>::type kr[CPS / 2], qr[CPS / 2];
-  const unsigned hd = (unsigned)(p.H * d);
 #pragma unroll
   for (int i = 0; i < CPS / 2; ++i) {
     const unsigned t = t0 + 8 * (i >> 2) + 4 * g + (i & 3);
@@ -337,40 +476,6 @@ __global__ __launch_bounds__(4 * DP) void dr_row_grad_kernel(const GradArgs p) {
     kr[i] = bload<TT>(rK, off);
     qr[i] = bload<TT>(rQ, off);
   }
-
-  // row factors, dv and dbeta
-#pragma unroll
-  for (int n = 0; n < CPS * PER / NTH; ++n) {
-    const int e = tid + NTH * n, row = e / PER, i0 = 4 * (e % PER);
-    const unsigned t = t0 + row, el = t * hd + h * d + i0;
-    f32x4 er, du, be, go;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const bool in = i0 + x < d;
-      const unsigned o = in ? (el + x) * (unsigned)sizeof(TT) : OOB_OFF;
-      er[x] = bits_f32(bload<float>(rE, in ? (el + x) * 4u : OOB_OFF));
-      du[x] = bits_f32(bload<float>(rU, in ? (el + x) * 4u : OOB_OFF));
-      go[x] = bits_f32(bload<TT>(rG, o));
-      be[x] = bits_f32(bload<TT>(rB, p.beta_per_head ? (t * p.H + h) * (unsigned)sizeof(TT) : o));
-    }
-    const f32x4 wv = be * du, db = er * du;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const unsigned o = i0 + x < d ? (el + x) * (unsigned)sizeof(TT) : OOB_OFF;
-      bstore<TT>(rDV, o, wv[x]);
-      if (!p.beta_per_head) bstore<TT>(rDB, o, db[x]);
-    }
-    if (p.beta_per_head) {  // summed over the rows: the PER lanes of this step
-      float s = (db[0] + db[1]) + (db[2] + db[3]);
-#pragma unroll
-      for (int m = 1; m < PER; m *= 2) s += __shfl_xor(s, m);
-      bstore<TT>(rDB, i0 == 0 ? (t * p.H + h) * (unsigned)sizeof(TT) : OOB_OFF, s);
-    }
-    *(f32x4*)(sD + row * LD + i0) = go;
-    *(f32x4*)(sU + row * LD + i0) = be * er;
-    *(f32x4*)(sW + row * LD + i0) = -wv;
-  }
-  __syncthreads();
 
   // the Gram tiles over the rows: M (0,0) (1,0) (1,1), N (0,0) (0,1) (1,1)
   for (int job = w; job < 6; job += 2 * CT) {
@@ -404,28 +509,29 @@ __global__ __launch_bounds__(4 * DP) void dr_row_grad_kernel(const GradArgs p) {
   const float* aD = sD + (32 * rt + li) * LD + 4 * g;
   const float* aU = sU + (32 * rt + li) * LD + 4 * g;
   const float* aW = sW + (32 * rt + li) * LD + 4 * g;
-  if (C > 0) {
-    const float* S0 = p.ckpt + ((bh * (n64 - 1) + C - 1) * DP + 4 * g) * DP + j;
-#pragma unroll 4
-    for (int kk = 0; kk < DP / 8; ++kk) {
-      const f32x4 dv = *(const f32x4*)(aD + 8 * kk), wv = *(const f32x4*)(aW + 8 * kk);
+  static_for<2 * ST>([&](auto sti) {
+    constexpr int st = decltype(sti)::value;
+    float(&v)[16] = sv[st & 1];
+    if (st < ST ? has0 : has1) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float s = S0[(8 * kk + e) * DP];
-        dq = mfma_f32(dv[e], s, dq);
-        dk = mfma_f32(wv[e], s, dk);
+      for (int x = 0; x < 4; ++x) {
+        const int at = 32 * (st % ST) + 8 * x;
+        if constexpr (st < ST) {
+          const f32x4 dv = *(const f32x4*)(aD + at), wv = *(const f32x4*)(aW + at);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            dq = mfma_f32(dv[e], v[4 * x + e], dq);
+            dk = mfma_f32(wv[e], v[4 * x + e], dk);
+          }
+        } else {
+          const f32x4 uv = *(const f32x4*)(aU + at);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) dk = mfma_f32(uv[e], v[4 * x + e], dk);
+        }
       }
     }
-  }
-  if (C < n64 - 1) {
-    const float* S1 = p.dckpt + ((bh * (n64 - 1) + C) * DP + 4 * g) * DP + j;
-#pragma unroll 4
-    for (int kk = 0; kk < DP / 8; ++kk) {
-      const f32x4 uv = *(const f32x4*)(aU + 8 * kk);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) dk = mfma_f32(uv[e], S1[(8 * kk + e) * DP], dk);
-    }
-  }
+    if constexpr (st + 2 < 2 * ST) load_stage(st + 2, v);
+  });
   __syncthreads();  // M and N
 
   bool finite = true;
@@ -871,7 +977,9 @@ void launch_bwd(hipStream_t s, const RowArgs& r, float* du, const GradArgs& a, c
   }
   vec ? dr_row_rev_kernel<TT, DP, false, true><<<grid, threads, 0, s>>>(r, du)
       : dr_row_rev_kernel<TT, DP, false, false><<<grid, threads, 0, s>>>(r, du);
-  dr_row_grad_kernel<TT, DP><<<(unsigned)((long)bh * ((r.T + CPS - 1) / CPS)), 4 * DP, 0, s>>>(a);
+  GradArgs g = a;
+  g.vec = r.d % 8 == 0 && (((uintptr_t)a.dout | (uintptr_t)a.beta | (uintptr_t)a.dv | (uintptr_t)a.dbeta) % 4 == 0);
+  dr_row_grad_kernel<TT, DP><<<(unsigned)((long)bh * ((r.T + CPS - 1) / CPS)), 4 * DP, 0, s>>>(g);
 }
 
 template <typename TT>
