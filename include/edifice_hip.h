@@ -257,8 +257,8 @@ int edf_fused_kda_scan_backward(void* stream, const void* q, const void* k, cons
                                 int dtype);
 
 /* No reference counterpart (its backward re-runs a checkpointing forward): a training KDA
- * forward that also keeps the states every 16 steps in a caller-kept context of
- * edf_kda_scan_context_bytes() bytes (one pass writes out and the states), and the backward
+ * forward that also keeps the states every 16 steps and the errors v - S k in a caller-kept context of
+ * edf_kda_scan_context_bytes() bytes (one pass writes out and both), and the backward
  * from that context (unchanged since), which then skips its forward re-run; gradients
  * bit-identical to edf_fused_kda_scan_backward, workspace edf_kda_scan_backward_workspace_bytes(). */
 size_t edf_kda_scan_context_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype);
@@ -399,7 +399,8 @@ int edf_fused_ttt_scan_backward_saved(void* stream, const void* q, const void* k
  * causal, dtype), nif.ex fused_flash_attention, and fused_flash_attention_launch
  * (native/cuda/fused_flash_attention.cu:168-191).  Extension: `lse` (may be NULL)
  * receives the row log-sum-exp for the backward.  bf16 with head_dim 32, 64 or 128
- * runs on MFMA; other head_dim (<= 256) and float32 run a wave-per-row kernel. */
+ * runs on bf16 MFMA, other head_dim <= 128 and float32 on float32 MFMA (bf16 forward, head_dim a multiple of 8:
+ * bf16 MFMA with P split into three exact bf16 parts), 128 < head_dim <= 256 a wave-per-row kernel. */
 int edf_fused_flash_attention(void* stream, const void* q, const void* k, const void* v, void* out, float* lse,
                               int batch, int num_heads, int seq_len, int head_dim, int causal, int dtype);
 
@@ -476,7 +477,8 @@ int edf_fused_laser_attention_backward(void* stream, const void* q, const void* 
  *   kernels) + seq_len >= 64 runs the chunked MFMA kernels,
  *   forward and backward, and then requires the workspace the *_workspace_bytes queries
  *   return (EDF_ERR_WORKSPACE when it is missing or short; the forward query returns 0
- *   for every other case); everything else runs the exact per-step kernels.
+ *   for every other case); everything else runs row scans, 16 steps at a time in
+ *   float32, or the per-step kernels where a batch row has 2 GiB and more.
  * ------------------------------------------------------------------------ */
 enum { EDF_BETA_PER_ELEMENT = 0, EDF_BETA_PER_HEAD = 1 };
 
@@ -522,13 +524,13 @@ int edf_fused_gated_delta_net_scan_backward(void* stream, const void* q, const v
  * context its forward call left in `forward_workspace` (the workspace of the forward with the
  * same q, k, v, beta, alpha, unchanged since).  On the chunked path (see above) this skips
  * the forward's recomputation; `workspace` needs
- * edf_delta_rule_saved_backward_workspace_bytes() bytes.  On the per-step path the forward's
+ * edf_delta_rule_saved_backward_workspace_bytes() bytes.  On the other paths the forward's
  * workspace is optional (edf_delta_rule_workspace_bytes() is 0 there); a forward workspace of
- * edf_delta_rule_forward_context_bytes() also receives the states every 16 steps, which this
- * backward then reads instead of recomputing them (bit-identical gradients); with a smaller
+ * edf_delta_rule_forward_context_bytes() also receives states and errors of
+ * its scan, which this backward then reads instead of recomputing them (bit-identical gradients); with a smaller
  * or NULL forward_workspace it recomputes, as edf_fused_gated_delta_net_scan_backward does.
  * edf_delta_rule_forward_context_bytes() is the chunked path's forward workspace on that
- * path and the per-step states otherwise: the forward workspace a training caller
+ * path and that record otherwise: the forward workspace a training caller
  * allocates for the saved backward. */
 size_t edf_delta_rule_forward_context_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype,
                                             int beta_mode);
