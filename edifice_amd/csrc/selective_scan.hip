@@ -124,7 +124,7 @@ __global__ __launch_bounds__(256) void ss_dtmean_kernel(const TI* __restrict__ d
   float s = 0.0f;
   constexpr int V = 16 / sizeof(TI);  // one 16-byte load per lane and step when the row allows it
   if (dim % V == 0 && ((uintptr_t)dt & 15) == 0) {
-    for (int d0 = lane * V; d0 < dim; d0 += 64 * V) {
+    for (int d0 = (blockIdx.y * 64 + lane) * V; d0 < dim; d0 += gridDim.y * 64 * V) {
       const uint4 u = *reinterpret_cast<const uint4*>(p + d0);
       const TI* e = reinterpret_cast<const TI*>(&u);
 #pragma unroll
@@ -794,7 +794,8 @@ __global__ __launch_bounds__(256) void ss_mean_fixup_kernel(const float* __restr
                                                             int ntile, long rows, int dim, int sp) {
   // 16 rows per workgroup.  The tile partials of a row sit `rows` apart (one per channel
   // tile): 16 lanes take 16 consecutive rows and the 16 lane groups a sixteenth of the tiles
-  // each, combined in a fixed order; then each wave updates whole rows, 16-byte accesses.
+  // each, combined in a fixed order; then each wave updates its rows' slice blockIdx.y of the
+  // columns, 16-byte accesses.
   constexpr int RW = 16;
   __shared__ float s_part[RW][RW + 1];
   __shared__ float s_tot[RW];
@@ -820,7 +821,7 @@ __global__ __launch_bounds__(256) void ss_mean_fixup_kernel(const float* __restr
     const float t = s_tot[r];
     const long base = (r0 + r) * dim;
     if (vec) {
-      for (int d0 = lane * V; d0 < dim; d0 += 64 * V) {
+      for (int d0 = (blockIdx.y * 64 + lane) * V; d0 < dim; d0 += gridDim.y * 64 * V) {
         const uint4 ud = *reinterpret_cast<const uint4*>(dt + base + d0);
         uint4 ug = *reinterpret_cast<const uint4*>(ddt + base + d0);
         const TI* vd = reinterpret_cast<const TI*>(&ud);
@@ -834,7 +835,7 @@ __global__ __launch_bounds__(256) void ss_mean_fixup_kernel(const float* __restr
         *reinterpret_cast<uint4*>(ddt + base + d0) = ug;
       }
     } else {
-      for (int d = lane; d < dim; d += 64) {
+      for (int d = blockIdx.y * 64 + lane; d < dim; d += gridDim.y * 64) {
         const float raw = ld(dt, base + d);
         const float dtr = sp ? softplus_f(raw) : raw;
         if (dtr >= DT_MIN && dtr <= DT_MAX)
@@ -1209,12 +1210,17 @@ int edf_fused_selective_scan_backward(void* stream, const void* x, const void* d
     if (rc) return rc;
   }
   if (mean_mode) {
+    // Few rows leave most CUs without a workgroup: the columns are then split too, up to 1024 workgroups, each
+    // slice forming the row totals again (the same sums): 2000 rows of 2048 bf16 24.7 -> 11.7 us.
+    const unsigned blocks = (unsigned)((rows + 15) / 16);
+    const int width = 64 * (io_dtype == EDF_BF16 ? 8 : 4);
+    const dim3 grid(blocks, (unsigned)std::max(1, std::min((hidden + width - 1) / width, (int)(1024 / blocks))));
     if (io_dtype == EDF_BF16)
-      ss_mean_fixup_kernel<bf16><<<(unsigned)((rows + 15) / 16), 256, 0, s>>>(
-          a.part_m, (const bf16*)dt, (bf16*)grad_dt, a.ntile, rows, hidden, a.dt_sp);
+      ss_mean_fixup_kernel<bf16><<<grid, 256, 0, s>>>(a.part_m, (const bf16*)dt, (bf16*)grad_dt, a.ntile, rows,
+                                                      hidden, a.dt_sp);
     else
-      ss_mean_fixup_kernel<float><<<(unsigned)((rows + 15) / 16), 256, 0, s>>>(
-          a.part_m, (const float*)dt, (float*)grad_dt, a.ntile, rows, hidden, a.dt_sp);
+      ss_mean_fixup_kernel<float><<<grid, 256, 0, s>>>(a.part_m, (const float*)dt, (float*)grad_dt, a.ntile, rows,
+                                                       hidden, a.dt_sp);
     rc = check_launch("selective scan dt-mean coupling");
     if (rc) return rc;
   }
