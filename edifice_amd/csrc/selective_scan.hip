@@ -124,7 +124,7 @@ __global__ __launch_bounds__(256) void ss_dtmean_kernel(const TI* __restrict__ d
   float s = 0.0f;
   constexpr int V = 16 / sizeof(TI);  // one 16-byte load per lane and step when the row allows it
   if (dim % V == 0 && ((uintptr_t)dt & 15) == 0) {
-    for (int d0 = (blockIdx.y * 64 + lane) * V; d0 < dim; d0 += gridDim.y * 64 * V) {
+    for (int d0 = lane * V; d0 < dim; d0 += 64 * V) {
       const uint4 u = *reinterpret_cast<const uint4*>(p + d0);
       const TI* e = reinterpret_cast<const TI*>(&u);
 #pragma unroll
