@@ -270,7 +270,7 @@ __global__ __launch_bounds__(256, DP <= 64 ? 2 : 1) void fa32_fwd_kernel(const A
     for (int x = 1; x < 16; ++x) mt = fmaxf(mt, s[x]);
     mt = fmaxf(mt, __shfl_xor(mt, 32));
     const float mn = fmaxf(m, mt);
-    const float c = mn * a.scale_log2;
+    const float c = mn == -INFINITY ? 0.0f : mn * a.scale_log2;  // (no finite score yet: every p is 0)
     const float al = m == -INFINITY ? 0.0f : fast_exp2(fmaf(m, a.scale_log2, -c));
     f32x16 p;
     float rs = 0.0f;
@@ -309,8 +309,8 @@ __global__ __launch_bounds__(256, DP <= 64 ? 2 : 1) void fa32_fwd_kernel(const A
     for (int i = 1; i < NW; ++i) mx = fmaxf(mx, sM[i][row]);
     float sum = 0.0f;
 #pragma unroll
-    for (int i = 0; i < NW; ++i)
-      sum += sM[i][row] == -INFINITY ? 0.0f : sL[i][row] * fast_exp2((sM[i][row] - mx) * a.scale_log2);
+    for (int i = 0; i < NW; ++i)  // (a wave without a finite score has the sum 0, or NaN where a score was)
+      sum += sM[i][row] == -INFINITY ? sL[i][row] : sL[i][row] * fast_exp2((sM[i][row] - mx) * a.scale_log2);
     return sum;
   };
   if (threadIdx.x < RB && q0 + threadIdx.x < T && a.lse_out != nullptr) {

@@ -93,3 +93,31 @@ def test_masked_values_take_no_part(d, dtype, rng):
     got = _run(q, k, v, bad_do, dtype, True)
     for i in (2, 3):
         assert torch.allclose(got[i][:, :, cut:], base[i][:, :, cut:], **near)
+
+
+@pytest.mark.parametrize("d,dtype", [(40, torch.float32), (64, torch.float32), (128, torch.float32),
+                                     (36, torch.bfloat16), (96, torch.bfloat16)], ids=str)
+@pytest.mark.parametrize("kind", ["plain", "causal", "fox"])
+def test_only_visible_score_of_a_tile_is_minus_infinity(kind, d, dtype, rng):
+    """A key whose score is -inf has probability 0, also where it is all that a query sees of a 32-key tile:
+    causal, key 32 is all that query 32 sees of its last tile; otherwise it is the whole last tile of 33 keys."""
+    announce("minus_infinity_tile", kind=kind, d=d, dtype=dtype)
+    shape = (1, 2, 33 if kind == "plain" else 40, d)
+    q, k, v, do = (rng.normal(scale=d ** -0.25, size=shape) for _ in range(4))
+    q[..., 0] = -np.abs(q[..., 0]) - 0.1
+    k[:, :, 32, 0] = np.inf
+    cs = np.cumsum(-np.abs(rng.normal(scale=0.2, size=shape[:3])), axis=-1) if kind == "fox" else None
+    got = _run(q, k, v, do, dtype, kind != "plain", cs)
+    qr, kr, vr, dor = (rounded(a, dtype) for a in (q, k, v, do))
+    kr[:, :, 32] = 0  # its score enters nothing: the reference leaves the key out by a bias
+    s = np.einsum("bhid,bhjd->bhij", qr, kr) / np.sqrt(d)
+    if kind == "fox":
+        cr = rounded(cs, dtype)
+        s += cr[..., :, None] - cr[..., None, :]
+    if kind != "plain":
+        s = np.where(np.tril(np.ones(s.shape[-2:], bool)), s, -np.inf)
+    s[..., 32] = -np.inf
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    assert_close(host(got[0]), np.einsum("bhij,bhjd->bhid", p, vr), TOL[dtype], "o")
+    assert_close(host(got[3]), np.einsum("bhij,bhid->bhjd", p, dor), TOL[dtype], "dv")
