@@ -28,7 +28,7 @@
 //   gram    forms the Gram tiles of chunk c + 1, the outputs of chunk c - 1, and stages k and q.
 // Forward without states, per call, against the per-step kernel it replaces (one lane per 8 state entries,
 // 574 cycles a step): 8 x 2048 x 8 x 128 bf16 529 -> 143 us, 4 x 1000 x 8 x 128 KDA 247 -> 94 us,
-// 2 x 777 x 8 x 64 f32 gated 129 -> 95 us.  One wave per block doing everything took 246 us for the first,
+// 2 x 777 x 8 x 64 f32 gated 129 -> 104 us.  One wave per block doing everything took 246 us for the first,
 // a chain wave that also held the state 235 us.
 #include "edf_abi.hpp"
 #include "edf_common.hpp"
@@ -54,6 +54,9 @@ template <typename TT, int DP, bool DECAY, bool VEC>
 __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_fwd_kernel(const RowArgs p) {
   typedef RowShared<TT, DP> Sh;
   constexpr int LD = Sh::LD, SW = Sh::SW, W = DP / SW;
+  // float32 sums the chunk's own terms apart from the state's and takes v last (edf_row_scan.hpp); bf16 values carry
+  // their rounding anyway and save the instructions
+  constexpr bool F32 = sizeof(TT) == 4;
   __shared__ __attribute__((aligned(16))) Sh sh;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l = threadIdx.x & 63, li = l & 15, grp = l >> 4;
@@ -90,10 +93,13 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_fwd_kern
       f32x4 gs[4][2];
 #pragma unroll
       for (int r = 0; r < 4; ++r) gs[r][0] = *(const f32x4*)&sh.gs[b][8 * r], gs[r][1] = *(const f32x4*)&sh.gs[b][8 * r + 4];
-      float v[4], bb[4][4], aa[4][4];
+      float vv[4][4], bb[4][4], aa[4][4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        v[r] = bits_f32(nv.v[r]);
+        if constexpr (F32)
+          gather4(bits_f32(nv.v[r]), vv[r]);
+        else
+          vv[r][0] = bits_f32(nv.v[r]);  // this lane's step
         gather4(bits_f32(nb.v[r]), bb[r]);
         if (DECAY)
           gather4(decay_of<TT>(na.v[r], t0 + 4 * r + grp < p.T && io.in, p.alpha_per_row), aa[r]);
@@ -101,32 +107,38 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_fwd_kern
           aa[r][0] = aa[r][1] = aa[r][2] = aa[r][3] = 1.0f;
       }
       load();  // the next chunk's, under this chunk's work
-      if (DECAY) pk *= dtot;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) pk = mfma4(Gx[r], U[r], pk);
-      f32x4 raw;
+      pk = tile_dot<F32>(Gx, U, DECAY ? pk * dtot : pk);
+      f32x4 raw, in = {0, 0, 0, 0};  // in: the part of p from the chunk's own steps (bf16: in pk)
       dtot = 1.0f;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         auto g = [&](int m, int n) { return gs[r][pair(m, n) >> 2][pair(m, n) & 3]; };
         const BlockDecay D(aa[r], grp);
         float y[4], u[4];
-        gather4(DECAY ? fmaf(-D.pre, pk[r], v[r]) : v[r] - pk[r], y);
+        const float pr = F32 ? pk[r] + in[r] : pk[r];
+        if constexpr (F32)
+          gather4(DECAY ? D.pre * pr : pr, y);
+        else
+          gather4(DECAY ? fmaf(D.pre, pr, -vv[r][0]) : pr - vv[r][0], y);
+        auto last = [&](float t, int m) { return F32 ? vv[r][m] - t : -t; };
+        y[0] = last(y[0], 0);
         u[0] = bb[r][0] * y[0];
-        y[1] = fmaf(-(DECAY ? g(0, 1) * D.r10 : g(0, 1)), u[0], y[1]);
+        y[1] = last(fmaf(DECAY ? g(0, 1) * D.r10 : g(0, 1), u[0], y[1]), 1);
         u[1] = bb[r][1] * y[1];
-        y[2] = fmaf(-(DECAY ? g(1, 2) * D.r21 : g(1, 2)), u[1],
-                    fmaf(-(DECAY ? g(0, 2) * D.r20 : g(0, 2)), u[0], y[2]));
+        y[2] = last(fmaf(DECAY ? g(1, 2) * D.r21 : g(1, 2), u[1],
+                         fmaf(DECAY ? g(0, 2) * D.r20 : g(0, 2), u[0], y[2])), 2);
         u[2] = bb[r][2] * y[2];
-        y[3] = fmaf(-(DECAY ? g(2, 3) * D.r32 : g(2, 3)), u[2],
-                    fmaf(-(DECAY ? g(1, 3) * D.r31 : g(1, 3)), u[1],
-                         fmaf(-(DECAY ? g(0, 3) * D.r30 : g(0, 3)), u[0], y[3])));
+        y[3] = last(fmaf(DECAY ? g(2, 3) * D.r32 : g(2, 3), u[2],
+                         fmaf(DECAY ? g(1, 3) * D.r31 : g(1, 3), u[1],
+                              fmaf(DECAY ? g(0, 3) * D.r30 : g(0, 3), u[0], y[3]))), 3);
         u[3] = bb[r][3] * y[3];
         if (keep) bstore<float>(rE, eoff + 4 * r * estep, pick4(y[0], y[1], y[2], y[3], grp));
         const float uo = pick4(u[0], u[1], u[2], u[3], grp);
         const float ue = DECAY ? uo * D.end : uo;
-        if (r < 3) pk = mfma4(G[r], ue, DECAY ? pk * D.all : pk);
+        f32x4& own = F32 ? in : pk;
+        if (r < 3) own = mfma4(G[r], ue, DECAY ? own * D.all : own);
         if (DECAY) {
+          if (F32) pk *= D.all;
 #pragma unroll
           for (int e = 0; e < r; ++e) U[e] *= D.all;
           dtot *= D.all;
@@ -205,13 +217,13 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_fwd_kern
       RowFrag<TT, DP> kf, qf;
       kf.template load<LD>(sh.k[c & 3], li, grp);
       qf.template load<LD>(sh.q[c % 3], li, grp);
-      const f32x4 G = gram<DP>(kf, kf);
+      const f32x4 G = gram<DECAY, DP>(kf, kf);
       sh.g[c & 1][l] = G;
       const float gv = gr == 0 ? G[0] : gr == 1 ? G[1] : gr == 2 ? G[2] : G[3];
       if (gm < gn) sh.gs[c & 1][8 * gr + pair(gm, gn)] = gv;
-      sh.gx[c & 1][l] = gram<DP>(kp, kf);
+      sh.gx[c & 1][l] = gram<DECAY, DP>(kp, kf);
       kp = kf;
-      return gram<DP>(kf, qf);
+      return gram<DECAY, DP>(kf, qf);
     };
     auto stage = [&](int c) {  // chunk c into its slot, chunk c + 1 on its way
       nk.store(sh.k[c & 3], l);
@@ -241,11 +253,14 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_fwd_kern
         if (!DECAY && !__any(!finite)) {
           // o = S q of the state before, plus u_s (k_s . q_t) over the steps s <= t of the chunk (a later
           // step's u enters with 0, so all must be finite)
+          f32x4 h;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) pq = mfma4(4 * r + grp <= t ? Hp[r] : 0.0f, U[r], pq);
+          for (int r = 0; r < 4; ++r) h[r] = 4 * r + grp <= t ? Hp[r] : 0.0f;
+          pq = tile_dot<F32>(h, U, pq);
 #pragma unroll
           for (int r = 0; r < 4; ++r) bstore<TT>(io.rO, ooff + 4 * r * io.step, pq[r]);
         } else {
+          f32x4 in = {0, 0, 0, 0};  // the part of o from the chunk's blocks before
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             float aa[4] = {1.0f, 1.0f, 1.0f, 1.0f}, u[4];
@@ -253,7 +268,7 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_fwd_kern
               gather4(decay_of<TT>(na.v[r], (c - 1) * CH + 4 * r + grp < p.T && io.in, p.alpha_per_row), aa);
             const BlockDecay D(aa, grp);
             gather4(U[r], u);
-            float o = D.pre * pq[r];
+            float o = F32 ? 0.0f : D.pre * pq[r];
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
               // decay from after step m to the lane's step; k_m . q of the lane's step
@@ -264,8 +279,11 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_fwd_kern
               const float hm = __shfl(Hp[r], 16 * m + 4 * grp + r);
               o = m <= grp ? fmaf(u[m] * rm, hm, o) : o;
             }
+            if (F32) o = fmaf(D.pre, pq[r] + in[r], o);
             bstore<TT>(io.rO, ooff + 4 * r * io.step, o);
-            if (r < 3) pq = mfma4(Hp[r], U[r] * D.end, pq * D.all);
+            f32x4& own = F32 ? in : pq;
+            if (r < 3) own = mfma4(Hp[r], U[r] * D.end, own * D.all);
+            if (F32) pq *= D.all;
           }
           if (DECAY) na.load(io.rA, io.astep, CH);
         }

@@ -22,7 +22,7 @@
 // the decay's gradient <dS_t - w_t k_t^T, S_{t-1}>, are formed one row per lane (dr_row_decay_grad_kernel).
 // Forward and backward, against one workgroup per 16 rows stepping through the sequence with partial dq and
 // dk per row block (its time is the chain of T steps): KDA 4x1000x8x128 bf16 875 -> 344 us,
-// GatedDeltaNet 2x777x8x64 float32 436 -> 213.
+// GatedDeltaNet 2x777x8x64 float32 470 -> 236 (213 before its float32 sums were split, see gram).
 #include "edf_abi.hpp"
 #include "edf_common.hpp"
 #include "edf_row_scan.hpp"
@@ -56,6 +56,8 @@ template <typename TT, int DP, bool DECAY, bool VEC>
 __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_rev_kernel(const RowArgs p, float* du) {
   typedef RevShared<TT, DP, DECAY> Sh;
   constexpr int LD = Sh::LD, SW = Sh::SW, W = DP / SW;
+  constexpr bool F32 = sizeof(TT) == 4;    // sums apart, as in the forward
+  constexpr bool LAST = DECAY && F32;
   __shared__ __attribute__((aligned(16))) Sh sh;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l = threadIdx.x & 63, li = l & 15, grp = l >> 4;
@@ -105,35 +107,43 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_rev_kern
         }
       }
       load();
-#pragma unroll
-      for (int r = 0; r < 4; ++r) e = mfma4(Gx[r], Wn[r], e);
-      if (DECAY) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) e = mfma4(Hx[r], Dn[r], e);
-      }
+      e = tile_dot<F32>(Gx, Wn, e);
+      if (DECAY) e = tile_dot<F32>(Hx, Dn, e);
       dtot = 1.0f;
-      f32x4 raw;
+      f32x4 raw, in = {0, 0, 0, 0};  // in: the part of e from the chunk's own steps (bf16: in e)
 #pragma unroll
       for (int r = 3; r >= 0; --r) {
         auto g = [&](int m, int n) { return gs[r][pair(m, n) >> 2][pair(m, n) & 3]; };
         const BlockDecay D(aa[r], grp);
         float y[4], w[4];
-        gather4(DECAY ? fmaf(D.end, e[r], x[r]) : e[r], y);
+        // what the chunk's do give within the block enters last (float32), as v in the forward
+        const float er = F32 ? e[r] + in[r] : e[r];
+        if constexpr (LAST)
+          gather4(D.end * er, y);
+        else
+          gather4(DECAY ? fmaf(D.end, er, x[r]) : er, y);
+        float xx[4] = {};
+        if constexpr (LAST) gather4(x[r], xx);
+        auto last = [&](float v, int m) { return LAST ? v + xx[m] : v; };
+        y[3] = last(y[3], 3);
         w[3] = bb[r][3] * y[3];
-        y[2] = fmaf(-(DECAY ? g(2, 3) * D.r32 : g(2, 3)), w[3], y[2]);
+        y[2] = last(fmaf(-(DECAY ? g(2, 3) * D.r32 : g(2, 3)), w[3], y[2]), 2);
         w[2] = bb[r][2] * y[2];
-        y[1] = fmaf(-(DECAY ? g(1, 2) * D.r21 : g(1, 2)), w[2], fmaf(-(DECAY ? g(1, 3) * D.r31 : g(1, 3)), w[3], y[1]));
+        y[1] = last(fmaf(-(DECAY ? g(1, 2) * D.r21 : g(1, 2)), w[2],
+                         fmaf(-(DECAY ? g(1, 3) * D.r31 : g(1, 3)), w[3], y[1])), 1);
         w[1] = bb[r][1] * y[1];
-        y[0] = fmaf(-(DECAY ? g(0, 1) * D.r10 : g(0, 1)), w[1],
-                    fmaf(-(DECAY ? g(0, 2) * D.r20 : g(0, 2)), w[2],
-                         fmaf(-(DECAY ? g(0, 3) * D.r30 : g(0, 3)), w[3], y[0])));
+        y[0] = last(fmaf(-(DECAY ? g(0, 1) * D.r10 : g(0, 1)), w[1],
+                         fmaf(-(DECAY ? g(0, 2) * D.r20 : g(0, 2)), w[2],
+                              fmaf(-(DECAY ? g(0, 3) * D.r30 : g(0, 3)), w[3], y[0]))), 0);
         w[0] = bb[r][0] * y[0];
         const float wo = -pick4(w[0], w[1], w[2], w[3], grp), wn = DECAY ? wo * D.pre : wo;
         raw[r] = wo;
-        if (r > 0) e = mfma4(G[r], wn, DECAY ? e * D.all : e);
+        f32x4& own = F32 ? in : e;
+        if (r > 0) own = mfma4(G[r], wn, DECAY ? own * D.all : own);
         if (DECAY) {
           const float dn = dc[r] * D.pre;
-          if (r > 0) e = mfma4(H[r], dn, e);
+          if (r > 0) own = mfma4(H[r], dn, own);
+          if (F32) e *= D.all;
 #pragma unroll
           for (int n = r + 1; n < 4; ++n) Wn[n] *= D.all, Dn[n] *= D.all;
           Dn[r] = dn;
@@ -213,9 +223,9 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_rev_kern
       qf.template load<LD>(sh.q[j & 3], li, grp);
       const f32x4 dc = {bits_f32(nd.v[0]), bits_f32(nd.v[1]), bits_f32(nd.v[2]), bits_f32(nd.v[3])};
       nd.load(io.rV, io.step, -CH);
-      const f32x4 G = gram<DP>(kf, kf), H = gram<DP>(qf, kf), Hx = gram<DP>(qp, kf);
+      const f32x4 G = gram<DECAY, DP>(kf, kf), H = gram<DECAY, DP>(qf, kf), Hx = gram<DECAY, DP>(qp, kf);
       sh.g[j & 1][l] = G;
-      sh.gx[j & 1][l] = gram<DP>(kp, kf);
+      sh.gx[j & 1][l] = gram<DECAY, DP>(kp, kf);
       const float gv = gr == 0 ? G[0] : gr == 1 ? G[1] : gr == 2 ? G[2] : G[3];
       if (gm < gn) sh.gs[j & 1][8 * gr + pair(gm, gn)] = gv;
       f32x4 x = {0, 0, 0, 0};
@@ -230,7 +240,8 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_rev_kern
           gather4(dc[r], dd);
           const BlockDecay D(aa, grp);
 #pragma unroll
-          for (int s = 0; s < 4; ++s) {
+          for (int n = 0; n < 4; ++n) {
+            const int s = F32 ? 3 - n : n;  // (float32: the lane's own step, whose term is the largest, last)
             // decay from after the lane's step to step s; q_s . k of the lane's step
             const float rs = s == 3   ? pick4(D.r30, D.r31, D.r32, 1.0f, grp)
                              : s == 2 ? pick4(D.r20, D.r21, 1.0f, 1.0f, grp)
@@ -245,14 +256,15 @@ __global__ __launch_bounds__(64 * (2 + (DP >= 64 ? 2 : 1))) void dr_row_rev_kern
         kp = kf, qp = qf;
         return;
       }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) x = mfma4(Hx[r], dp[r], x);
+      x = tile_dot<F32>(Hx, dp, x);
       const bool finite = fabsf(dc[0]) < INFINITY && fabsf(dc[1]) < INFINITY && fabsf(dc[2]) < INFINITY &&
                           fabsf(dc[3]) < INFINITY;
       if (!__any(!finite)) {
         // do_s (q_s . k_t) over the steps s >= t of the chunk (an earlier step's do enters with 0)
+        f32x4 h;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) x = mfma4(4 * r + grp >= t ? H[r] : 0.0f, dc[r], x);
+        for (int r = 0; r < 4; ++r) h[r] = 4 * r + grp >= t ? H[r] : 0.0f;
+        x = tile_dot<F32>(h, dc, x);
       } else {
 #pragma unroll
         for (int s = 0; s < CH; ++s) {
@@ -310,6 +322,7 @@ EDF_DEVICE f32x16 mfma_f32(float a, float b, f32x16 c) {
 template <typename TT, int DP>
 __global__ __launch_bounds__(4 * DP) void dr_row_grad_kernel(const GradArgs p) {
   constexpr int LD = DP + 4, LM = CPS + 4, CT = DP / 32, NTH = 4 * DP, PER = DP / 4;
+  constexpr int NA = sizeof(TT) == 4 ? 2 : 1;  // accumulators per sum (see below)
   __shared__ __attribute__((aligned(16))) float sD[CPS * LD], sU[CPS * LD], sW[CPS * LD];
   __shared__ __attribute__((aligned(16))) float sM[CPS * LM], sN[CPS * LM];
   const int n64 = (p.T + CPS - 1) / CPS;
@@ -484,28 +497,38 @@ __global__ __launch_bounds__(4 * DP) void dr_row_grad_kernel(const GradArgs p) {
     const int tr = isM ? (jj > 0) : (jj > 1), tc = isM ? (jj > 1) : (jj > 0);
     const float* A = (isM ? sD : sU) + (32 * tr + li) * LD + 4 * g;
     const float* B = (isM ? sU : sW) + (32 * tc + li) * LD + 4 * g;
-    f32x16 acc = zero16();
+    f32x16 acc[NA];
+#pragma unroll
+    for (int n = 0; n < NA; ++n) acc[n] = zero16();
 #pragma unroll 4
     for (int kk = 0; kk < DP / 8; ++kk) {
       const f32x4 av = *(const f32x4*)(A + 8 * kk), bv = *(const f32x4*)(B + 8 * kk);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = mfma_f32(av[e], bv[e], acc);
+      for (int e = 0; e < 4; ++e) acc[e % NA] = mfma_f32(av[e], bv[e], acc[e % NA]);
     }
+#pragma unroll
+    for (int n = 1; n < NA; ++n) acc[0] += acc[n];
     const int col = 32 * tc + li;
 #pragma unroll
     for (int x = 0; x < 16; ++x) {
       const int row = 32 * tr + d_row(x, g);
       if (isM) {
-        sM[row * LM + col] = col <= row ? acc[x] : 0.0f;
+        sM[row * LM + col] = col <= row ? acc[0][x] : 0.0f;
       } else if (row <= col) {
-        const float v = row < col ? acc[x] : 0.0f;
+        const float v = row < col ? acc[0][x] : 0.0f;
         sN[row * LM + col] = v;
         sN[col * LM + row] = v;
       }
     }
   }
 
-  f32x16 dq = zero16(), dk = zero16();
+  // float32: the terms of S0, dS1 and the chunk's own steps in accumulators of their own
+  f32x16 dqs[NA], dks[2 * NA - 1];
+#pragma unroll
+  for (int n = 0; n < NA; ++n) dqs[n] = zero16();
+#pragma unroll
+  for (int n = 0; n < 2 * NA - 1; ++n) dks[n] = zero16();
+  f32x16 &dq = dqs[0], &dk = dks[0], &dk1 = dks[NA - 1], &dqc = dqs[NA - 1], &dkc = dks[2 * NA - 2];
   const float* aD = sD + (32 * rt + li) * LD + 4 * g;
   const float* aU = sU + (32 * rt + li) * LD + 4 * g;
   const float* aW = sW + (32 * rt + li) * LD + 4 * g;
@@ -526,7 +549,7 @@ __global__ __launch_bounds__(4 * DP) void dr_row_grad_kernel(const GradArgs p) {
         } else {
           const f32x4 uv = *(const f32x4*)(aU + at);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) dk = mfma_f32(uv[e], v[4 * x + e], dk);
+          for (int e = 0; e < 4; ++e) dk1 = mfma_f32(uv[e], v[4 * x + e], dk1);
         }
       }
     }
@@ -547,17 +570,18 @@ __global__ __launch_bounds__(4 * DP) void dr_row_grad_kernel(const GradArgs p) {
       const bool useM = rt == 1 || kk < 4, useT = rt == 0 || kk >= 4;
       const f32x4 nv = *(const f32x4*)(aN + 8 * kk);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) dk = mfma_f32(nv[e], bits_f32(kr[4 * kk + e]), dk);
+      for (int e = 0; e < 4; ++e) dkc = mfma_f32(nv[e], bits_f32(kr[4 * kk + e]), dkc);
       if (useM) {
         const f32x4 mv = *(const f32x4*)(aM + 8 * kk);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) dq = mfma_f32(mv[e], bits_f32(kr[4 * kk + e]), dq);
+        for (int e = 0; e < 4; ++e) dqc = mfma_f32(mv[e], bits_f32(kr[4 * kk + e]), dqc);
       }
       if (useT) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) dk = mfma_f32(aT[(8 * kk + e) * LM], bits_f32(qr[4 * kk + e]), dk);
+        for (int e = 0; e < 4; ++e) dkc = mfma_f32(aT[(8 * kk + e) * LM], bits_f32(qr[4 * kk + e]), dkc);
       }
     }
+    if constexpr (NA > 1) dq += dqc, dk += dk1 + dkc;
   } else {  // a step outside a sum must not enter it even with 0: the pairs one by one
 #pragma unroll 1
     for (int s = 0; s < CPS; ++s) {
@@ -571,6 +595,7 @@ __global__ __launch_bounds__(4 * DP) void dr_row_grad_kernel(const GradArgs p) {
         if (s != t) dk[x] = fmaf(sN[t * LM + s], ks, dk[x]);
       }
     }
+    if constexpr (NA > 1) dk += dk1;
   }
 #pragma unroll
   for (int x = 0; x < 16; ++x) {
@@ -744,8 +769,10 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
       s0[jt] = __builtin_amdgcn_raw_buffer_load_b128(rS0, at, blk, 0);
       s1[jt] = __builtin_amdgcn_raw_buffer_load_b128(rS1, at, blk, 0);
     }
-    f32x4 pk = zero, pq = zero, ek = zero;
-    float z = 0.0f;
+    // float32: several chains, added as a tree (four at 128 columns spill: 768 -> 864 us, KDA 8x777x8x128)
+    constexpr int NA = sizeof(TT) == 4 ? (DP == 128 ? 2 : 4) : 1;
+    f32x4 pk[NA] = {}, pq[NA] = {}, ek[NA] = {};
+    float zs[NA] = {};
 #pragma unroll
     for (int jt = 0; jt < NT; ++jt) {
       const f32x4 kf = *(const f32x4*)(sK + li * LD + 16 * jt + 4 * grp);
@@ -753,35 +780,46 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float x0 = bits_f32(s0[jt][e]), x1 = bits_f32(s1[jt][e]);
-        pk = mfma4(kf[e], x0, pk);
-        pq = mfma4(qf[e], x0, pq);
-        ek = mfma4(kf[e], x1, ek);
-        z = fmaf(x0, x1, z);
+        pk[e % NA] = mfma4(kf[e], x0, pk[e % NA]);
+        pq[e % NA] = mfma4(qf[e], x0, pq[e % NA]);
+        ek[e % NA] = mfma4(kf[e], x1, ek[e % NA]);
+        zs[e % NA] = fmaf(x0, x1, zs[e % NA]);
       }
     }
+    auto sum = [&](auto at) {  // at(n), n < NA, as a tree
+      if constexpr (NA == 4) return (at(0) + at(1)) + (at(2) + at(3));
+      else if constexpr (NA == 2) return at(0) + at(1);
+      else return at(0);
+    };
+    float z = sum([&](int n) { return zs[n]; });
     z += __shfl_xor(z, 16);
     z += __shfl_xor(z, 32);
     if (grp == 0) sZ[16 * it + li] = z;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int at = (4 * grp + r) * LD + 16 * it + li;
-      sP[at] = pk[r];
-      sO[at] = pq[r];
-      sE[at] = ek[r];
+      sP[at] = sum([&](int n) { return pk[n][r]; });
+      sO[at] = sum([&](int n) { return pq[n][r]; });
+      sE[at] = sum([&](int n) { return ek[n][r]; });
     }
   }
   if (w >= 2) {  // G(t, s) = k_t . k_s, H(t, s) = q_t . k_s
-    f32x4 acc = zero;
+    constexpr int NG = sizeof(TT) == 4 ? 8 : 1;  // chains, as in gram
+    f32x4 acc[NG] = {};
     const float* A = w == 2 ? sK : sQ;
 #pragma unroll
     for (int jt = 0; jt < NT; ++jt) {
       const int at = li * LD + 16 * jt + 4 * grp;
       const f32x4 av = *(const f32x4*)(A + at), bv = *(const f32x4*)(sK + at);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = mfma4(av[e], bv[e], acc);
+      for (int e = 0; e < 4; ++e) acc[(4 * jt + e) % NG] = mfma4(av[e], bv[e], acc[(4 * jt + e) % NG]);
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) (w == 2 ? sG : sH)[(4 * grp + r) * CH + li] = acc[r];
+    for (int n = NG / 2; n > 0; n /= 2)
+#pragma unroll
+      for (int m = 0; m < n; ++m) acc[m] += acc[m + n];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) (w == 2 ? sG : sH)[(4 * grp + r) * CH + li] = acc[0][r];
   }
   __syncthreads();
 
@@ -897,9 +935,9 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
   }
 
   // dq, dk: wave (cg, ks) forms the products of its rows; part 0 then finishes dq, part 1 dk
-  f32x4 dq[VC], dk[VC];
+  f32x4 dq[VC], dk[VC], dk1[VC];  // (float32: the terms of dS1 by themselves)
 #pragma unroll
-  for (int n = 0; n < VC; ++n) dq[n] = dk[n] = zero;
+  for (int n = 0; n < VC; ++n) dq[n] = dk[n] = dk1[n] = zero;
   if (ks < KS) {
 #pragma unroll
     for (int x = 0; x < KX; ++x) {
@@ -911,8 +949,13 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
         for (int n = 0; n < VC; ++n) {
           dq[n] = mfma4(dv[e], bits_f32(s0[x][e][n]), dq[n]);
           dk[n] = mfma4(wn[e], bits_f32(s0[x][e][n]), dk[n]);
-          dk[n] = mfma4(uv[e], bits_f32(s1[x][e][n]), dk[n]);
+          f32x4& to = sizeof(TT) == 4 ? dk1[n] : dk[n];
+          to = mfma4(uv[e], bits_f32(s1[x][e][n]), to);
         }
+    }
+    if constexpr (sizeof(TT) == 4) {
+#pragma unroll
+      for (int n = 0; n < VC; ++n) dk[n] += dk1[n];
     }
 #pragma unroll
     for (int n = 0; n < VC; ++n) {
@@ -932,14 +975,24 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
   }
   if (!(sBad[0] | sBad[1] | sBad[2] | sBad[3])) {
     const f32x4 av = *(const f32x4*)((isq ? sM : sN) + li * LM + 4 * grp);
+    // the chunk's own steps; float32: four steps at a time, added as a tree (one chain through all of them would
+    // round the largest term again with every other)
+    constexpr int NC4 = sizeof(TT) == 4 ? 4 : 1;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int s = 4 * grp + e;
+    for (int n = 0; n < VC; ++n) {
+      f32x4 ck[NC4] = {}, cq[NC4] = {};
+      if constexpr (NC4 == 1) ck[0] = acc[n];
 #pragma unroll
-      for (int n = 0; n < VC; ++n) {
-        acc[n] = mfma4(av[e], sK[s * LD + j0 + n], acc[n]);
-        if (!isq) acc[n] = mfma4(sM[s * LM + li], sQ[s * LD + j0 + n], acc[n]);
+      for (int e = 0; e < 4; ++e) {
+        const int s = 4 * grp + e;
+        ck[e % NC4] = mfma4(av[e], sK[s * LD + j0 + n], ck[e % NC4]);
+        f32x4& to = NC4 == 1 ? ck[0] : cq[e % NC4];
+        if (!isq) to = mfma4(sM[s * LM + li], sQ[s * LD + j0 + n], to);
       }
+      if constexpr (NC4 == 1)
+        acc[n] = ck[0];
+      else
+        acc[n] += ((ck[0] + ck[1]) + (ck[2] + ck[3])) + ((cq[0] + cq[1]) + (cq[2] + cq[3]));
     }
   } else {  // a step outside a sum must not enter it even with 0
     for (int s = 0; s < CH; ++s)

@@ -85,21 +85,33 @@ template <int W> struct RowFrag<float, W> {
 
 // The chunk's Gram tile a b^T: register r of (li, grp) = a[step 4 r + grp] . b[step sigma(li)], the A
 // operand of block r in a sum over a's steps.
-template <int DP>
+template <bool DECAY, int DP>
 EDF_DEVICE f32x4 gram(const RowFrag<bf16, DP>& a, const RowFrag<bf16, DP>& b) {
   f32x4 c = {0, 0, 0, 0};
 #pragma unroll
   for (int kk = 0; kk < DP / 32; ++kk) c = mfma32k(a.f[kk], b.f[kk], c);
   return c;
 }
-template <int DP>
+// float32 with a decay: the tile's rounding is most of a call's error (the steps next to each other carry the
+// result, so it is not averaged over a long state), so it is summed in eight chains, added as a tree; without a decay
+// one chain is enough.  Error against float64 at 2 x 1500 x 4 x 64, decay per head: out 1.6e-7 with one chain, 0.9e-7
+// with eight (the per-step kernel 0.8e-7); the gram wave's additions cost 9% of a call.
+template <bool DECAY, int DP>
 EDF_DEVICE f32x4 gram(const RowFrag<float, DP>& a, const RowFrag<float, DP>& b) {
-  f32x4 c = {0, 0, 0, 0};
+  constexpr int N = DECAY ? 8 : 1;
+  f32x4 c[N] = {};
 #pragma unroll
   for (int jt = 0; jt < DP / 16; ++jt)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) c = mfma4(a.f[jt][e], b.f[jt][e], c);
-  return c;
+    for (int e = 0; e < 4; ++e) {
+      const int n = (4 * jt + e) % N;
+      c[n] = mfma4(a.f[jt][e], b.f[jt][e], c[n]);
+    }
+#pragma unroll
+  for (int n = N / 2; n > 0; n /= 2)
+#pragma unroll
+    for (int i = 0; i < n; ++i) c[i] += c[i + n];
+  return c[0];
 }
 
 // pa, pb: the [step][row] tiles of a[step] . S[row] and b[step] . S[row] over W columns (one split of
@@ -125,14 +137,16 @@ EDF_DEVICE void state_dots(const RowFrag<bf16, W>& a, const RowFrag<bf16, W>& b,
 template <int W>
 EDF_DEVICE void state_dots(const RowFrag<float, W>& a, const RowFrag<float, W>& b, const f32x4 (&S)[W / 16], f32x4& pa,
                            f32x4& pb) {
-  pa = pb = f32x4{0, 0, 0, 0};
+  f32x4 ca[4] = {}, cb[4] = {};
 #pragma unroll
   for (int jt = 0; jt < W / 16; ++jt)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      pa = mfma4(a.f[jt][e], S[jt][e], pa);
-      pb = mfma4(b.f[jt][e], S[jt][e], pb);
+      ca[e] = mfma4(a.f[jt][e], S[jt][e], ca[e]);
+      cb[e] = mfma4(b.f[jt][e], S[jt][e], cb[e]);
     }
+  pa = (ca[0] + ca[1]) + (ca[2] + ca[3]);
+  pb = (cb[0] + cb[1]) + (cb[2] + cb[3]);
 }
 
 template <int W>
@@ -148,12 +162,12 @@ EDF_DEVICE f32x4 state_dot(const RowFrag<bf16, W>& a, const f32x4 (&S)[W / 16]) 
 }
 template <int W>
 EDF_DEVICE f32x4 state_dot(const RowFrag<float, W>& a, const f32x4 (&S)[W / 16]) {
-  f32x4 c[2] = {};
+  f32x4 c[4] = {};
 #pragma unroll
   for (int jt = 0; jt < W / 16; ++jt)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) c[e & 1] = mfma4(a.f[jt][e], S[jt][e], c[e & 1]);
-  return c[0] + c[1];
+    for (int e = 0; e < 4; ++e) c[e] = mfma4(a.f[jt][e], S[jt][e], c[e]);
+  return (c[0] + c[1]) + (c[2] + c[3]);
 }
 
 // The A operands of S += u^T tile over W columns: for bf16 element r of f[jt] is step 4 r + grp, column
@@ -193,10 +207,13 @@ EDF_DEVICE void state_add(f32x4 (&S)[W / 16], const ColFrag<bf16, W>& k, f32x4 u
 }
 template <int W>
 EDF_DEVICE void state_add(f32x4 (&S)[W / 16], const ColFrag<float, W>& k, f32x4 u) {
+  f32x4 c[W / 16] = {};  // the chunk's steps summed by themselves: one rounding of S per chunk
 #pragma unroll
   for (int r = 0; r < 4; ++r)
 #pragma unroll
-    for (int jt = 0; jt < W / 16; ++jt) S[jt] = mfma4(k.f[jt][r], u[r], S[jt]);
+    for (int jt = 0; jt < W / 16; ++jt) c[jt] = mfma4(k.f[jt][r], u[r], c[jt]);
+#pragma unroll
+  for (int jt = 0; jt < W / 16; ++jt) S[jt] += c[jt];
 }
 
 // S[row][column] += sum over the chunk's steps of x[step][row] q[step][column] - w[step][row] k[step][column],
@@ -216,14 +233,32 @@ EDF_DEVICE void state_add2(f32x4 (&S)[W / 16], const ColFrag<bf16, W>& q, const 
 template <int W>
 EDF_DEVICE void state_add2(f32x4 (&S)[W / 16], const ColFrag<float, W>& q, const unsigned (&x)[4],
                            const ColFrag<float, W>& k, f32x4 w) {
+  f32x4 c[W / 16] = {};
 #pragma unroll
   for (int r = 0; r < 4; ++r)
 #pragma unroll
-    for (int jt = 0; jt < W / 16; ++jt) S[jt] = mfma4(q.f[jt][r], bits_f32(x[r]), S[jt]);
+    for (int jt = 0; jt < W / 16; ++jt) {
+      c[jt] = mfma4(q.f[jt][r], bits_f32(x[r]), c[jt]);
+      c[jt] = mfma4(k.f[jt][r], -w[r], c[jt]);
+    }
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
+  for (int jt = 0; jt < W / 16; ++jt) S[jt] += c[jt];
+}
+
+// acc plus the sum over the 16 steps of tile[step][.] x[step][row].  APART (float32): the four blocks side by side and
+// acc last, which rounds at the size of acc once, not 16 times.
+template <bool APART>
+EDF_DEVICE f32x4 tile_dot(f32x4 tile, f32x4 x, f32x4 acc) {
+  if constexpr (APART) {
+    f32x4 c[4];
 #pragma unroll
-    for (int jt = 0; jt < W / 16; ++jt) S[jt] = mfma4(k.f[jt][r], -w[r], S[jt]);
+    for (int r = 0; r < 4; ++r) c[r] = mfma4(tile[r], x[r], f32x4{0, 0, 0, 0});
+    return acc + ((c[0] + c[1]) + (c[2] + c[3]));
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc = mfma4(tile[r], x[r], acc);
+    return acc;
+  }
 }
 
 // Value of each of the four groups, in every lane of the same li.  The swaps are not volatile (unlike
