@@ -769,8 +769,9 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
       s0[jt] = __builtin_amdgcn_raw_buffer_load_b128(rS0, at, blk, 0);
       s1[jt] = __builtin_amdgcn_raw_buffer_load_b128(rS1, at, blk, 0);
     }
-    // float32: several chains, added as a tree (four at 128 columns spill: 768 -> 864 us, KDA 8x777x8x128)
-    constexpr int NA = sizeof(TT) == 4 ? (DP == 128 ? 2 : 4) : 1;
+    // float32: several chains, added as a tree (four at 128 columns spill: 768 -> 864 us, KDA 8x777x8x128; at 32 they
+    // cost the occupancy)
+    constexpr int NA = sizeof(TT) == 4 ? (DP == 64 ? 4 : 2) : 1;
     f32x4 pk[NA] = {}, pq[NA] = {}, ek[NA] = {};
     float zs[NA] = {};
 #pragma unroll
@@ -804,7 +805,7 @@ __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayAr
     }
   }
   if (w >= 2) {  // G(t, s) = k_t . k_s, H(t, s) = q_t . k_s
-    constexpr int NG = sizeof(TT) == 4 ? 8 : 1;  // chains, as in gram
+    constexpr int NG = sizeof(TT) == 4 ? (DP == 32 ? 4 : 8) : 1;  // chains, as in gram
     f32x4 acc[NG] = {};
     const float* A = w == 2 ? sK : sQ;
 #pragma unroll

@@ -93,12 +93,12 @@ EDF_DEVICE f32x4 gram(const RowFrag<bf16, DP>& a, const RowFrag<bf16, DP>& b) {
   return c;
 }
 // float32 with a decay: the tile's rounding is most of a call's error (the steps next to each other carry the
-// result, so it is not averaged over a long state), so it is summed in eight chains, added as a tree; without a decay
-// one chain is enough.  Error against float64 at 2 x 1500 x 4 x 64, decay per head: out 1.6e-7 with one chain, 0.9e-7
+// result, so it is not averaged over a long state), so it is summed in eight chains (32 columns: four), added as a
+// tree; without a decay one chain is enough.  Error against float64 at 2 x 1500 x 4 x 64, decay per head: out 1.6e-7 with one chain, 0.9e-7
 // with eight (the per-step kernel 0.8e-7); the gram wave's additions cost 9% of a call.
 template <bool DECAY, int DP>
 EDF_DEVICE f32x4 gram(const RowFrag<float, DP>& a, const RowFrag<float, DP>& b) {
-  constexpr int N = DECAY ? 8 : 1;
+  constexpr int N = DECAY ? (DP == 32 ? 4 : 8) : 1;
   f32x4 c[N] = {};
 #pragma unroll
   for (int jt = 0; jt < DP / 16; ++jt)
