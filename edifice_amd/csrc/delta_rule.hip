@@ -1,9 +1,11 @@
 // C-ABI entry points of the delta rule (DeltaNet / GatedDeltaNet), forward and backward.
 // Dispatch: the chunked MFMA kernels (delta_rule_chunk.hip) take bf16, per-head beta,
 // head_dim 64 .. 128 (a multiple of 8; zero-padded to 128 inside), seq >= 64 (forward and
-// backward); every other case takes the row scans (delta_rule_row.hip, delta_rule_row_bwd.hip), the
-// exact per-step kernels (delta_rule_seq.hip) only batch rows of 2 GiB and more.
+// backward); every other case takes the row scans (delta_rule_row.hip, delta_rule_row_bwd.hip) or, by
+// row_path() below, the exact per-step kernels (delta_rule_seq.hip).
 #include "edf_abi.hpp"
+
+#include <algorithm>
 
 namespace edf {
 size_t dr_seq_backward_workspace_bytes(int batch, int heads, int seq, int d);
@@ -16,6 +18,9 @@ int dr_seq_backward_run(void* stream, const void* q, const void* k, const void* 
                         void* dalpha, void* workspace, int batch, int seq, int heads, int d, int dtype,
                         int beta_per_head, int alpha_per_row, const float* context);
 bool dr_row_takes(int batch, int heads, int seq, int d);
+int dr_row_run(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
+               void* out, int batch, int seq, int heads, int d, int dtype, int beta_per_head, int alpha_per_row,
+               float* ckpt, float* err, int cw);
 size_t dr_row_context_bytes(int batch, int heads, int seq, int d, bool decay);
 int dr_row_record_run(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
                       void* out, int batch, int seq, int heads, int d, int dtype, int beta_per_head,
@@ -49,24 +54,66 @@ int check_dr(int batch, int seq, int heads, int d, int dtype, int beta_mode) {
   return EDF_OK;
 }
 
-// The record of a forward and the workspace of a backward off the chunked path: the row scans' (the
-// queries of the delta rule do not know whether a decay is given: the larger need), the per-step
-// kernels' for batch rows of 2 GiB and more.
-size_t unchunked_context_bytes(int batch, int heads, int seq, int d) {
-  if (!dr_row_takes(batch, heads, seq, d)) return dr_seq_context_bytes(batch, heads, seq, d);
-  return dr_row_context_bytes(batch, heads, seq, d, true);
+// Off the chunked path: the row scans, or the per-step kernels where they are the faster ones with the backward.  The
+// row scans cost whole chunks of 16 steps, states at least 32 wide and a workgroup per 16 rows and per 16 (64) steps
+// in the gradients; the per-step kernels a chain of steps.  bfloat16, us with gradients, per-step / row scans:
+//                                      DeltaNet     GatedDeltaNet
+//   one chunk     d 64,  8 heads x 16    17 / 22      18 / 23
+//                 d 64,  512 x 16        51 / 44      56 / 39
+//                 d 128, 128 x 16        53 / 34      55 / 39
+//   narrow        d 16,  8 x 48, 64      22 / 25, 27 / 27    25 / 25, 31 / 27
+//                 d 16,  128 x 128       48 / 36      58 / 55
+//                 d 16,  512 x 256      109 / 118    125 / 208
+//                 d 32,  8 x 32, 48      20 / 23, 27 / 24    22 / 24, 29 / 25
+//                 d 32,  512 x 64, 128   60 / 37, 106 / 66   66 / 71, 120 / 119
+// float32's row scans take up to a third longer than bfloat16's with a decay (their sums are split), so their lines
+// lie further out.  Batch rows of (seq + 96) H d 4 >= 2 GiB, of either type, are past the row scans' byte offsets.
+bool row_path(int batch, int heads, int seq, int d, int dtype, bool decay) {
+  if (!dr_row_takes(batch, heads, seq, d)) return false;
+  const long bh = (long)batch * heads;
+  const bool f32 = dtype != EDF_BF16;
+  if (d <= 16) return seq >= 64 && bh < (f32 && decay ? 128 : 256);
+  if (seq <= 16) return f32 ? d > 64 && bh >= 128 && !decay : (d > 32 && bh >= 512) || (d > 64 && bh >= 128);
+  if (d <= 32) return bh < 256 ? seq >= 48 : !decay || (!f32 && seq >= 128);
+  return !(f32 && decay && bh < 128 && seq <= 32);
 }
-size_t unchunked_backward_bytes(int batch, int heads, int seq, int d) {
-  if (!dr_row_takes(batch, heads, seq, d)) return dr_seq_backward_workspace_bytes(batch, heads, seq, d);
-  return dr_row_backward_workspace_bytes(batch, heads, seq, d, true);
+// A forward that keeps no record.  On a full grid of short sequences float32 row scans, which hold two or three
+// workgroups per CU, are the slower ones although they win with the backward: DeltaNet 512 heads of d 128, 32 steps
+// 54 us per-step, 72 row scans; GatedDeltaNet 58 and 88, at 128 steps 232 and 254.
+bool row_forward(int batch, int heads, int seq, int d, int dtype, bool decay) {
+  if (!row_path(batch, heads, seq, d, dtype, decay)) return false;
+  return !(dtype != EDF_BF16 && (long)batch * heads * ((d + 15) / 16) >= 768 && seq < (decay ? 256 : 64));
+}
+
+// The record of a forward and the workspace of a backward.
+size_t unchunked_context_bytes(int batch, int heads, int seq, int d, int dtype, bool decay) {
+  return row_path(batch, heads, seq, d, dtype, decay) ? dr_row_context_bytes(batch, heads, seq, d, decay)
+                                               : dr_seq_context_bytes(batch, heads, seq, d);
+}
+size_t unchunked_backward_bytes(int batch, int heads, int seq, int d, int dtype, bool decay) {
+  return row_path(batch, heads, seq, d, dtype, decay) ? dr_row_backward_workspace_bytes(batch, heads, seq, d, decay)
+                                               : dr_seq_backward_workspace_bytes(batch, heads, seq, d);
+}
+// What serves a call with a decay and one without: the queries that do not say which.
+size_t any_context_bytes(int batch, int heads, int seq, int d, int dtype) {
+  return std::max(unchunked_context_bytes(batch, heads, seq, d, dtype, false),
+                  unchunked_context_bytes(batch, heads, seq, d, dtype, true));
+}
+size_t any_backward_bytes(int batch, int heads, int seq, int d, int dtype) {
+  return std::max(unchunked_backward_bytes(batch, heads, seq, d, dtype, false),
+                  unchunked_backward_bytes(batch, heads, seq, d, dtype, true));
 }
 
 int unchunked_fwd(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
                   void* out, int batch, int seq, int heads, int d, int dtype, int beta_per_head, int alpha_per_row,
                   void* context) {
-  if (context != nullptr && dr_row_takes(batch, heads, seq, d))
+  const bool decay = alpha != nullptr;
+  if (context != nullptr && row_path(batch, heads, seq, d, dtype, decay))
     return dr_row_record_run(stream, q, k, v, beta, alpha, out, batch, seq, heads, d, dtype, beta_per_head,
                              alpha_per_row, context);
+  if (context == nullptr && row_forward(batch, heads, seq, d, dtype, decay))
+    return dr_row_run(stream, q, k, v, beta, alpha, out, batch, seq, heads, d, dtype, beta_per_head, alpha_per_row,
+                      nullptr, nullptr, 0);
   return dr_seq_run(stream, q, k, v, beta, alpha, out, batch, seq, heads, d, dtype, beta_per_head, alpha_per_row,
                     (float*)context);
 }
@@ -76,7 +123,7 @@ int unchunked_bwd(void* stream, const void* q, const void* k, const void* v, con
                   const void* grad_out, void* dq, void* dk, void* dv, void* dbeta, void* dalpha, void* workspace,
                   int batch, int seq, int heads, int d, int dtype, int beta_per_head, int alpha_per_row,
                   const void* context) {
-  if (dr_row_takes(batch, heads, seq, d))
+  if (row_path(batch, heads, seq, d, dtype, alpha != nullptr))
     return dr_row_backward_run(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch,
                                seq, heads, d, dtype, beta_per_head, alpha_per_row, context);
   return dr_seq_backward_run(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch, seq,
@@ -98,7 +145,7 @@ int fwd(void* stream, const void* q, const void* k, const void* v, const void* b
   }
   // a workspace of edf_delta_rule_forward_context_bytes() (optional) also receives what the saved
   // backward reads
-  const bool keep = workspace && ws_bytes >= unchunked_context_bytes(batch, heads, seq, d);
+  const bool keep = workspace && ws_bytes >= unchunked_context_bytes(batch, heads, seq, d, dtype, alpha != nullptr);
   return unchunked_fwd(stream, q, k, v, beta, alpha, out, batch, seq, heads, d, dtype, per_head, 0,
                        keep ? workspace : nullptr);
 }
@@ -117,7 +164,7 @@ int bwd(void* stream, const void* q, const void* k, const void* v, const void* b
     return dr_chunk_backward_run(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch,
                                  seq, heads, d);
   }
-  const size_t need = unchunked_backward_bytes(batch, heads, seq, d);
+  const size_t need = unchunked_backward_bytes(batch, heads, seq, d, dtype, alpha != nullptr);
   EDF_REQUIRE(workspace && ws_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
   return unchunked_bwd(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch, seq, heads,
                        d, dtype, per_head, 0, nullptr);
@@ -143,9 +190,9 @@ int bwd_saved(void* stream, const void* q, const void* k, const void* v, const v
                                        workspace, batch, seq, heads, d);
   }
   // the forward's record when its workspace held one, else the backward recomputes it
-  const size_t need = unchunked_backward_bytes(batch, heads, seq, d);
+  const size_t need = unchunked_backward_bytes(batch, heads, seq, d, dtype, alpha != nullptr);
   EDF_REQUIRE(workspace && ws_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
-  const bool saved = fwd_ws && fwd_ws_bytes >= unchunked_context_bytes(batch, heads, seq, d);
+  const bool saved = fwd_ws && fwd_ws_bytes >= unchunked_context_bytes(batch, heads, seq, d, dtype, alpha != nullptr);
   return unchunked_bwd(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch, seq, heads,
                        d, dtype, per_head, 0, saved ? fwd_ws : nullptr);
 }
@@ -159,7 +206,7 @@ size_t edf_delta_rule_saved_backward_workspace_bytes(int batch, int seq_len, int
   if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
   if (edf::dr_chunk_eligible(seq_len, head_dim, dtype, beta_mode == EDF_BETA_PER_HEAD))
     return edf::dr_chunk_saved_backward_workspace_bytes(batch, seq_len, num_heads, head_dim);
-  return edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim);
+  return edf::any_backward_bytes(batch, num_heads, seq_len, head_dim, dtype);
 }
 
 int edf_fused_delta_rule_scan_backward_saved(void* stream, const void* q, const void* k, const void* v,
@@ -179,7 +226,7 @@ size_t edf_delta_rule_forward_context_bytes(int batch, int seq_len, int num_head
   if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0 || head_dim > 128) return 0;
   if (edf::dr_chunk_eligible(seq_len, head_dim, dtype, beta_mode == EDF_BETA_PER_HEAD))
     return edf::dr_chunk_workspace_bytes(batch, seq_len, num_heads, head_dim);
-  return edf::unchunked_context_bytes(batch, num_heads, seq_len, head_dim);
+  return edf::any_context_bytes(batch, num_heads, seq_len, head_dim, dtype);
 }
 
 size_t edf_delta_rule_workspace_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype,
@@ -195,7 +242,7 @@ size_t edf_delta_rule_backward_workspace_bytes(int batch, int seq_len, int num_h
   if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
   if (edf::dr_chunk_eligible(seq_len, head_dim, dtype, beta_mode == EDF_BETA_PER_HEAD))
     return edf::dr_chunk_backward_workspace_bytes(batch, seq_len, num_heads, head_dim);
-  return edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim);
+  return edf::any_backward_bytes(batch, num_heads, seq_len, head_dim, dtype);
 }
 
 int edf_fused_delta_net_scan(void* stream, const void* q, const void* k, const void* v, const void* beta, void* out,
@@ -237,9 +284,8 @@ int edf_fused_gated_delta_net_scan_backward(void* stream, const void* q, const v
 
 // KDA: per-row log-space decay, per-head beta; never the chunked kernels (which take one decay per head).
 size_t edf_kda_scan_backward_workspace_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype) {
-  (void)dtype;
   if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
-  return edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim);
+  return edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim, dtype, true);
 }
 
 int edf_fused_kda_scan(void* stream, const void* q, const void* k, const void* v, const void* alpha,
@@ -261,16 +307,15 @@ int edf_fused_kda_scan_backward(void* stream, const void* q, const void* k, cons
   if (rc) return rc;
   EDF_REQUIRE(q && k && v && alpha && beta && grad_out && grad_q && grad_k && grad_v && grad_alpha && grad_beta,
               EDF_ERR_INVALID_ARG, "null tensor pointer");
-  const size_t need = edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim);
+  const size_t need = edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim, dtype, true);
   EDF_REQUIRE(workspace && workspace_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
   return edf::unchunked_bwd(stream, q, k, v, beta, alpha, grad_out, grad_q, grad_k, grad_v, grad_beta,
                                   grad_alpha, workspace, batch, seq_len, num_heads, head_dim, dtype, 1, 1, nullptr);
 }
 
 size_t edf_kda_scan_context_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype) {
-  (void)dtype;
   if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0 || head_dim > 128) return 0;
-  return edf::unchunked_context_bytes(batch, num_heads, seq_len, head_dim);
+  return edf::unchunked_context_bytes(batch, num_heads, seq_len, head_dim, dtype, true);
 }
 
 int edf_fused_kda_scan_with_context(void* stream, const void* q, const void* k, const void* v, const void* alpha,
@@ -279,7 +324,7 @@ int edf_fused_kda_scan_with_context(void* stream, const void* q, const void* k, 
   int rc = edf::check_dr(batch, seq_len, num_heads, head_dim, dtype, EDF_BETA_PER_HEAD);
   if (rc) return rc;
   EDF_REQUIRE(q && k && v && alpha && beta && out, EDF_ERR_INVALID_ARG, "null tensor pointer");
-  const size_t need = edf::unchunked_context_bytes(batch, num_heads, seq_len, head_dim);
+  const size_t need = edf::unchunked_context_bytes(batch, num_heads, seq_len, head_dim, dtype, true);
   EDF_REQUIRE(context && context_bytes >= need, EDF_ERR_WORKSPACE, "context too small: need %zu bytes", need);
   return edf::unchunked_fwd(stream, q, k, v, beta, alpha, out, batch, seq_len, num_heads, head_dim, dtype, 1, 1,
                          context);
@@ -294,10 +339,10 @@ int edf_fused_kda_scan_backward_saved(void* stream, const void* q, const void* k
   if (rc) return rc;
   EDF_REQUIRE(q && k && v && alpha && beta && grad_out && grad_q && grad_k && grad_v && grad_alpha && grad_beta,
               EDF_ERR_INVALID_ARG, "null tensor pointer");
-  const size_t needc = edf::unchunked_context_bytes(batch, num_heads, seq_len, head_dim);
+  const size_t needc = edf::unchunked_context_bytes(batch, num_heads, seq_len, head_dim, dtype, true);
   EDF_REQUIRE(context && context_bytes >= needc, EDF_ERR_WORKSPACE,
               "context too small: need the %zu bytes the forward filled", needc);
-  const size_t need = edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim);
+  const size_t need = edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim, dtype, true);
   EDF_REQUIRE(workspace && workspace_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
   return edf::unchunked_bwd(stream, q, k, v, beta, alpha, grad_out, grad_q, grad_k, grad_v, grad_beta,
                                   grad_alpha, workspace, batch, seq_len, num_heads, head_dim, dtype, 1, 1,

@@ -12,8 +12,10 @@
 //   dv = beta ds_k, dbeta = err ds_k, dk = dS_tot^T (beta err) - S_g^T (beta ds_k),
 //   dalpha = sum(dS_to_decayed * S_prev), dS_prev = alpha dS_to_decayed).
 //
-// The exact per-step path: it serves batch rows of 2 GiB and more; smaller ones run 16 steps at a time on
-// the matrix cores (delta_rule_row.hip, delta_rule_row_bwd.hip).
+// The exact per-step path: per-element beta, float32 I/O, any head_dim <= 128.  It serves short
+// sequences, narrow heads in number and batch rows past the row scans' byte offsets (the rule:
+// delta_rule.hip); the rest runs 16 steps at a time on the matrix cores (delta_rule_row.hip,
+// delta_rule_row_bwd.hip).
 //
 // Rows of S evolve independently given k, q, alpha and the row's beta, so a workgroup
 // owns one block of RB = 16 rows of one (batch, head) state (DP / 16 workgroups per
@@ -28,10 +30,6 @@
 #include "edf_common.hpp"
 
 namespace edf {
-bool dr_row_takes(int batch, int heads, int seq, int d);
-int dr_row_run(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
-               void* out, int batch, int seq, int heads, int d, int dtype, int beta_per_head, int alpha_per_row,
-               float* ckpt, float* err, int cw);
 namespace {
 
 constexpr int CK = 16;  // steps per staged chunk / checkpoint interval
@@ -126,7 +124,11 @@ EDF_DEVICE void fwd_step(float (&S)[DP / 16], const Stage<DP>& sm, int tt, int t
   for (int c = 0; c < NC; ++c) S[c] = fmaf(e, sm.k[tt][tc + 16 * c], at * S[c]);
 }
 
-// OUTM: 0 no output (p.out null), 1 output stored by the row's lane 0.
+// OUTM: 0 no output (p.out null), 1 output stored by the row's lane 0 (tensors of 2 GiB per
+// batch row and more), 2 output through a buffer resource over the batch row, every lane
+// storing (lanes other than the row's lane 0, rows past d and steps past T at an offset the
+// hardware drops): no branch in the unrolled steps, which a per-step branch splits into
+// basic blocks, each waiting for its own LDS reads.
 template <typename TT, int DP, bool DECAY, int OUTM>
 __global__ __launch_bounds__(256) void dr_seq_fwd_kernel(const DRArgs p) {
   constexpr int NC = DP / 16;
@@ -136,7 +138,15 @@ __global__ __launch_bounds__(256) void dr_seq_fwd_kernel(const DRArgs p) {
   const int rb = blockIdx.y, i = rb * RB + tr;
   const int b = (int)(bh / p.H), h = (int)(bh % p.H);
   const int nch = (p.T + CK - 1) / CK;
+  const long rowel = (long)p.T * p.H * p.d;  // output elements of one batch row
+  const rsrc_t r_out = make_rsrc(OUTM == 2 ? (const TT*)p.out + (long)b * rowel : (const TT*)p.k,
+                                 OUTM == 2 ? (unsigned)(rowel * sizeof(TT)) : 0u);
   const bool orow = tc == 0 && i < p.d;
+  // OUTM 2: the lane's byte offset at step 0, out of bounds for lanes that store nothing; a
+  // step past T lands past the batch row (the host keeps (T + CK) H d elements under 2 GiB,
+  // so no offset wraps)
+  const unsigned obase = orow ? (unsigned)(((long)h * p.d + i) * sizeof(TT)) : OOB_OFF;
+  const unsigned ostep = (unsigned)((long)p.H * p.d * sizeof(TT));
   float S[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) S[c] = 0.0f;
@@ -159,7 +169,11 @@ __global__ __launch_bounds__(256) void dr_seq_fwd_kernel(const DRArgs p) {
 #pragma unroll
         for (int c = 0; c < NC; ++c) o = fmaf(S[c], sm.q[tt][tc + 16 * c], o);
         o = row16_sum(o);
-        if (orow && t0 + tt < p.T) st((TT*)p.out, (((long)b * p.T + t0 + tt) * p.H + h) * p.d + i, o);
+        if constexpr (OUTM == 2) {
+          bstore<TT>(r_out, obase + (unsigned)(t0 + tt) * ostep, o);
+        } else if (orow && t0 + tt < p.T) {
+          st((TT*)p.out, (((long)b * p.T + t0 + tt) * p.H + h) * p.d + i, o);
+        }
       }
     }
     if (p.ckpt != nullptr) {
@@ -383,6 +397,8 @@ template <typename TT, int DP, bool DECAY>
 void fwd_out(hipStream_t s, dim3 grid, const DRArgs& a) {
   if (a.out == nullptr)
     dr_seq_fwd_kernel<TT, DP, DECAY, 0><<<grid, 256, 0, s>>>(a);
+  else if ((long)(a.T + CK) * a.H * a.d * (long)sizeof(TT) < (1L << 31))
+    dr_seq_fwd_kernel<TT, DP, DECAY, 2><<<grid, 256, 0, s>>>(a);
   else
     dr_seq_fwd_kernel<TT, DP, DECAY, 1><<<grid, 256, 0, s>>>(a);
 }
@@ -466,9 +482,6 @@ size_t dr_seq_context_bytes(int batch, int heads, int seq, int d) {
 int dr_seq_run(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
                void* out, int batch, int seq, int heads, int d, int dtype, int beta_per_head, int alpha_per_row,
                float* context) {
-  if (dr_row_takes(batch, heads, seq, d))  // (a call that keeps states, and that these take, does not come here)
-    return dr_row_run(stream, q, k, v, beta, alpha, out, batch, seq, heads, d, dtype, beta_per_head, alpha_per_row,
-                      nullptr, nullptr, 0);
   DRArgs a{};
   a.q = q; a.k = k; a.v = v; a.beta = beta; a.alpha = alpha; a.out = out;
   a.ckpt = context;  // also store the checkpoints (one pass writes both)
@@ -499,20 +512,26 @@ int dr_seq_backward_run(void* stream, const void* q, const void* k, const void* 
   const long nbth = (long)bh * seq;
   const int nrb = pad_dim(d) / RB;
   hipStream_t s = as_stream(stream);
+  // forward pass that only writes the checkpoints
+  DRArgs f = a;
+  f.out = nullptr;
   const long n4 = d % 4 == 0 ? 2 * nbth * d / 4 : 0;  // vector items of the reduction (see the kernel)
   const long nred = 2 * nbth * d + 2 * nbth - 3 * n4;
   const unsigned gred = (unsigned)((nred + 255) / 256);
   int rc;
-  if (!context) {  // the forward's stored checkpoints, or a pass that writes only them
-    rc = dr_seq_run(stream, q, k, v, beta, alpha, nullptr, batch, seq, heads, d, dtype, beta_per_head, alpha_per_row,
-                    a.ckpt);
-    if (rc) return rc;
-  }
   if (dtype == EDF_BF16) {
+    if (!context) {  // the forward's stored checkpoints, or a pass that writes only them
+      rc = launch_seq<bf16>(s, f, false, bh);
+      if (rc) return rc;
+    }
     rc = launch_seq<bf16>(s, a, true, bh);
     if (rc) return rc;
     dr_seq_reduce_kernel<bf16><<<gred, 256, 0, s>>>(a, nbth, nrb);
   } else {
+    if (!context) {
+      rc = launch_seq<float>(s, f, false, bh);
+      if (rc) return rc;
+    }
     rc = launch_seq<float>(s, a, true, bh);
     if (rc) return rc;
     dr_seq_reduce_kernel<float><<<gred, 256, 0, s>>>(a, nbth, nrb);

@@ -478,7 +478,8 @@ int edf_fused_laser_attention_backward(void* stream, const void* q, const void* 
  *   forward and backward, and then requires the workspace the *_workspace_bytes queries
  *   return (EDF_ERR_WORKSPACE when it is missing or short; the forward query returns 0
  *   for every other case); everything else runs row scans, 16 steps at a time in
- *   float32, or the per-step kernels where a batch row has 2 GiB and more.
+ *   float32, or the exact per-step kernels: short sequences, many narrow heads, and batch
+ *   rows with (seq_len + 96) * num_heads * head_dim * 4 bytes past 2 GiB.
  * ------------------------------------------------------------------------ */
 enum { EDF_BETA_PER_ELEMENT = 0, EDF_BETA_PER_HEAD = 1 };
 

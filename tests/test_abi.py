@@ -265,3 +265,27 @@ def test_selective_scan_plan_by_grid(monkeypatch, batch, dim, n, plan):
         size[p] = nat.query("edf_selective_scan_backward_workspace_bytes", batch, 64, dim, n, 0, 1)
     assert size[""] == size[plan]
     assert dim == 16 or size["narrow"] != size["wide"]
+
+
+@pytest.mark.parametrize("batch,seq,heads,d,dtype,rows", [
+    (1, 16, 8, 64, 1, False), (64, 16, 8, 64, 1, True), (64, 16, 8, 64, 0, False), (16, 16, 8, 128, 1, True),
+    (1, 17, 8, 64, 1, True), (1, 17, 8, 64, 0, False), (1, 33, 8, 64, 0, True), (1, 63, 8, 16, 1, False),
+    (1, 64, 8, 16, 1, True), (16, 64, 8, 16, 0, False), (32, 512, 8, 16, 1, False), (1, 47, 8, 32, 1, False),
+    (1, 48, 8, 32, 1, True), (32, 127, 8, 32, 1, False), (32, 128, 8, 32, 1, True), (32, 1024, 8, 32, 0, False),
+    (4, 1000, 8, 128, 1, True), (1, 32768, 128, 128, 1, False)])
+def test_delta_rule_path_by_size(batch, seq, heads, d, dtype, rows):
+    """The row scans' record (states every 16 steps at a width of 32, 64 or 128, and err) or the per-step kernels'
+    (states alone, from a width of 16) shows which of them takes a call with a decay; narrow, short and very large
+    calls stay per-step."""
+    from edifice_amd import _native as nat
+
+    def up(v):
+        return (v + 255) // 256 * 256
+
+    bh, n = batch * heads, (seq + 15) // 16
+    w = 32 if d <= 32 else 64 if d <= 64 else 128
+    ws = 16 if d <= 16 else w
+    got = nat.query("edf_kda_scan_context_bytes", batch, seq, heads, d, dtype)
+    assert got == (up(bh * n * w * w * 4) + up(bh * seq * d * 4) if rows else up(bh * n * ws * ws * 4))
+    # a query that does not say whether there is a decay serves both
+    assert nat.query("edf_delta_rule_forward_context_bytes", batch, seq, heads, d, dtype, 0) >= got

@@ -116,3 +116,50 @@ def test_float32_error(kind, d, rng):
     print({n: f"{e:.2e}" for n, e in err.items()}, flush=True)
     bound = FLOAT32_ERROR[kind]
     assert err["out"] <= bound[0] and max(err.values()) <= bound[1], err
+
+
+@pytest.mark.parametrize("kind", ["element", "gated", "kda"])
+@pytest.mark.parametrize("shape", [(32, 40, 8, 32), (32, 70, 8, 16), (2, 47, 2, 24), (1, 63, 4, 8), (1, 16, 2, 128),
+                                   (3, 9, 2, 64), (32, 96, 8, 24)])
+def test_per_step_kernels(shape, kind, rng):
+    """The sizes that stay with the per-step kernels (short sequences, narrow heads in number)."""
+    announce("per_step", shape=shape, kind=kind)
+    a = _inputs(rng, *shape, kind)
+    do = rng.normal(size=shape)
+    t = {n: to_dev(x, torch.float32).requires_grad_() for n, x in a.items()}
+    out = _call(kind, t)
+    grads = dict(zip(t, torch.autograd.grad(out, list(t.values()), to_dev(do, torch.float32))))
+    r = {n: rounded(x, torch.float32) for n, x in a.items()}
+    want = _oracle(kind, r, rounded(do, torch.float32))
+    for name, g, w in [("o", out, _oracle(kind, r))] + [("d" + n, g, want["d" + n]) for n, g in grads.items()]:
+        err = np.linalg.norm(host(g) - w) / np.linalg.norm(w)
+        assert err <= REL[torch.float32], f"{name}: {err:.2e}"
+
+
+def test_batch_rows_past_2_gib(rng):
+    """A batch row of more than 2 GiB (past the buffer resources of the row scans and of the per-step kernels'
+    branch-free stores): its first and last heads are those of a call with these heads alone."""
+    T, H, d, few = 4100, 16384, 16, 4
+    announce("rows_past_2_gib", T=T, H=H, d=d)
+    if torch.cuda.mem_get_info()[0] < 80 << 30:
+        pytest.skip("needs 80 GB of device memory")
+    gen = torch.Generator(device="cuda").manual_seed(7)
+
+    def n(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen, dtype=torch.bfloat16)
+
+    t = [n(1, T, H, d), n(1, T, H, d).mul_(0.25), n(1, T, H, d), n(1, T, H, d).sigmoid_(), n(1, T, H).sigmoid_()]
+    do = n(1, T, H, d)
+    assert t[0].numel() * 2 > 2 ** 31
+    from edifice_amd import fused_scan as fs
+
+    def run(sl):
+        ts = [x[:, :, sl].contiguous().requires_grad_() for x in t]
+        out = fs.gated_delta_net_scan(*ts)
+        return [out.detach(), *torch.autograd.grad(out, ts, do[:, :, sl].contiguous())]
+
+    whole = run(slice(None))
+    for sl in (slice(0, few), slice(H - few, H)):
+        for i, (g, w) in enumerate(zip(whole, run(sl))):
+            err = (g[:, :, sl].double() - w.double()).norm() / w.double().norm()
+            assert err <= 2.0 ** -7, (i, float(err))  # two bfloat16 roundings of one value
