@@ -17,7 +17,7 @@
 //     (keys permuted consistently in the V^T reads), so P never goes through LDS;
 //   * causal: key tiles above the diagonal are skipped, only diagonal tiles are
 //     masked, and query blocks are issued heaviest-first.
-// float32 and the other head widths: flash_attn_f32.hip (to 128), here one wave per query (wider).
+// float32 and the other head widths: flash_attn_f32.hip (to 128), here one wave per query (wider, or a few steps).
 #include "edf_abi.hpp"
 #include "edf_common.hpp"
 #include "edf_mfma.hpp"
@@ -25,7 +25,7 @@
 #include <type_traits>
 
 namespace edf {
-bool fa32_takes(int batch_heads, int T, int HD, int dtype);
+bool fa32_takes(int batch_heads, int T, int HD, int dtype, bool fox);
 int fa32_forward(hipStream_t s, const void* q, const void* k, const void* v, const void* cs, void* out, float* lse,
                  int BH, int T, int HD, int causal, int dtype);
 namespace {
@@ -534,7 +534,8 @@ __global__ __launch_bounds__(256, 2) void fa_fwd128_kernel(const bf16* __restric
   if (myq < T && g == 0 && LSE != nullptr) LSE[bh * T + myq] = (m * scale_log2 + __log2f(lsum)) * LN2;
 }
 
-// Heads wider than 128: one wave per query row, lanes over head_dim (any dtype, head_dim <= 256).
+// Heads wider than 128 and the shortest sequences: one wave per query row, lanes over head_dim (any dtype, head_dim
+// <= 256).
 template <typename TT, int DPL>
 __global__ __launch_bounds__(256) void fa_fwd_wave_kernel(const TT* __restrict__ Q, const TT* __restrict__ K,
                                                           const TT* __restrict__ V, TT* __restrict__ O,
@@ -641,13 +642,15 @@ void launch_wave_fwd(hipStream_t s, const void* q, const void* k, const void* v,
                      int HD, int causal, float scale_log2, const void* cs, float sqd) {
   const long rows = (long)BH * T;
   const unsigned grid = (unsigned)((rows + 3) / 4);
-  fa_fwd_wave_kernel<TT, 4><<<grid, 256, 0, s>>>((const TT*)q, (const TT*)k, (const TT*)v, (TT*)o, lse, BH, T, HD,
-                                                 scale_log2, causal, (const TT*)cs, sqd);
+  auto kernel = HD <= 64 ? fa_fwd_wave_kernel<TT, 1> : HD <= 128 ? fa_fwd_wave_kernel<TT, 2> : fa_fwd_wave_kernel<TT, 4>;
+  kernel<<<grid, 256, 0, s>>>((const TT*)q, (const TT*)k, (const TT*)v, (TT*)o, lse, BH, T, HD, scale_log2, causal,
+                              (const TT*)cs, sqd);
 }
 
 // Flash attention (cs null) and FoX attention (causal).  bf16 at head_dim 32, 64 and 128 takes the
 // bf16 MFMA kernels; float32, and bf16 at the other widths up to 128, keep scores and probabilities
-// in float32 on the f32 MFMA (flash_attn_f32.hip); wider heads one wave per query row.
+// in float32 on the matrix cores (flash_attn_f32.hip); wider heads and the shortest sequences (fa32_takes) one wave
+// per query row.
 int fa_fwd_run(hipStream_t s, const void* q, const void* k, const void* v, const void* cs, void* out, float* lse,
                int BH, int T, int HD, int causal, int dtype) {
   const float scale_log2 = LOG2E / sqrtf((float)HD);
@@ -658,7 +661,7 @@ int fa_fwd_run(hipStream_t s, const void* q, const void* k, const void* v, const
     launch_mfma_fwd<64>(s, q, k, v, out, lse, BH, T, causal, scale_log2, cs, sqd);
   else if (dtype == EDF_BF16 && HD == 32)
     launch_mfma_fwd<32>(s, q, k, v, out, lse, BH, T, causal, scale_log2, cs, sqd);
-  else if (fa32_takes(BH, T, HD, dtype))
+  else if (fa32_takes(BH, T, HD, dtype, cs != nullptr))
     return fa32_forward(s, q, k, v, cs, out, lse, BH, T, HD, causal, dtype);
   else if (dtype == EDF_BF16)
     launch_wave_fwd<bf16>(s, q, k, v, out, lse, BH, T, HD, causal, scale_log2, cs, sqd);

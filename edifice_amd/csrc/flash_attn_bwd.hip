@@ -28,7 +28,7 @@
 #include <type_traits>
 
 namespace edf {
-bool fa32_takes(int batch_heads, int T, int HD, int dtype);
+bool fa32_takes(int batch_heads, int T, int HD, int dtype, bool fox);
 int fa32_backward(hipStream_t s, const void* q, const void* k, const void* v, const void* dout, const float* lse,
                   const float* dd, void* dq, void* dk, void* dv, const void* cs, float* dcsk, void* dcs, int BH, int T,
                   int HD, int causal, int dtype);
@@ -817,7 +817,7 @@ __global__ __launch_bounds__(256, 2) void fa_bwd_dq128_kernel(const bf16* __rest
   }
 }
 
-// ---- wave-per-row kernels (heads wider than 128) ------------------------
+// ---- wave-per-row kernels (heads wider than 128, and a few steps) -------
 template <typename TT, int DPL>
 __global__ __launch_bounds__(256) void fa_bwd_dq_wave_kernel(const TT* __restrict__ Q, const TT* __restrict__ K,
                                                              const TT* __restrict__ V, const TT* __restrict__ dO,
@@ -1015,10 +1015,14 @@ void launch_wave_bwd(hipStream_t s, const void* q, const void* k, const void* v,
   const unsigned grid = (unsigned)((rows + 3) / 4);
   const TT *Q = (const TT*)q, *K = (const TT*)k, *V = (const TT*)v, *G = (const TT*)go, *CS = (const TT*)cs;
   // dK/dV first: with FoX the dQ kernel adds the key side of d cs that it writes
-  fa_bwd_dkdv_wave_kernel<TT, 4><<<grid, 256, 0, s>>>(Q, K, V, G, lse, Dd, (TT*)dk, (TT*)dv, BH, T, HD, scale_log2,
-                                                      scale, causal, CS, dcsk, sqd);
-  fa_bwd_dq_wave_kernel<TT, 4><<<grid, 256, 0, s>>>(Q, K, V, G, lse, Dd, (TT*)dq, BH, T, HD, scale_log2, scale,
-                                                    causal, CS, dcsk, (TT*)dcs, sqd);
+  auto dkdv = HD <= 64    ? fa_bwd_dkdv_wave_kernel<TT, 1>
+              : HD <= 128 ? fa_bwd_dkdv_wave_kernel<TT, 2>
+                          : fa_bwd_dkdv_wave_kernel<TT, 4>;
+  auto dqk = HD <= 64    ? fa_bwd_dq_wave_kernel<TT, 1>
+             : HD <= 128 ? fa_bwd_dq_wave_kernel<TT, 2>
+                         : fa_bwd_dq_wave_kernel<TT, 4>;
+  dkdv<<<grid, 256, 0, s>>>(Q, K, V, G, lse, Dd, (TT*)dk, (TT*)dv, BH, T, HD, scale_log2, scale, causal, CS, dcsk, sqd);
+  dqk<<<grid, 256, 0, s>>>(Q, K, V, G, lse, Dd, (TT*)dq, BH, T, HD, scale_log2, scale, causal, CS, dcsk, (TT*)dcs, sqd);
 }
 
 // ---------------------------------------------------------------------------
@@ -1066,7 +1070,7 @@ int fa_bwd_run(hipStream_t s, const void* q, const void* k, const void* v, const
     else
       launch_mfma_bwd<32>(s, q, k, v, grad_out, lse, Dd, grad_q, grad_k, grad_v, BH, seq_len, causal, scale_log2,
                           scale);
-  } else if (fa32_takes(BH, seq_len, head_dim, dtype)) {
+  } else if (fa32_takes(BH, seq_len, head_dim, dtype, false)) {
     return fa32_backward(s, q, k, v, grad_out, lse, Dd, grad_q, grad_k, grad_v, nullptr, nullptr, nullptr, BH, seq_len,
                          head_dim, causal, dtype);
   } else if (dtype == EDF_BF16) {
@@ -1213,7 +1217,7 @@ int edf_fused_fox_attention_backward(void* stream, const void* q, const void* k,
     else
       launch_mfma_bwd<32>(s, q, k, v, grad_out, lse, Dd, grad_q, grad_k, grad_v, BH, seq_len, 1, scale_log2, scale,
                           cs, dcsk, grad_cs, sqd);
-  } else if (fa32_takes(BH, seq_len, head_dim, dtype)) {
+  } else if (fa32_takes(BH, seq_len, head_dim, dtype, true)) {
     return fa32_backward(s, q, k, v, grad_out, lse, Dd, grad_q, grad_k, grad_v, cs, dcsk, grad_cs, BH, seq_len,
                          head_dim, 1, dtype);
   } else if (dtype == EDF_BF16) {

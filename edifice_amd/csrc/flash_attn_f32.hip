@@ -781,8 +781,13 @@ void by_width(hipStream_t s, const Args& a, unsigned grid, int causal, bool bwd)
 
 }  // namespace
 
-// Whether these kernels take a head: its rows addressed by 31-bit byte offsets.
-bool fa32_takes(int batch_heads, int T, int HD, int dtype) {
+// Whether these kernels take a call: rows of a head addressed by 31-bit byte offsets, and more than a few of them.
+// A tile costs the same however many of its 32 rows are there, so the shortest sequences keep one wave per query
+// (flash_attn.hip, flash_attn_bwd.hip); us with gradients, wave per query / tiles, 32 heads, causal:
+//   float32 d 64:  seq 8 20 / 28, seq 16 31 / 28        d 96: seq 16 40 / 39, seq 24 56 / 39
+//           d 128: seq 16 42 / 55, seq 24 57 / 55       FoX d 128: seq 24 61 / 81, seq 32 76 / 82, seq 48 112 / 84
+bool fa32_takes(int batch_heads, int T, int HD, int dtype, bool fox) {
+  if (T < (HD <= 64 ? 16 : HD <= 96 ? 17 : fox ? 33 : 25)) return false;
   const long nb = (long)((T + RB - 1) / RB) * batch_heads;
   return HD <= 128 && (long)(T + 256) * HD * (dtype == EDF_BF16 ? 2 : 4) < (1L << 31) && nb < (1L << 31);
 }

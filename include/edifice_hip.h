@@ -400,7 +400,8 @@ int edf_fused_ttt_scan_backward_saved(void* stream, const void* q, const void* k
  * (native/cuda/fused_flash_attention.cu:168-191).  Extension: `lse` (may be NULL)
  * receives the row log-sum-exp for the backward.  bf16 with head_dim 32, 64 or 128
  * runs on bf16 MFMA, other head_dim <= 128 and float32 on float32 MFMA (bf16 forward, head_dim a multiple of 8:
- * bf16 MFMA with P split into three exact bf16 parts), 128 < head_dim <= 256 a wave-per-row kernel. */
+ * bf16 MFMA with P split into three exact bf16 parts), 128 < head_dim <= 256 and, off the bf16 kernels, the shortest
+ * sequences (fewer than 16 to 33 steps, by width) a wave-per-row kernel. */
 int edf_fused_flash_attention(void* stream, const void* q, const void* k, const void* v, void* out, float* lse,
                               int batch, int num_heads, int seq_len, int head_dim, int causal, int dtype);
 

@@ -121,3 +121,28 @@ def test_only_visible_score_of_a_tile_is_minus_infinity(kind, d, dtype, rng):
     p /= p.sum(-1, keepdims=True)
     assert_close(host(got[0]), np.einsum("bhij,bhjd->bhid", p, vr), TOL[dtype], "o")
     assert_close(host(got[3]), np.einsum("bhij,bhid->bhjd", p, dor), TOL[dtype], "dv")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("kind", ["plain", "causal", "fox"])
+@pytest.mark.parametrize("d", [40, 72, 100, 130, 192, 256])
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 24, 25, 32, 33])
+def test_short_sequences_and_wide_heads(T, d, kind, dtype, rng):
+    """Both sides of the lengths at which one wave per query gives way to tiles, and heads wider than 128, which
+    keep it."""
+    announce("short_and_wide", T=T, d=d, kind=kind, dtype=dtype)
+    shape = (2, 3, T, d)
+    q, k, v, do = (rng.normal(scale=d ** -0.25, size=shape) for _ in range(4))
+    cs = np.cumsum(-np.abs(rng.normal(scale=0.2, size=shape[:3])), axis=-1) if kind == "fox" else None
+    got = _run(q, k, v, do, dtype, kind == "causal", cs)
+    qr, kr, vr, dor = (rounded(a, dtype) for a in (q, k, v, do))
+    if kind == "fox":
+        cr = rounded(cs, dtype)
+        want = [scans.fox_attention(qr, kr, vr, cr), *scans.fox_attention_backward(qr, kr, vr, cr, dor)]
+    else:
+        want = [scans.flash_attention(qr, kr, vr, kind == "causal"),
+                *scans.flash_attention_backward(qr, kr, vr, dor, kind == "causal")]
+    for name, g, w in zip(("o", "dq", "dk", "dv", "dcs"), got, want):
+        # one key: dq, dk and dcs are exactly 0, what is left of dP - D is the rounding of its two equal terms
+        floor = 1.0 if T == 1 and name in ("dq", "dk", "dcs") else np.abs(w).max()
+        assert np.abs(host(g) - w).max() <= TOL[dtype] * floor, name
