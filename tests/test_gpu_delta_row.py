@@ -118,6 +118,57 @@ def test_float32_error(kind, d, rng):
     assert err["out"] <= bound[0] and max(err.values()) <= bound[1], err
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("kind", ["element", "head", "gated", "kda"])
+@pytest.mark.parametrize("shape", [(2, 64, 2, 32), (1, 65, 3, 40), (2, 128, 1, 64), (1, 129, 2, 96), (2, 200, 2, 128),
+                                   (1, 193, 3, 16), (1, 100, 2, 24)])
+def test_row_scan_chunks(shape, kind, dtype, rng):
+    """Several chunks of 16 and tiles of 64 steps, whole and with a remainder, several heads: kept states before and
+    state gradients after a tile, at every padded width."""
+    if kind == "head" and dtype == torch.bfloat16 and shape[3] >= 64:
+        pytest.skip("bf16 with a beta per head takes the chunked kernels at this width")
+    announce("row_scan_chunks", shape=shape, kind=kind, dtype=dtype)
+    a = _inputs(rng, *shape, kind)
+    do = rng.normal(size=shape)
+    t = {n: to_dev(x, dtype).requires_grad_() for n, x in a.items()}
+    out = _call(kind, t)
+    grads = dict(zip(t, torch.autograd.grad(out, list(t.values()), to_dev(do, dtype))))
+    r = {n: rounded(x, dtype) for n, x in a.items()}
+    want = _oracle(kind, r, rounded(do, dtype))
+    for name, g, w in [("o", out, _oracle(kind, r))] + [("d" + n, g, want["d" + n]) for n, g in grads.items()]:
+        err = np.linalg.norm(host(g) - w) / np.linalg.norm(w)
+        assert err <= REL[dtype], f"{name}: {err:.2e}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("kind", ["element", "gated", "kda"])
+def test_unseen_steps_take_no_part_in_gradients(kind, dtype, rng):
+    """No gradient at a step sees the output gradients and queries of earlier steps, and neither the output nor dq
+    at a step sees later keys: infinite ones, from inside a chunk on, leave them as they are."""
+    announce("unseen_gradients", kind=kind, dtype=dtype)
+    shape, cut = (1, 90, 2, 64), 37
+    a = _inputs(rng, *shape, kind)
+    do = rng.normal(size=shape)
+    near = dict(rtol=1e-4, atol=1e-5) if dtype == torch.float32 else dict(rtol=2.0 ** -6, atol=1e-3)
+
+    def run(name=None, at=None):
+        b = {n: x.copy() for n, x in a.items()} | {"do": do.copy()}
+        if name:
+            b[name][:, at] = np.inf
+        t = {n: to_dev(x, dtype).requires_grad_() for n, x in b.items() if n != "do"}
+        out = _call(kind, t)
+        return out, dict(zip(t, torch.autograd.grad(out, list(t.values()), to_dev(b["do"], dtype))))
+
+    base_out, base = run()
+    for name in ("do", "q"):
+        _, got = run(name, slice(0, cut))
+        for n, g in got.items():
+            assert torch.allclose(g[:, cut:].float(), base[n][:, cut:].float(), **near), (name, n)
+    out, got = run("k", slice(cut, None))
+    assert torch.allclose(out[:, :cut].float(), base_out[:, :cut].float(), **near)
+    assert torch.allclose(got["q"][:, :cut].float(), base["q"][:, :cut].float(), **near)
+
+
 @pytest.mark.parametrize("kind", ["element", "gated", "kda"])
 @pytest.mark.parametrize("shape", [(32, 40, 8, 32), (32, 70, 8, 16), (2, 47, 2, 24), (1, 63, 4, 8), (1, 16, 2, 128),
                                    (3, 9, 2, 64), (32, 96, 8, 24)])
