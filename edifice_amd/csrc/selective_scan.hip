@@ -900,12 +900,15 @@ inline int forced_plan() {
 //   channels down.  16 states, D = 2048, T = 1000, forward / backward us, wide -> narrow: B = 2 bf16
 //   70 / 217 -> 45 / 147, f32 68 / 212 -> 46 / 152; B = 4 bf16 72 / 220 -> 55 / 176, f32 70 / 240 -> 58 / 218;
 //   8 states, B = 4: bf16 65 / 209 -> 58 / 188, f32 62 / 221 -> 60 / 201.  At three quarters float32 is slower
-//   (8 states, B = 5: 63 / 229 wide, 61 / 247 narrow).
-// - Otherwise the forward keeps the wide plan (fewer dB / dC partials, longer rows) unless the narrow one has
-//   fewer channels per CU: 8 states, B = 16 bf16 135 us wide, 177 narrow.
+//   (8 states, B = 5: 63 / 229 wide, 61 / 247 narrow).  A backward of fewer than 64 steps and 16 states keeps the
+//   wide plan: its dB / dC partials, four times as many in the narrow one, are then what costs (T = 64, B = 4,
+//   D = 1024 .. 3072, 4 or 8 states: narrow 1.01 to 1.10 of wide; from T = 250 on 0.77 to 1.02).
+// - Otherwise the forward takes the narrow plan where it has fewer channels per CU, or as many on a grid of three
+//   and more wide workgroups per CU, where more of its waves are resident (T = 64 .. 2000, of wide: 4 states 0.85 to
+//   0.98, 8 states 0.84 to 1.12, 0.94 on average, 16 states 0.78 to 0.98; with two per CU 4 and 8 states 0.96 to 1.11).
 // - The backward, whose LDS keeps few workgroups resident, counts a CU's channels as slowed where its resident
 //   waves do not fill 12 slots: 4 states, B = 24 710 us wide, 565 narrow.
-inline SSPlan choose_plan(int batch, int dim, int NP, bool bwd) {
+inline SSPlan choose_plan(int batch, int seq, int dim, int NP, bool bwd) {
   const int SW = NP < 4 ? NP : 4, CW = 64 / SW, NSG = NP / SW;
   const int gw = wide_groups(NP);
   const SSPlan wide{gw, gw * CW, (dim + gw * CW - 1) / (gw * CW)}, narrow{1, CW, (dim + CW - 1) / CW};
@@ -924,8 +927,10 @@ inline SSPlan choose_plan(int batch, int dim, int NP, bool bwd) {
     return Load{per_cu, per_cu * pl.CT, per_cu * nw, (double)(per_cu * pl.CT) / std::min(1.0, resident / 12.0)};
   };
   const Load w = load(wide), n = load(narrow);
-  if (w.per_cu == 1 && n.waves < 12) return 3 * n.channels <= 2 * w.channels ? narrow : wide;
-  return (bwd ? n.slowed < w.slowed : n.channels < w.channels) ? narrow : wide;
+  if (w.per_cu == 1 && n.waves < 12)
+    return 3 * n.channels <= 2 * w.channels && !(bwd && seq < 64 && NP < 16) ? narrow : wide;
+  if (bwd) return n.slowed < w.slowed ? narrow : wide;
+  return n.channels < w.channels || (n.channels == w.channels && w.per_cu >= 3) ? narrow : wide;
 }
 
 // caller-owned "states" buffer: checkpoints [batch][nck][NP][dim] float32, then y before the
@@ -941,7 +946,7 @@ struct WsLayout {
 inline WsLayout bwd_layout(int batch, int seq, int dim, int nst, bool need_ckpt, bool mean_mode) {
   const int N = padded_state(nst);
   WsLayout w{};
-  const int nt = choose_plan(batch, dim, N, true).ntile;
+  const int nt = choose_plan(batch, seq, dim, N, true).ntile;
   size_t off = 0;
   w.ckpt = off;
   if (need_ckpt) off += ckpt_bytes(batch, seq, dim, nst);
@@ -985,7 +990,7 @@ void launch_fwd_g(hipStream_t s, const SSArgs& a) {
 
 template <typename TI, typename TP, int N>
 void launch_fwd_t(hipStream_t s, SSArgs a) {
-  const SSPlan pl = choose_plan(a.batch, a.dim, N, false);
+  const SSPlan pl = choose_plan(a.batch, a.seq, a.dim, N, false);
   a.ntile = pl.ntile;
   constexpr int GW = ss_gwide<N>();
   if constexpr (GW != 1) {
@@ -1026,7 +1031,7 @@ void launch_bwd_t(hipStream_t s, const SSArgs& a) {
   // a.ntile (and the partial buffers sized from it) come from the same plan
   constexpr int GW = ss_gwide<N>();
   if constexpr (GW != 1) {
-    if (choose_plan(a.batch, a.dim, N, true).G == GW) return launch_bwd_g<TI, TP, N, GW>(s, a);
+    if (choose_plan(a.batch, a.seq, a.dim, N, true).G == GW) return launch_bwd_g<TI, TP, N, GW>(s, a);
   }
   launch_bwd_g<TI, TP, N, 1>(s, a);
 }
@@ -1174,7 +1179,7 @@ int edf_fused_selective_scan_backward(void* stream, const void* x, const void* d
     });
     if (rc) return rc;
   }
-  a.ntile = choose_plan(batch, hidden, padded_state(state), true).ntile;
+  a.ntile = choose_plan(batch, seq_len, hidden, padded_state(state), true).ntile;
   a.dout = grad_out;
   a.dx = grad_x;
   a.ddt = grad_dt;
@@ -1225,6 +1230,12 @@ int edf_fused_selective_scan_backward(void* stream, const void* x, const void* d
     if (rc) return rc;
   }
   return EDF_OK;
+}
+
+// 1: the narrow plan, 2: the wide one (tests/edifice_hip_probes.h)
+int edf_debug_selective_scan_plan(int batch, int seq_len, int hidden, int state, int backward) {
+  const int N = edf::padded_state(state);
+  return edf::choose_plan(batch, seq_len, hidden, N, backward != 0).G == edf::wide_groups(N) ? 2 : 1;
 }
 
 }  // extern "C"

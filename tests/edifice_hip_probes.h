@@ -1,5 +1,5 @@
 /* Layout probes of the gfx950 HIP library: TEST INFRASTRUCTURE, not part of the C ABI in
- * include/edifice_hip.h.  libedifice_hip.so exports these three entry points only so that
+ * include/edifice_hip.h.  libedifice_hip.so exports the first three entry points only so that
  * tests/test_gpu_mfma_layout.py can pin the lane layouts the kernels assume; no caller of
  * the library binds them.  Each returns EDF_OK or an EDF_ERR_* code like the product entry
  * points. */
@@ -35,6 +35,10 @@ int edf_debug_lds_read_tr16(void* stream, const void* x, void* out);
  * striding over the buffers: the HBM rate a plain streaming kernel reaches, against which
  * bench.py reads the bandwidth-bound scans. */
 int edf_probe_stream(void* stream, const void* in0, const void* in1, void* out, long n_bytes, int nin, int blocks);
+
+/* The plan that a selective scan of these sizes takes: 1 narrow (one channel group per workgroup), 2 wide.  Runs on
+ * the host; used by tests/test_abi.py to pin the rule. */
+int edf_debug_selective_scan_plan(int batch, int seq_len, int hidden, int state, int backward);
 
 #ifdef __cplusplus
 }

@@ -289,3 +289,13 @@ def test_delta_rule_path_by_size(batch, seq, heads, d, dtype, rows):
     assert got == (up(bh * n * w * w * 4) + up(bh * seq * d * 4) if rows else up(bh * n * ws * ws * 4))
     # a query that does not say whether there is a decay serves both
     assert nat.query("edf_delta_rule_forward_context_bytes", batch, seq, heads, d, dtype, 0) >= got
+
+
+@pytest.mark.parametrize("batch,seq,dim,n,backward,plan", [
+    (32, 128, 3072, 4, 0, 1), (32, 128, 2048, 8, 0, 1), (24, 500, 2048, 4, 0, 1), (16, 500, 2048, 8, 0, 2),
+    (2, 1000, 2048, 16, 0, 1), (2, 1000, 2048, 16, 1, 1), (4, 63, 2048, 8, 1, 2), (4, 64, 2048, 8, 1, 1),
+    (4, 63, 2048, 16, 1, 1), (5, 1000, 2048, 8, 1, 2)])
+def test_selective_scan_plan_of_each_direction(lib, batch, seq, dim, n, backward, plan):
+    """Full grids with equal channels per CU go narrow in the forward from three wide workgroups per CU on; the
+    shortest backwards of narrow states stay wide."""
+    assert lib.edf_debug_selective_scan_plan(batch, seq, dim, n, backward) == plan
