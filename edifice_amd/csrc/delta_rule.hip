@@ -25,7 +25,7 @@ size_t dr_row_context_bytes(int batch, int heads, int seq, int d, bool decay);
 int dr_row_record_run(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
                       void* out, int batch, int seq, int heads, int d, int dtype, int beta_per_head,
                       int alpha_per_row, void* context);
-size_t dr_row_backward_workspace_bytes(int batch, int heads, int seq, int d, bool decay);
+size_t dr_row_backward_workspace_bytes(int batch, int heads, int seq, int d, bool decay, bool saved);
 int dr_row_backward_run(void* stream, const void* q, const void* k, const void* v, const void* beta,
                         const void* alpha, const void* grad_out, void* dq, void* dk, void* dv, void* dbeta,
                         void* dalpha, void* workspace, int batch, int seq, int heads, int d, int dtype,
@@ -85,13 +85,13 @@ bool row_forward(int batch, int heads, int seq, int d, int dtype, bool decay) {
   return !(dtype != EDF_BF16 && (long)batch * heads * ((d + 15) / 16) >= 768 && seq < (decay ? 256 : 64));
 }
 
-// The record of a forward and the workspace of a backward.
+// The record of a forward and the workspace of a backward; saved: with the forward's record at hand.
 size_t unchunked_context_bytes(int batch, int heads, int seq, int d, int dtype, bool decay) {
   return row_path(batch, heads, seq, d, dtype, decay) ? dr_row_context_bytes(batch, heads, seq, d, decay)
                                                : dr_seq_context_bytes(batch, heads, seq, d);
 }
-size_t unchunked_backward_bytes(int batch, int heads, int seq, int d, int dtype, bool decay) {
-  return row_path(batch, heads, seq, d, dtype, decay) ? dr_row_backward_workspace_bytes(batch, heads, seq, d, decay)
+size_t unchunked_backward_bytes(int batch, int heads, int seq, int d, int dtype, bool decay, bool saved) {
+  return row_path(batch, heads, seq, d, dtype, decay) ? dr_row_backward_workspace_bytes(batch, heads, seq, d, decay, saved)
                                                : dr_seq_backward_workspace_bytes(batch, heads, seq, d);
 }
 // What serves a call with a decay and one without: the queries that do not say which.
@@ -100,8 +100,8 @@ size_t any_context_bytes(int batch, int heads, int seq, int d, int dtype) {
                   unchunked_context_bytes(batch, heads, seq, d, dtype, true));
 }
 size_t any_backward_bytes(int batch, int heads, int seq, int d, int dtype) {
-  return std::max(unchunked_backward_bytes(batch, heads, seq, d, dtype, false),
-                  unchunked_backward_bytes(batch, heads, seq, d, dtype, true));
+  return std::max(unchunked_backward_bytes(batch, heads, seq, d, dtype, false, false),
+                  unchunked_backward_bytes(batch, heads, seq, d, dtype, true, false));
 }
 
 int unchunked_fwd(void* stream, const void* q, const void* k, const void* v, const void* beta, const void* alpha,
@@ -164,7 +164,7 @@ int bwd(void* stream, const void* q, const void* k, const void* v, const void* b
     return dr_chunk_backward_run(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch,
                                  seq, heads, d);
   }
-  const size_t need = unchunked_backward_bytes(batch, heads, seq, d, dtype, alpha != nullptr);
+  const size_t need = unchunked_backward_bytes(batch, heads, seq, d, dtype, alpha != nullptr, false);
   EDF_REQUIRE(workspace && ws_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
   return unchunked_bwd(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch, seq, heads,
                        d, dtype, per_head, 0, nullptr);
@@ -190,9 +190,9 @@ int bwd_saved(void* stream, const void* q, const void* k, const void* v, const v
                                        workspace, batch, seq, heads, d);
   }
   // the forward's record when its workspace held one, else the backward recomputes it
-  const size_t need = unchunked_backward_bytes(batch, heads, seq, d, dtype, alpha != nullptr);
-  EDF_REQUIRE(workspace && ws_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
   const bool saved = fwd_ws && fwd_ws_bytes >= unchunked_context_bytes(batch, heads, seq, d, dtype, alpha != nullptr);
+  const size_t need = unchunked_backward_bytes(batch, heads, seq, d, dtype, alpha != nullptr, saved);
+  EDF_REQUIRE(workspace && ws_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
   return unchunked_bwd(stream, q, k, v, beta, alpha, grad_out, dq, dk, dv, dbeta, dalpha, workspace, batch, seq, heads,
                        d, dtype, per_head, 0, saved ? fwd_ws : nullptr);
 }
@@ -219,6 +219,22 @@ int edf_fused_delta_rule_scan_backward_saved(void* stream, const void* q, const 
   return edf::bwd_saved(stream, q, k, v, beta, alpha, grad_out, grad_q, grad_k, grad_v, grad_beta, grad_alpha,
                         forward_workspace, forward_workspace_bytes, workspace, workspace_bytes, batch, seq_len,
                         num_heads, head_dim, dtype, beta_mode);
+}
+
+size_t edf_delta_rule_context_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype, int beta_mode,
+                                    int has_alpha) {
+  if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0 || head_dim > 128) return 0;
+  if (edf::dr_chunk_eligible(seq_len, head_dim, dtype, beta_mode == EDF_BETA_PER_HEAD))
+    return edf::dr_chunk_workspace_bytes(batch, seq_len, num_heads, head_dim);
+  return edf::unchunked_context_bytes(batch, num_heads, seq_len, head_dim, dtype, has_alpha != 0);
+}
+
+size_t edf_delta_rule_context_backward_workspace_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype,
+                                                       int beta_mode, int has_alpha) {
+  if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
+  if (edf::dr_chunk_eligible(seq_len, head_dim, dtype, beta_mode == EDF_BETA_PER_HEAD))
+    return edf::dr_chunk_saved_backward_workspace_bytes(batch, seq_len, num_heads, head_dim);
+  return edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim, dtype, has_alpha != 0, true);
 }
 
 size_t edf_delta_rule_forward_context_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype,
@@ -285,7 +301,7 @@ int edf_fused_gated_delta_net_scan_backward(void* stream, const void* q, const v
 // KDA: per-row log-space decay, per-head beta; never the chunked kernels (which take one decay per head).
 size_t edf_kda_scan_backward_workspace_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype) {
   if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
-  return edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim, dtype, true);
+  return edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim, dtype, true, false);
 }
 
 int edf_fused_kda_scan(void* stream, const void* q, const void* k, const void* v, const void* alpha,
@@ -307,10 +323,15 @@ int edf_fused_kda_scan_backward(void* stream, const void* q, const void* k, cons
   if (rc) return rc;
   EDF_REQUIRE(q && k && v && alpha && beta && grad_out && grad_q && grad_k && grad_v && grad_alpha && grad_beta,
               EDF_ERR_INVALID_ARG, "null tensor pointer");
-  const size_t need = edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim, dtype, true);
+  const size_t need = edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim, dtype, true, false);
   EDF_REQUIRE(workspace && workspace_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
   return edf::unchunked_bwd(stream, q, k, v, beta, alpha, grad_out, grad_q, grad_k, grad_v, grad_beta,
                                   grad_alpha, workspace, batch, seq_len, num_heads, head_dim, dtype, 1, 1, nullptr);
+}
+
+size_t edf_kda_scan_context_backward_workspace_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype) {
+  if (batch <= 0 || seq_len <= 0 || num_heads <= 0 || head_dim <= 0) return 0;
+  return edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim, dtype, true, true);
 }
 
 size_t edf_kda_scan_context_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype) {
@@ -342,7 +363,7 @@ int edf_fused_kda_scan_backward_saved(void* stream, const void* q, const void* k
   const size_t needc = edf::unchunked_context_bytes(batch, num_heads, seq_len, head_dim, dtype, true);
   EDF_REQUIRE(context && context_bytes >= needc, EDF_ERR_WORKSPACE,
               "context too small: need the %zu bytes the forward filled", needc);
-  const size_t need = edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim, dtype, true);
+  const size_t need = edf::unchunked_backward_bytes(batch, num_heads, seq_len, head_dim, dtype, true, true);
   EDF_REQUIRE(workspace && workspace_bytes >= need, EDF_ERR_WORKSPACE, "workspace too small: need %zu bytes", need);
   return edf::unchunked_bwd(stream, q, k, v, beta, alpha, grad_out, grad_q, grad_k, grad_v, grad_beta,
                                   grad_alpha, workspace, batch, seq_len, num_heads, head_dim, dtype, 1, 1,

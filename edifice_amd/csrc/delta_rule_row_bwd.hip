@@ -1072,9 +1072,9 @@ int dr_row_record_run(void* stream, const void* q, const void* k, const void* v,
                     state_width(d));
 }
 
-// Workspace: state gradients, du, and a record of its own for a caller without the forward's.
-size_t dr_row_backward_workspace_bytes(int batch, int heads, int seq, int d, bool decay) {
-  return 2 * dr_row_context_bytes(batch, heads, seq, d, decay);
+// Workspace: state gradients and du; without the forward's record (saved) one of its own behind them.
+size_t dr_row_backward_workspace_bytes(int batch, int heads, int seq, int d, bool decay, bool saved) {
+  return (saved ? 1 : 2) * dr_row_context_bytes(batch, heads, seq, d, decay);
 }
 
 int dr_row_backward_run(void* stream, const void* q, const void* k, const void* v, const void* beta,

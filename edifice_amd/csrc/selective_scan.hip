@@ -901,8 +901,8 @@ inline int forced_plan() {
 //   70 / 217 -> 45 / 147, f32 68 / 212 -> 46 / 152; B = 4 bf16 72 / 220 -> 55 / 176, f32 70 / 240 -> 58 / 218;
 //   8 states, B = 4: bf16 65 / 209 -> 58 / 188, f32 62 / 221 -> 60 / 201.  At three quarters float32 is slower
 //   (8 states, B = 5: 63 / 229 wide, 61 / 247 narrow).  A backward of fewer than 64 steps and 16 states keeps the
-//   wide plan: its dB / dC partials, four times as many in the narrow one, are then what costs (T = 64, B = 4,
-//   D = 1024 .. 3072, 4 or 8 states: narrow 1.01 to 1.10 of wide; from T = 250 on 0.77 to 1.02).
+//   wide plan: its dB / dC partials, four times as many in the narrow one, are then what costs (T = 64 and half
+//   the channels per CU, 4 or 8 states: narrow 1.01 to 1.10 of wide; from T = 250 on 0.83 to 1.02).
 // - Otherwise the forward takes the narrow plan where it has fewer channels per CU, or as many on a grid of three
 //   and more wide workgroups per CU, where more of its waves are resident (T = 64 .. 2000, of wide: 4 states 0.85 to
 //   0.98, 8 states 0.84 to 1.12, 0.94 on average, 16 states 0.78 to 0.98; with two per CU 4 and 8 states 0.96 to 1.11).

@@ -1042,11 +1042,12 @@ class _DeltaRule(torch.autograd.Function):
             raise EdificeHipError(f"alpha must be [B,T,H], got {tuple(alpha.shape)}")
         dt = dtype_flag(q)
         out = torch.empty_like(v)
-        # with gradients to come, a workspace that also keeps the states the backward reads
-        # (the chunked path's per-chunk context, or the per-step path's 16-step states)
-        query = ("edf_delta_rule_forward_context_bytes" if any(ctx.needs_input_grad)
-                 else "edf_delta_rule_workspace_bytes")
-        wsb = nat.query(query, bsz, seq, nh, hd, dt, mode)
+        # with gradients to come, a workspace that also keeps what the backward reads (the chunked path's
+        # per-chunk context, or states and errors of the row scans or states of the per-step kernels)
+        if any(ctx.needs_input_grad):
+            wsb = nat.query("edf_delta_rule_context_bytes", bsz, seq, nh, hd, dt, mode, alpha is not None)
+        else:
+            wsb = nat.query("edf_delta_rule_workspace_bytes", bsz, seq, nh, hd, dt, mode)
         ws = _u8(wsb, q) if wsb else None
         if alpha is None:
             nat.call("edf_fused_delta_net_scan", _stream(), _p(q), _p(k), _p(v), _p(beta), _p(out), _p(ws), wsb,
@@ -1067,7 +1068,11 @@ class _DeltaRule(torch.autograd.Function):
         dt = dtype_flag(q)
         dq, dk, dv, db = (torch.empty_like(t) for t in (q, k, v, beta))
         da = torch.empty_like(alpha) if alpha is not None else None
-        wsb = nat.query("edf_delta_rule_saved_backward_workspace_bytes", bsz, seq, nh, hd, dt, ctx.mode)
+        if ctx.fwd_ws is not None:
+            wsb = nat.query("edf_delta_rule_context_backward_workspace_bytes", bsz, seq, nh, hd, dt, ctx.mode,
+                            alpha is not None)
+        else:  # a second backward through a retained graph recomputes the record
+            wsb = nat.query("edf_delta_rule_saved_backward_workspace_bytes", bsz, seq, nh, hd, dt, ctx.mode)
         ws = _u8(wsb, q)
         nat.call("edf_fused_delta_rule_scan_backward_saved", _stream(), _p(q), _p(k), _p(v), _p(beta), _p(alpha),
                  _p(do), _p(dq), _p(dk), _p(dv), _p(db), _p(da), _p(ctx.fwd_ws), ctx.fwd_wsb, _p(ws), wsb,
@@ -1087,7 +1092,7 @@ class _KDA(torch.autograd.Function):
             raise EdificeHipError("kda_scan needs alpha [B, T, H, d] and beta [B, T, H]")
         out = torch.empty_like(v)
         ctx.rec, ctx.recb = None, 0
-        if any(ctx.needs_input_grad):  # keep the 16-step states the backward reads
+        if any(ctx.needs_input_grad):  # keep the states and errors the backward reads
             ctx.recb = nat.query("edf_kda_scan_context_bytes", bsz, seq, nh, hd, dtype_flag(q))
             ctx.rec = _u8(ctx.recb, q)
             nat.call("edf_fused_kda_scan_with_context", _stream(), _p(q), _p(k), _p(v), _p(alpha), _p(beta), _p(out),
@@ -1104,7 +1109,7 @@ class _KDA(torch.autograd.Function):
         do = do.contiguous().to(q.dtype)
         bsz, seq, nh, hd = q.shape
         dq, dk, dv, da, db = (torch.empty_like(t) for t in (q, k, v, alpha, beta))
-        wsb = nat.query("edf_kda_scan_backward_workspace_bytes", bsz, seq, nh, hd, dtype_flag(q))
+        wsb = nat.query("edf_kda_scan_context_backward_workspace_bytes", bsz, seq, nh, hd, dtype_flag(q))
         ws = _u8(wsb, q)
         nat.call("edf_fused_kda_scan_backward_saved", _stream(), _p(q), _p(k), _p(v), _p(alpha), _p(beta), _p(do),
                  _p(dq), _p(dk), _p(dv), _p(da), _p(db), _p(ctx.rec), ctx.recb, _p(ws), wsb, bsz, seq, nh, hd,

@@ -260,7 +260,9 @@ int edf_fused_kda_scan_backward(void* stream, const void* q, const void* k, cons
  * forward that also keeps the states every 16 steps and the errors v - S k in a caller-kept context of
  * edf_kda_scan_context_bytes() bytes (one pass writes out and both), and the backward
  * from that context (unchanged since), which then skips its forward re-run; gradients
- * bit-identical to edf_fused_kda_scan_backward, workspace edf_kda_scan_backward_workspace_bytes(). */
+ * bit-identical to edf_fused_kda_scan_backward, workspace edf_kda_scan_context_backward_workspace_bytes()
+ * (half of edf_kda_scan_backward_workspace_bytes() and less: no room for a record of its own). */
+size_t edf_kda_scan_context_backward_workspace_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype);
 size_t edf_kda_scan_context_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype);
 int edf_fused_kda_scan_with_context(void* stream, const void* q, const void* k, const void* v, const void* alpha,
                                     const void* beta, void* out, void* context, size_t context_bytes, int batch,
@@ -533,7 +535,16 @@ int edf_fused_gated_delta_net_scan_backward(void* stream, const void* q, const v
  * or NULL forward_workspace it recomputes, as edf_fused_gated_delta_net_scan_backward does.
  * edf_delta_rule_forward_context_bytes() is the chunked path's forward workspace on that
  * path and that record otherwise: the forward workspace a training caller
- * allocates for the saved backward. */
+ * allocates for the saved backward.
+ * These two queries do not say whether there is an alpha, nor whether the record will be there, and
+ * return what serves every case.  A caller that knows both asks for what its calls use:
+ * edf_delta_rule_context_bytes() for the forward workspace, and for this backward's workspace, given a
+ * forward_workspace that holds the record, edf_delta_rule_context_backward_workspace_bytes()
+ * (8x2048x8x128 without alpha: 188 and 188 MiB, the queries above 576 and 1152). */
+size_t edf_delta_rule_context_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype, int beta_mode,
+                                    int has_alpha);
+size_t edf_delta_rule_context_backward_workspace_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype,
+                                                       int beta_mode, int has_alpha);
 size_t edf_delta_rule_forward_context_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype,
                                             int beta_mode);
 size_t edf_delta_rule_saved_backward_workspace_bytes(int batch, int seq_len, int num_heads, int head_dim, int dtype,

@@ -299,3 +299,25 @@ def test_selective_scan_plan_of_each_direction(lib, batch, seq, dim, n, backward
     """Full grids with equal channels per CU go narrow in the forward from three wide workgroups per CU on; the
     shortest backwards of narrow states stay wide."""
     assert lib.edf_debug_selective_scan_plan(batch, seq, dim, n, backward) == plan
+
+
+def test_delta_rule_training_memory():
+    """A call says whether it has a decay and its record: without a decay the states of every 64 steps are kept, with
+    a record the backward needs no room for another; queries that do not say are never smaller."""
+    from edifice_amd import _native as nat
+    a = (8, 2048, 8, 128, 1, 0)
+    states, rows = 64 * 31 * 128 * 128 * 4, 8 * 2048 * 8 * 128 * 4
+    assert nat.query("edf_delta_rule_context_bytes", *a, 0) == states + rows
+    assert nat.query("edf_delta_rule_context_backward_workspace_bytes", *a, 0) == states + rows
+    with_decay = 64 * 128 * 128 * 128 * 4 + rows
+    assert nat.query("edf_delta_rule_context_bytes", *a, 1) == with_decay
+    assert nat.query("edf_kda_scan_context_bytes", *a[:5]) == with_decay
+    assert nat.query("edf_kda_scan_context_backward_workspace_bytes", *a[:5]) == with_decay
+    assert nat.query("edf_kda_scan_backward_workspace_bytes", *a[:5]) == 2 * with_decay
+    assert nat.query("edf_delta_rule_forward_context_bytes", *a) == with_decay
+    assert nat.query("edf_delta_rule_saved_backward_workspace_bytes", *a) == 2 * with_decay
+    chunked = (4, 4096, 16, 128, 1, 1)
+    for name in ("edf_delta_rule_forward_context_bytes", "edf_delta_rule_saved_backward_workspace_bytes"):
+        same = {"edf_delta_rule_forward_context_bytes": "edf_delta_rule_context_bytes"}.get(
+            name, "edf_delta_rule_context_backward_workspace_bytes")
+        assert nat.query(name, *chunked) == nat.query(same, *chunked, 1) == nat.query(same, *chunked, 0)

@@ -214,3 +214,16 @@ def test_batch_rows_past_2_gib(rng):
         for i, (g, w) in enumerate(zip(whole, run(sl))):
             err = (g[:, :, sl].double() - w.double()).norm() / w.double().norm()
             assert err <= 2.0 ** -7, (i, float(err))  # two bfloat16 roundings of one value
+
+
+@pytest.mark.parametrize("kind", ["element", "gated"])
+def test_second_backward_recomputes_the_record(kind, rng):
+    """A retained graph's second backward, whose record is gone, gives the same gradients."""
+    announce("second_backward", kind=kind)
+    a = _inputs(rng, 1, 70, 2, 48, kind)
+    t = {n: to_dev(x, torch.float32).requires_grad_() for n, x in a.items()}
+    out = _call(kind, t)
+    do = torch.ones_like(out)
+    first = torch.autograd.grad(out, list(t.values()), do, retain_graph=True)
+    for g, w in zip(torch.autograd.grad(out, list(t.values()), do), first):
+        assert torch.equal(g, w)
