@@ -430,7 +430,7 @@ def bench_fox(torch, steps, warmup, B=4, H=32, T=4096, d=128):
 
 
 def bench_kda(torch, steps, warmup, B=8, T=2048, H=8, d=128):
-    """KDA (per-row log decay, per-head beta), bf16, on the exact per-step kernels: fwd and bwd
+    """KDA (per-row log decay, per-head beta), bf16, on the row scans: fwd and bwd
     time per call and tokens/s (B T per call)."""
     from edifice_amd import _native as nat
 

@@ -50,7 +50,9 @@ def sources():
 # without spilling (measured: backward 3.01 -> 2.82 ms at config 4, identical results).
 # The chunked delta rule's kernels scale and convert their MFMA accumulators with VALU
 # work after every product; kept in VGPRs they need no v_accvgpr moves (config 3: output
-# kernel 84.6 -> 79.2 us, the others unchanged; identical results).
+# kernel 84.6 -> 79.2 us, the others unchanged; identical results).  The row scans do the same
+# with theirs at every step of a chunk (without the flag 8x2048x8x128 bf16 608 -> 623 us, KDA
+# 4x1000x8x128 344 -> 350, 2x777x8x64 float32 gated 239 -> 267).
 PER_FILE_FLAGS = {
     "flash_attn_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "delta_rule_chunk.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],

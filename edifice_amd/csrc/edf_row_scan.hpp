@@ -193,9 +193,10 @@ template <int W> struct ColFrag<float, W> {
 };
 
 // S[row][column] += sum over the chunk's steps of u[step][row] tile[step][column].  Both products of
-// a tile are 32 deep (the second half of the small one zero): a 16-deep product accumulated into by
-// a 32-deep one right behind it lost part of its result (half of a tile's registers, seen as 1e-6
-// differences in the state), so chained products keep to one shape.
+// a tile are 32 deep (the second half of the small one zero).  A first form with a 16-deep product for the small
+// part gave states 1e-6 off this one, for a cause that was not found: alone, a 16-deep product with a 32-deep one
+// right behind it on the same accumulator gives bit for bit what it gives with waits between (both register forms of
+// the accumulators), and differs from two 32-deep ones by an ulp in an element of eight.  So one shape is kept.
 template <int W>
 EDF_DEVICE void state_add(f32x4 (&S)[W / 16], const ColFrag<bf16, W>& k, f32x4 u) {
   const Split4 s = split4(u);

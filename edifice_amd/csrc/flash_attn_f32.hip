@@ -25,8 +25,10 @@
 //
 // Bound: the f32 MFMA rate (154 TFLOP/s for a large float32 product on this card); short sequences by
 // the longest wave.  Measured against one wave per query walking the keys, which this replaces (forward
-// and backward, 2 x 8 x 1000 x 64 float32 causal: 3883 -> 163 us; forward, 2 x 16 x 1500 x 96 bf16:
-// 9468 -> 329 us = 84 TFLOP/s; 4 x 16 x 2048 x 64 float32: 120 TFLOP/s forward, 86 backward).
+// and backward, 2 x 8 x 1000 float32 causal: 64 columns 3883 -> 163 us, 96 5290 -> 206, 128 5366 -> 373; bf16, 80
+// columns 4377 -> 200; 4 x 16 x 2048 x 64 float32: 120 TFLOP/s forward, 86 backward).  At 128 columns dK/dV holds
+// the row and column fragments of Q and dO at once, past its registers: 101 are spilled in float32, 90 in bf16 (FoX
+// 308 and 637), which is why that width falls behind.
 #include "edf_abi.hpp"
 #include "edf_common.hpp"
 #include "edf_mfma.hpp"

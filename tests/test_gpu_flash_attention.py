@@ -18,7 +18,7 @@ CASES = [
     (1, 2, 160, 128, torch.bfloat16, False),  # whole 32-query tiles, a partial 64-key tile
     (2, 1, 256, 128, torch.bfloat16, True),
     (1, 1, 1, 128, torch.bfloat16, True),
-    (1, 3, 33, 24, torch.bfloat16, True),     # odd head_dim: wave-per-row path
+    (1, 3, 33, 24, torch.bfloat16, True),     # head_dim off 32 / 64 / 128: float32 probabilities
     (2, 2, 40, 16, torch.float32, True),
     (1, 2, 77, 64, torch.float32, False),
     (1, 1, 96, 128, torch.float32, True),
