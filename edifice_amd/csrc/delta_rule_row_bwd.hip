@@ -656,7 +656,8 @@ EDF_DEVICE float scatter64(float (&buf)[64], int lane) {
 // in a lane (whole 256-byte rows of S per load) and a part of the rows, the parts added in LDS.
 // The states before the first chunk and the gradients after the last are zero: an empty buffer reads so, and the
 // loads stay unconditional, in flight together (each behind a branch was waited for by itself: with the row phase on
-// two of the four waves, 159k cycles a workgroup at KDA 4x1000x8x128 bf16, 74k now).
+// two of the four waves, 159k cycles a workgroup at KDA 4x1000x8x128 bf16, 74k now).  At 128 columns it spills 13
+// registers in bf16 and 34 in float32, whose sums take more of them.
 template <typename TT, int DP>
 __global__ __launch_bounds__(256, 2) void dr_row_decay_grad_kernel(const DecayArgs p) {
   constexpr int LD = DP + 4, NT = DP / 16, LM = CH + 4, NP = 136 + 120;
